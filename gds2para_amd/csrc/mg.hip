@@ -638,6 +638,22 @@ __global__ void k_form_freq(int64_t n, double w, const double *__restrict__ A0, 
   out[i] = {(A0 ? A0[i] : 0.0) + a1 * A1[i], w * A2[i]};
 }
 
+// out = N^-1 G^T (nn x ne; N^-1 complex, G^T real and mostly zero)
+__global__ void k_coarse_ng(int64_t nn, int64_t ne, const C2<double> *__restrict__ ninv, const double *__restrict__ gt,
+                            C2<double> *__restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nn * ne) return;
+  const int64_t a = t / ne, i = t - a * ne;
+  C2<double> v = {0., 0.};
+  for (int64_t b = 0; b < nn; ++b) {
+    const double g = gt[b * ne + i];
+    const C2<double> m = ninv[a * nn + b];
+    v.x += m.x * g;
+    v.y += m.y * g;
+  }
+  out[t] = v;
+}
+
 // Augmented [A_b | I] of every block b of the auxiliary coarsest level at
 // angular frequency w, A_b = -w^2 NL0 + i w NL1 restricted to the block's
 // coarse indices (perm), row-major b x 2b at aoff[b].  One workgroup per block.
@@ -690,7 +706,7 @@ __global__ void k_blk_to_dense(int b, const C2<double> *__restrict__ aug, C2<dou
 
 int64_t coarse_entry_bytes(const Hierarchy &H) {
   const int64_t ne = H.neL, nn = H.nnL;
-  return (int64_t)sizeof(C2<double>) * (ne * ne + nn * nn + ne * nn + (H.aux.eig ? 0 : H.aux.inv_len));
+  return (int64_t)sizeof(C2<double>) * (ne * ne + 2 * ne * nn + (H.aux.eig ? 0 : H.aux.inv_len));
 }
 
 namespace {
@@ -725,8 +741,8 @@ gp_status coarse_table_write(const Hierarchy &H, CoarseCache &C, hipStream_t s) 
     C2<double> *b = (C2<double> *)C.e[q].mem;
     h[q] = (const double *)b;
     h[C.cap + q] = (const double *)(b + ne * ne);
-    h[2 * C.cap + q] = (const double *)(b + ne * ne + nn * nn);
-    h[3 * C.cap + q] = (const double *)(b + ne * ne + nn * nn + ne * nn);
+    h[2 * C.cap + q] = (const double *)(b + ne * ne + ne * nn);
+    h[3 * C.cap + q] = (const double *)(b + ne * ne + 2 * ne * nn);
   }
   GP_HIP(hipMemcpyAsync((void *)C.tab, h.data(), sizeof(double *) * h.size(), hipMemcpyHostToDevice, s));
   GP_HIP(hipStreamSynchronize(s));  // h goes out of scope
@@ -845,6 +861,10 @@ gp_status coarse_cache_lookup(const Hierarchy &H, CoarseCache &C, const std::vec
     for (int32_t t = 0; t < (int32_t)C.e.size(); ++t)
       if (C.e[t].mem && C.e[t].omega == omegas[i]) { q = t; break; }
     if (q < 0) {
+      Arena T;
+      struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
+      C2<double> *nbuf = nullptr;
+      GP_TRY(T.alloc(&nbuf, nn * nn));
       GP_TRY(coarse_make_room(C, eb, s));
       for (int32_t t = 0; t < (int32_t)C.e.size(); ++t)
         if (!C.e[t].mem) { q = t; break; }
@@ -858,7 +878,7 @@ gp_status coarse_cache_lookup(const Hierarchy &H, CoarseCache &C, const std::vec
       x.omega = omegas[i];
       x.bytes = std::max<int64_t>(eb, 16);
       C.bytes += x.bytes;
-      C2<double> *kb = (C2<double> *)x.mem, *nbuf = kb + ne * ne, *bb = nbuf + nn * nn, *ab = bb + ne * nn;
+      C2<double> *kb = (C2<double> *)x.mem, *pb = kb + ne * ne, *bb = pb + ne * nn, *ab = bb + ne * nn;
       const double w = x.omega;
       if (ne) k_form_freq<<<blocks_for(ne * ne), 256, 0, s>>>(ne * ne, w, H.KLd[0], H.KLd[1], H.KLd[2], kb);
       if (nn) {
@@ -867,6 +887,8 @@ gp_status coarse_cache_lookup(const Hierarchy &H, CoarseCache &C, const std::vec
       }
       GP_TRY(dense_inverse_batched(kb, (int)ne, 1, s));
       GP_TRY(dense_inverse_batched(nbuf, (int)nn, 1, s));
+      if (nn) k_coarse_ng<<<blocks_for(nn * ne), 256, 0, s>>>(nn, ne, nbuf, H.GTLd, pb);
+      GP_HIP(hipStreamSynchronize(s));  // nbuf is freed here
       if (na && !H.aux.eig) GP_TRY(aux_coarse_inverse(H.aux, w, ab, s));
       fresh = true;
     }
@@ -908,7 +930,7 @@ gp_status vwork_create(gp_layout *lay, const Hierarchy &H, int k, VWork<T> *w) {
     GP_TRY(A.alloc(&w->res[l], ne)); GP_TRY(A.alloc(&w->tmp[l], ne)); GP_TRY(A.alloc(&w->rn[l], nn));
     GP_TRY(A.alloc(&w->dn[l], nn)); GP_TRY(A.alloc(&w->dn2[l], nn));
   }
-  w->gtl = H.GTLd;
+  GP_TRY(A.alloc(&w->crs, std::max<int64_t>((H.neL + H.nnL) * k, 1)));
   const AuxAMG &X = H.aux;
   w->ar.assign(X.L.size(), nullptr); w->ax.assign(X.L.size(), nullptr); w->at.assign(X.L.size(), nullptr);
   for (size_t l = 0; l < X.L.size(); ++l) {
@@ -1950,61 +1972,55 @@ __global__ void k_add(int64_t n, C2<T> *__restrict__ a, const C2<T> *__restrict_
   if (i < n) { a[i].x += b[i].x; a[i].y += b[i].y; }
 }
 
-// Exact coarsest solve in FP64, one block per column:
-//   phi = N^-1 (G^T r);  u = K^-1 (r - B phi)
+// Exact coarsest solve in FP64 of k columns,
+//   phi = N^-1 (G^T r);  rs = r - B phi;  u = K^-1 rs,
+// as three dense products, each spread over the chip with a wavefront per
+// row: N^-1 G^T is kept per frequency (coarse_cache_lookup).  The level has at
+// most ~400 edges, so the products are bound by latency and, where one
+// workgroup walks a column's matrices alone, by what one CU can load: one
+// workgroup per column with a thread per row, each lane reading its own line
+// per entry, took 213 us at 48x48x12 (266 edges, 98 nodes, 16 columns); with
+// 16 lanes per row in one workgroup 23 us plus 4 for u; these take 16 us.
+template <class T, class TX>
+__device__ __forceinline__ C2<double> dense_row(int64_t nc, const C2<double> *__restrict__ M,
+                                                const C2<TX> *__restrict__ x, int64_t xs) {
+  const int lane = threadIdx.x & 63;
+  C2<double> t = {0., 0.};
+#pragma unroll 4
+  for (int64_t b = lane; b < nc; b += 64) {
+    const C2<double> m = M[b];
+    const C2<TX> v = x[b * xs];
+    t.x += m.x * (double)v.x - m.y * (double)v.y;
+    t.y += m.x * (double)v.y + m.y * (double)v.x;
+  }
+  for (int o = 32; o > 0; o >>= 1) { t.x += __shfl_xor(t.x, o); t.y += __shfl_xor(t.y, o); }
+  return t;
+}
+
+// step 0: phi (T and, column by column, FP64 in ph); 1: rs; 2: u.  Grid
+// (rows / 4, columns).
 template <class T>
-__global__ void k_coarse(int64_t ne, int64_t nn, int k, const int32_t *__restrict__ fidx,
-                         const double *const *__restrict__ tab, int cap,
-                         const double *__restrict__ gtl, const C2<T> *__restrict__ r, C2<T> *__restrict__ u,
-                         C2<T> *__restrict__ phi) {
-  extern __shared__ double sm[];
-  double *rr = sm;               // 2*ne
-  double *rn = rr + 2 * ne;      // 2*nn
-  double *ph = rn + 2 * nn;      // 2*nn
-  double *rs = ph + 2 * nn;      // 2*ne
-  const int j = blockIdx.x;
+__global__ void __launch_bounds__(256) k_coarse(int step, int64_t ne, int64_t nn, int k, const int32_t *__restrict__ fidx,
+                                                const double *const *__restrict__ tab, int cap,
+                                                const C2<T> *__restrict__ r, C2<double> *__restrict__ ph,
+                                                C2<double> *__restrict__ rs, C2<T> *__restrict__ phi,
+                                                C2<T> *__restrict__ u) {
+  const int j = blockIdx.y;
+  const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= (step == 0 ? nn : ne)) return;  // uniform across the wavefront
   const int f = fidx[j];
-  for (int64_t i = threadIdx.x; i < ne; i += blockDim.x) { rr[2 * i] = (double)r[i * k + j].x; rr[2 * i + 1] = (double)r[i * k + j].y; }
-  __syncthreads();
-  for (int64_t a = threadIdx.x; a < nn; a += blockDim.x) {
-    double sx = 0, sy = 0;
-    for (int64_t i = 0; i < ne; ++i) { double g = gtl[a * ne + i]; sx += g * rr[2 * i]; sy += g * rr[2 * i + 1]; }
-    rn[2 * a] = sx; rn[2 * a + 1] = sy;
+  const bool first = (threadIdx.x & 63) == 0;
+  if (step == 0) {
+    const C2<double> t = dense_row<T, T>(ne, (const C2<double> *)tab[cap + f] + i * ne, r + j, k);
+    if (first) { ph[(int64_t)j * nn + i] = t; phi[i * k + j] = {(T)t.x, (T)t.y}; }
+  } else if (step == 1) {
+    const C2<T> r0 = r[i * k + j];
+    const C2<double> t = dense_row<T, double>(nn, (const C2<double> *)tab[2 * cap + f] + i * nn, ph + (int64_t)j * nn, 1);
+    if (first) rs[(int64_t)j * ne + i] = {(double)r0.x - t.x, (double)r0.y - t.y};
+  } else {
+    const C2<double> t = dense_row<T, double>(ne, (const C2<double> *)tab[f] + i * ne, rs + (int64_t)j * ne, 1);
+    if (first) u[i * k + j] = {(T)t.x, (T)t.y};
   }
-  __syncthreads();
-  const double *Ni = tab[cap + f];
-  for (int64_t a = threadIdx.x; a < nn; a += blockDim.x) {
-    double sx = 0, sy = 0;
-    for (int64_t b = 0; b < nn; ++b) {
-      double mx = Ni[2 * (a * nn + b)], my = Ni[2 * (a * nn + b) + 1];
-      sx += mx * rn[2 * b] - my * rn[2 * b + 1];
-      sy += mx * rn[2 * b + 1] + my * rn[2 * b];
-    }
-    ph[2 * a] = sx; ph[2 * a + 1] = sy;
-  }
-  __syncthreads();
-  const double *Bf = tab[2 * cap + f];
-  for (int64_t i = threadIdx.x; i < ne; i += blockDim.x) {
-    double sx = rr[2 * i], sy = rr[2 * i + 1];
-    for (int64_t a = 0; a < nn; ++a) {
-      double mx = Bf[2 * (i * nn + a)], my = Bf[2 * (i * nn + a) + 1];
-      sx -= mx * ph[2 * a] - my * ph[2 * a + 1];
-      sy -= mx * ph[2 * a + 1] + my * ph[2 * a];
-    }
-    rs[2 * i] = sx; rs[2 * i + 1] = sy;
-  }
-  __syncthreads();
-  const double *Ki = tab[f];
-  for (int64_t i = threadIdx.x; i < ne; i += blockDim.x) {
-    double sx = 0, sy = 0;
-    for (int64_t b = 0; b < ne; ++b) {
-      double mx = Ki[2 * (i * ne + b)], my = Ki[2 * (i * ne + b) + 1];
-      sx += mx * rs[2 * b] - my * rs[2 * b + 1];
-      sy += mx * rs[2 * b + 1] + my * rs[2 * b];
-    }
-    u[i * k + j] = {(T)sx, (T)sy};
-  }
-  for (int64_t a = threadIdx.x; a < nn; a += blockDim.x) phi[a * k + j] = {(T)ph[2 * a], (T)ph[2 * a + 1]};
 }
 
 // y = r - M2(w) x  (mode 0),  y -= M2(w) x  (mode 1),  y = M2(w) x (mode 2); M2 = c1 v0 + i c2 v1
@@ -2347,8 +2363,11 @@ static gp_status vcycle_level(const Hierarchy &H, VWork<T> &w, hipStream_t s, in
   C2<T> *r = w.r[l], *u = w.u[l], *phi = w.phi[l], *res = w.res[l], *tmp = w.tmp[l];
   C2<T> *rn = w.rn[l], *d1 = w.dn[l], *d2 = w.dn2[l];
   if (l + 1 == (int)H.L.size()) {
-    size_t shm = sizeof(double) * (4 * ne + 4 * nn);
-    k_coarse<T><<<k, 256, shm, s>>>(ne, nn, k, w.fidx, w.tab, w.cap, w.gtl, r, u, phi);
+    C2<double> *ph = w.crs, *rs = w.crs + nn * k;
+    for (int step = 0; step < 3; ++step) {
+      const dim3 grid((unsigned)(((step == 0 ? nn : ne) + 3) / 4), (unsigned)k);
+      if (grid.x) k_coarse<T><<<grid, 256, 0, s>>>(step, ne, nn, k, w.fidx, w.tab, w.cap, r, ph, rs, phi, u);
+    }
     return GP_OK;
   }
   const MatV<T> K = view<T>(L.K, L.Kf), B = view<T>(L.B, L.Bf), N = view<T>(L.N, L.Nf);

@@ -203,7 +203,7 @@ struct Hierarchy {
 
 // Coarsest-level operators per frequency, formed and inverted on the device
 // once per distinct frequency.  tab holds device pointers
-// [kinv | ninv | bl | ainv] x cap, indexed by an entry's slot.  A solve pins
+// [K^-1 | N^-1 G^T | B | ainv] x cap, indexed by an entry's slot.  A solve pins
 // the entry of every device slot's frequency until that slot takes another
 // column or the solve ends; unpinned entries are evicted least recently used
 // first once the cache holds more than max_entries entries or max_bytes bytes
@@ -211,7 +211,7 @@ struct Hierarchy {
 // distinct frequencies are in flight than it allows).
 struct CoarseEntry {
   double omega = 0;
-  void *mem = nullptr;           // one allocation: kinv, ninv, bl, ainv
+  void *mem = nullptr;           // one allocation: K^-1, N^-1 G^T, B, ainv
   int64_t bytes = 0;
   int pins = 0;
   uint64_t used = 0;
@@ -282,7 +282,7 @@ struct VWork {
   int32_t *fidx = nullptr;            // per slot: frequency slot in the CoarseCache
   const double *const *tab = nullptr; // CoarseCache::tab
   int cap = 0;
-  const double *gtl = nullptr;        // coarsest G^T (nnL x neL), real
+  C2<double> *crs = nullptr;          // coarsest solve in FP64: phi, then the edge right-hand sides, column by column
   std::vector<C2<T> *> r, u, phi, res, tmp, rn, dn, dn2;
   // auxiliary AMG: per-level rhs / iterate / scratch, level-0 output, saved input
   std::vector<C2<T> *> ar, ax, at;

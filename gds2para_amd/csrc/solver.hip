@@ -1353,6 +1353,7 @@ int64_t bytes_per_slot(const Hierarchy &H, int m, bool f32, bool v32) {
   if (v32) b += n * tv;  // the Arnoldi vector in the basis precision
   for (const MgLevel &L : H.L) b += (5 * L.ne + 3 * L.nn) * tz;
   for (const AuxLevel &L : H.aux.L) b += 3 * L.n * tz;
+  b += (H.neL + H.nnL) * 16;
   return b + (n + na) * tz;
 }
 

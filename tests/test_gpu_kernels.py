@@ -1,0 +1,34 @@
+"""Kernels at the sizes where they can go wrong: remainders of their row and
+column groups, the smallest and the largest of their ranges."""
+import numpy as np
+import pytest
+
+from gds2para_amd import _capi as capi
+from gds2para_amd import mesh as M
+from gds2para_amd.layout import Layout
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", [capi.GP_PREC_FP64, capi.GP_PREC_MIXED])
+@pytest.mark.parametrize("cells,slots", [((2, 2, 6), 1), ((4, 3, 6), 4), ((4, 4, 6), 16), ((3, 3, 7), 64)])
+def test_coarsest_solve_alone(cells, slots, prec):
+    """A grid of at most 400 edges has no coarser level: the dense coarsest
+    solve of the whole system is the preconditioner.  Its error is the
+    rounding of its inverses and of FP32 vectors, amplified by the 1e9 between
+    the curl-curl and the mass terms, so a few steps reach 1e-8; a coarsest
+    solve that skips or mixes rows or columns leaves an indefinite system of
+    126 to 390 unknowns to plain GMRES.  Every column must end inside its
+    first restart cycle."""
+    m = M.Mesh(M.plate_spec(cells=cells, f=1e9))
+    lay = Layout(m)
+    lay.prepare(prec)
+    edges = [e[0] for e in lay.hierarchy_info()["edge"]]
+    print(f"[kernels] coarsest {cells}: {edges} edges, {slots} slots, precision {prec}", flush=True)
+    assert len(edges) == 1 and edges[0] <= 400
+    fs = np.geomspace(1e9, 1e10, slots)
+    Z, st, _ = lay.solve(fs, precision=prec, rtol=1e-8, batch=slots, restart=16)
+    print(f"[kernels]   iterations {max(st['iters'])}", flush=True)
+    assert st["status"] == capi.GP_OK and st["converged"] == slots
+    assert max(st["iters"]) <= 16
+    lay.close()
