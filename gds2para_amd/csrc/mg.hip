@@ -1615,15 +1615,13 @@ bool edge_march(const Hierarchy &H, int k, const SellV<float> &K, const SellV<fl
   return true;
 }
 
-// SELL nodal l1-Jacobi (contract of k_node); long rows (lidx >= 0) take their
-// product N_eps d, N_sig d from lp = [nlong][2][k]
+// SELL nodal l1-Jacobi (contract of k_node) of an operator without listed rows
 template <class T, int SPL, int LPR, int ES>
 __global__ void __launch_bounds__(256) k_node_sell(int64_t nr, int k, SellV<T> N, const T *__restrict__ c1v,
                                                    const T *__restrict__ c2v, const T *__restrict__ nd0,
                                                    const T *__restrict__ nd1, const T *__restrict__ nl0,
                                                    const T *__restrict__ nl1, const C2<T> *__restrict__ rn,
-                                                   const C2<T> *__restrict__ d, C2<T> *__restrict__ dout, T damp,
-                                                   const int32_t *__restrict__ lidx, const C2<T> *__restrict__ lp) {
+                                                   const C2<T> *__restrict__ d, C2<T> *__restrict__ dout, T damp) {
   constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each;
                            // ES such groups split the row's entries
   const int64_t t_ = xcd_block_id() * blockDim.x + threadIdx.x;
@@ -1641,17 +1639,6 @@ __global__ void __launch_bounds__(256) k_node_sell(int64_t nr, int k, SellV<T> N
 #pragma unroll
     for (int q = 0; q < KS; ++q) acc[q] = {0, 0};
   if (d) {
-    const int32_t lq = lidx ? lidx[i] : -1;
-    if (lq >= 0 && es == 0) {
-      C2<T> s0[KS], s1[KS];
-      load_slots<T, KS>(lp + ((int64_t)lq * 2) * k + j0, s0);
-      load_slots<T, KS>(lp + ((int64_t)lq * 2 + 1) * k + j0, s1);
-#pragma unroll
-      for (int q = 0; q < KS; ++q) {
-        acc[q].x -= c1[q] * s0[q].x - c2[q] * s1[q].y;
-        acc[q].y -= c1[q] * s0[q].y + c2[q] * s1[q].x;
-      }
-    } else if (lq < 0) {
       const int64_t sl = pos >> 6;
       const int lane = (int)(pos & 63);
       const int64_t b0 = N.base[sl];
@@ -1664,7 +1651,6 @@ __global__ void __launch_bounds__(256) k_node_sell(int64_t nr, int k, SellV<T> N
           acc[q].y -= ar * x[q].y + ai * x[q].x;
         }
       });
-    }
   }
   es_reduce<T, KS, LPR, ES>(acc);
   if (es != 0) return;
@@ -1681,11 +1667,10 @@ __global__ void __launch_bounds__(256) k_node_sell(int64_t nr, int k, SellV<T> N
   store_slots<T, KS>(dout + i * k + j0, o);
 }
 
-// SELL y = M x (real M) or y += M x; long rows from lp = [nlong][1][k]
+// SELL y = M x (real M) or y += M x, an operator without listed rows
 template <class T, int SPL, int LPR, int ES>
 __global__ void __launch_bounds__(256) k_spmv_real_sell(int64_t nr, int k, SellV<T> M, const C2<T> *__restrict__ x,
-                                                        C2<T> *__restrict__ y, int accumulate,
-                                                        const int32_t *__restrict__ lidx, const C2<T> *__restrict__ lp) {
+                                                        C2<T> *__restrict__ y, int accumulate) {
   constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each;
                            // ES such groups split the row's entries
   const int64_t t_ = xcd_block_id() * blockDim.x + threadIdx.x;
@@ -1697,10 +1682,7 @@ __global__ void __launch_bounds__(256) k_spmv_real_sell(int64_t nr, int k, SellV
   C2<T> acc[KS];
 #pragma unroll
   for (int q = 0; q < KS; ++q) acc[q] = {0, 0};
-  const int32_t lq = lidx ? lidx[i] : -1;
-  if (lq >= 0) {
-    if (es == 0) load_slots<T, KS>(lp + (int64_t)lq * k + j0, acc);
-  } else {
+  {
     const int64_t sl = pos >> 6;
     const int lane = (int)(pos & 63);
     const int64_t b0 = M.base[sl];
@@ -1721,6 +1703,191 @@ __global__ void __launch_bounds__(256) k_spmv_real_sell(int64_t nr, int k, SellV
   store_slots<T, KS>(y + i * k + j0, acc);
 }
 
+// Products with the auxiliary operators (N, P, P^T, Gx^T): 24 entries or fewer
+// in most rows of the finest level, 30-250 in nearly every row of the coarse
+// ones, up to 1e5 in the conductor aggregates' rows.  One launch takes all but
+// the longest rows whole:
+//   * the first nbw workgroups give each chunk of a listed row (kLongRow) a
+//     wavefront: LPR lanes hold an entry's SPL slots each, 64 / LPR entries
+//     side by side, so the CSR's indices and values are read in order and the
+//     walk of 256 entries takes four rounds at 16 slots.  A row of one chunk
+//     ends here; the others leave partial sums to k_aux_fin;
+//   * the rest walk the short rows' SELL copy, LPR lanes per row.
+// Listed and short rows in one SELL copy (the layout before, with separate
+// launches for rows above 256 entries) left every launch waiting for its
+// longest row: at 48x48x12 with 16 slots 45 / 59 / 65 / 63 us for the residual
+// on the four levels, @@ now.
+//   AX_REAL: y (+)= M x, and with z also z = y / d(w)   (the next sweep from 0)
+//   AX_RES:  y = r - M(w) x
+//   AX_JAC:  y = x + (r - M(w) x) / d(w)
+enum AuxMode { AX_REAL = 0, AX_RES = 1, AX_JAC = 2 };
+
+template <class T>
+struct AuxEp {
+  const C2<T> *r = nullptr;   // AX_RES, AX_JAC
+  C2<T> *y = nullptr;
+  int accumulate = 0;         // AX_REAL
+  C2<T> *z = nullptr;         // AX_REAL
+  const T *d0 = nullptr, *d1 = nullptr, *l0 = nullptr, *l1 = nullptr;  // diagonals (of y's level)
+};
+
+// what the epilogue of a row reads, loaded before its walk
+template <class T, int KS, int MODE>
+struct AuxRow {
+  C2<T> b[KS], x0[KS];
+  T d0, d1, l0, l1;
+  __device__ __forceinline__ void load(const AuxEp<T> &ep, const C2<T> *__restrict__ x, int64_t i, int k, int j0) {
+    if (MODE != AX_REAL) load_slots<T, KS>(ep.r + i * k + j0, b);
+    else if (ep.accumulate) load_slots<T, KS>(ep.y + i * k + j0, b);
+    if (MODE == AX_JAC) load_slots<T, KS>(x + i * k + j0, x0);
+    if (MODE == AX_JAC || (MODE == AX_REAL && ep.z)) { d0 = ep.d0[i]; d1 = ep.d1[i]; l0 = ep.l0[i]; l1 = ep.l1[i]; }
+  }
+  __device__ __forceinline__ void store(const AuxEp<T> &ep, int64_t i, int k, int j0, const T (&c1)[KS], const T (&c2)[KS],
+                                        const C2<T> (&acc)[KS]) {
+    C2<T> o[KS];
+#pragma unroll
+    for (int q = 0; q < KS; ++q) {
+      if (MODE == AX_REAL) o[q] = ep.accumulate ? C2<T>{b[q].x + acc[q].x, b[q].y + acc[q].y} : acc[q];
+      else o[q] = {b[q].x - acc[q].x, b[q].y - acc[q].y};
+    }
+    if (MODE == AX_JAC || (MODE == AX_REAL && ep.z)) {
+      C2<T> z[KS];
+#pragma unroll
+      for (int q = 0; q < KS; ++q) {
+        const C2<T> dg = l1diag<T>({c1[q] * d0, c2[q] * d1}, fabs(c1[q]) * l0 + c2[q] * l1);
+        z[q] = cdiv(o[q], dg);
+        if (MODE == AX_JAC) z[q] = {x0[q].x + z[q].x, x0[q].y + z[q].y};
+      }
+      if (MODE == AX_JAC) { store_slots<T, KS>(ep.y + i * k + j0, z); return; }
+      store_slots<T, KS>(ep.z + i * k + j0, z);
+    }
+    store_slots<T, KS>(ep.y + i * k + j0, o);
+  }
+};
+
+template <class T, int SPL, int LPR, int MODE>
+__global__ void __launch_bounds__(256) k_aux(int64_t nr, int k, unsigned nbw, SellV<T> S, MatV<T> M,
+                                             const T *__restrict__ c1v, const T *__restrict__ c2v,
+                                             const C2<T> *__restrict__ x, AuxEp<T> ep, C2<T> *__restrict__ part) {
+  constexpr int KS = SPL, G = 64 / LPR;
+  C2<T> acc[KS];
+  T c1[KS], c2[KS];
+#pragma unroll
+  for (int q = 0; q < KS; ++q) acc[q] = {0, 0};
+  AuxRow<T, KS, MODE> row;
+  if (blockIdx.x < nbw) {
+    const int c = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (c >= M.nchunk) return;  // uniform across the wavefront
+    const int lane = threadIdx.x & 63, g = lane / LPR;
+    const int j0 = ((int)blockIdx.y * LPR + lane % LPR) * SPL;
+#pragma unroll
+    for (int q = 0; q < KS; ++q) { c1[q] = c1v[j0 + q]; c2[q] = c2v[j0 + q]; }
+    const int64_t b = M.lcb[c], e = M.lce[c];
+    const bool whole = c < M.nsingle;
+    const int64_t i = whole ? (int64_t)M.lrows[c] : 0;
+    if (whole && g == 0) row.load(ep, x, i, k, j0);
+    for (int64_t p = b; p < e; p += 4 * G) {
+      int32_t ci[4];
+      T a0[4], a1[4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {  // past the end: the last entry's column with value 0
+        const int64_t t = p + h * G + g;
+        const bool in = t < e;
+        const int64_t tt = in ? t : e - 1;
+        ci[h] = M.ci[tt];
+        a0[h] = in ? M.v[0][tt] : (T)0;
+        if (MODE != AX_REAL) a1[h] = in ? M.v[1][tt] : (T)0;
+      }
+      C2<T> xv[4][KS];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) load_slots<T, KS>(x + (int64_t)ci[h] * k + j0, xv[h]);
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int q = 0; q < KS; ++q) {
+          if (MODE == AX_REAL) {
+            acc[q].x += a0[h] * xv[h][q].x;
+            acc[q].y += a0[h] * xv[h][q].y;
+          } else {
+            const T ar = c1[q] * a0[h], ai = c2[q] * a1[h];
+            acc[q].x += ar * xv[h][q].x - ai * xv[h][q].y;
+            acc[q].y += ar * xv[h][q].y + ai * xv[h][q].x;
+          }
+        }
+    }
+    es_reduce<T, KS, LPR, G>(acc);
+    if (g != 0) return;
+    if (whole) row.store(ep, i, k, j0, c1, c2, acc);
+    else store_slots<T, KS>(part + (int64_t)(c - M.nsingle) * k + j0, acc);
+    return;
+  }
+  // the short rows: nbw is a multiple of 8, so workgroup b of them sits on
+  // XCD b % 8 as xcd_block_id() has it
+  const unsigned nb = gridDim.x - nbw, bb = blockIdx.x - nbw;
+  const unsigned per = nb >> 3, rem = nb & 7u, xc = bb & 7u;
+  const int64_t t_ = (int64_t)(xc * per + (xc < rem ? xc : rem) + (bb >> 3)) * blockDim.x + threadIdx.x;
+  const int64_t i = t_ / LPR;
+  if (i >= nr || (M.lidx && M.lidx[i] >= 0)) return;
+  const int j0 = ((int)blockIdx.y * LPR + (int)(t_ - i * LPR)) * SPL;
+#pragma unroll
+  for (int q = 0; q < KS; ++q) { c1[q] = c1v[j0 + q]; c2[q] = c2v[j0 + q]; }
+  row.load(ep, x, i, k, j0);
+  sell_row<T, KS, MODE == AX_REAL ? 1 : 2>(S, S.base[i >> 6], S.w[i >> 6], (int)(i & 63), x, k, j0,
+                                           [&](T a0, T a1, T, const C2<T>(&xv)[KS]) {
+#pragma unroll
+    for (int q = 0; q < KS; ++q) {
+      if (MODE == AX_REAL) {
+        acc[q].x += a0 * xv[q].x;
+        acc[q].y += a0 * xv[q].y;
+      } else {
+        const T ar = c1[q] * a0, ai = c2[q] * a1;
+        acc[q].x += ar * xv[q].x - ai * xv[q].y;
+        acc[q].y += ar * xv[q].y + ai * xv[q].x;
+      }
+    }
+  });
+  row.store(ep, i, k, j0, c1, c2, acc);
+}
+
+// rows of several chunks: one workgroup per row and slot group sums their
+// partial sums in a fixed order and ends the row
+template <class T, int SPL, int LPR, int MODE>
+__global__ void __launch_bounds__(256) k_aux_fin(int k, MatV<T> M, const T *__restrict__ c1v, const T *__restrict__ c2v,
+                                                 const C2<T> *__restrict__ x, AuxEp<T> ep,
+                                                 const C2<T> *__restrict__ part) {
+  constexpr int KS = SPL, G = 64 / LPR;
+  __shared__ C2<T> red[4][LPR * KS];
+  const int q0 = M.nsingle + (int)blockIdx.x;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sub = lane % LPR, g = lane / LPR;
+  const int j0 = ((int)blockIdx.y * LPR + sub) * SPL;
+  C2<T> acc[KS];
+#pragma unroll
+  for (int q = 0; q < KS; ++q) acc[q] = {0, 0};
+  for (int c = M.lqp[q0] + wave * G + g; c < M.lqp[q0 + 1]; c += 4 * G) {
+    C2<T> v[KS];
+    load_slots<T, KS>(part + (int64_t)(c - M.nsingle) * k + j0, v);
+#pragma unroll
+    for (int q = 0; q < KS; ++q) { acc[q].x += v[q].x; acc[q].y += v[q].y; }
+  }
+  es_reduce<T, KS, LPR, G>(acc);
+  if (g == 0)
+#pragma unroll
+    for (int q = 0; q < KS; ++q) red[wave][sub * KS + q] = acc[q];
+  __syncthreads();
+  if (threadIdx.x >= LPR) return;
+  T c1[KS], c2[KS];
+#pragma unroll
+  for (int q = 0; q < KS; ++q) {
+    c1[q] = c1v[j0 + q];
+    c2[q] = c2v[j0 + q];
+    for (int w = 1; w < 4; ++w) { acc[q].x += red[w][sub * KS + q].x; acc[q].y += red[w][sub * KS + q].y; }
+  }
+  AuxRow<T, KS, MODE> row;
+  const int64_t i = M.lrows[q0];
+  row.load(ep, x, i, k, j0);
+  row.store(ep, i, k, j0, c1, c2, acc);
+}
+
 // Optional epilogue of k_spmv2_sell over level-0 edge rows: u = damp y / d_l1,
 // the edge smoother's first sweep from zero, formed from y while it is in
 // registers instead of by a separate pass over y.
@@ -1736,7 +1903,6 @@ template <class T, int SPL, int LPR, int ES>
 __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> M, const T *__restrict__ c1v,
                                                     const T *__restrict__ c2v, const C2<T> *__restrict__ r,
                                                     const C2<T> *__restrict__ x, C2<T> *__restrict__ y, int mode,
-                                                    const int32_t *__restrict__ lidx, const C2<T> *__restrict__ lp,
                                                     Jac0<T> jz) {
   constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each;
                            // ES such groups split the row's entries
@@ -1752,16 +1918,7 @@ __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> 
   C2<T> acc[KS];
 #pragma unroll
   for (int q = 0; q < KS; ++q) acc[q] = {0, 0};
-  const int32_t lq = lidx ? lidx[i] : -1;
-  if (lq >= 0) {
-    if (es == 0) {
-      C2<T> s0[KS], s1[KS];
-      load_slots<T, KS>(lp + ((int64_t)lq * 2) * k + j0, s0);
-      load_slots<T, KS>(lp + ((int64_t)lq * 2 + 1) * k + j0, s1);
-#pragma unroll
-      for (int q = 0; q < KS; ++q) acc[q] = {c1[q] * s0[q].x - c2[q] * s1[q].y, c1[q] * s0[q].y + c2[q] * s1[q].x};
-    }
-  } else {
+  {
     const int64_t sl = pos >> 6;
     const int lane = (int)(pos & 63);
     const int64_t b0 = M.base[sl];
@@ -2096,7 +2253,7 @@ MatV<double> view<double>(const Csr &c, const CsrF &) {
   MatV<double> v; v.nr = c.nr; v.nc = c.nc; v.rp = c.rp; v.ci = c.ci; v.nv = c.nv;
   for (int k = 0; k < c.nv; ++k) v.v[k] = c.v[k];
   v.nlong = c.nlong; v.lrows = c.lrows; v.lidx = c.lidx;
-  v.nchunk = c.nchunk; v.lcb = c.lcb; v.lce = c.lce; v.lqp = c.lqp;
+  v.nchunk = c.nchunk; v.nsingle = c.nsingle; v.lcb = c.lcb; v.lce = c.lce; v.lqp = c.lqp;
   v.dg[0] = c.dg[0]; v.dg[1] = c.dg[1];
   return v;
 }
@@ -2105,7 +2262,7 @@ MatV<float> view<float>(const Csr &, const CsrF &f) {
   MatV<float> v; v.nr = f.nr; v.nc = f.nc; v.rp = f.rp; v.ci = f.ci; v.nv = f.nv;
   for (int k = 0; k < f.nv; ++k) v.v[k] = f.v[k];
   v.nlong = f.nlong; v.lrows = f.lrows; v.lidx = f.lidx;
-  v.nchunk = f.nchunk; v.lcb = f.lcb; v.lce = f.lce; v.lqp = f.lqp;
+  v.nchunk = f.nchunk; v.nsingle = f.nsingle; v.lcb = f.lcb; v.lce = f.lce; v.lqp = f.lqp;
   v.dg[0] = f.dg[0]; v.dg[1] = f.dg[1];
   return v;
 }
@@ -2276,37 +2433,37 @@ SellV<float> sv<float>(const Sell &, const SellF &f) {
 template <class T>
 void node_sell(int64_t nr, int64_t smin, int k, const SellV<T> &N, const MatV<T> &Nc, const T *c1, const T *c2, const T *nd0,
                const T *nd1, const T *nl0, const T *nl1, const C2<T> *rn, const C2<T> *d, C2<T> *dout, T damp,
-               const int32_t *lidx, const C2<T> *lp, hipStream_t s) {
+               hipStream_t s) {
   if (nr == 0) return;
   if (nr < smin) {
-    k_node<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Nc, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp, lp);
+    k_node<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Nc, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp, nullptr);
     return;
   }
-  GP_LANES_ES_DISPATCH(k_node_sell, N, nr, k, N, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp, lidx, lp);
+  GP_LANES_ES_DISPATCH(k_node_sell, N, nr, k, N, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp);
 }
 
 template <class T>
 void spmv_real_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const MatV<T> &Mc, const C2<T> *x, C2<T> *y, int accumulate,
-                    const int32_t *lidx, const C2<T> *lp, hipStream_t s) {
+                    hipStream_t s) {
   if (nr == 0) return;
   if (nr < smin) {
-    k_spmv_real<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, x, y, accumulate, lp);
+    k_spmv_real<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, x, y, accumulate, nullptr);
     return;
   }
-  GP_LANES_ES_DISPATCH(k_spmv_real_sell, M, nr, k, M, x, y, accumulate, lidx, lp);
+  GP_LANES_ES_DISPATCH(k_spmv_real_sell, M, nr, k, M, x, y, accumulate);
 }
 
 // Returns whether the optional epilogue jz ran (sliced-ELL path only).
 template <class T>
 bool spmv2_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const MatV<T> &Mc, const T *c1, const T *c2, const C2<T> *r,
-                const C2<T> *x, C2<T> *y, int mode, const int32_t *lidx, const C2<T> *lp, hipStream_t s,
+                const C2<T> *x, C2<T> *y, int mode, hipStream_t s,
                 const Jac0<T> &jz = Jac0<T>()) {
   if (nr == 0) return false;
   if (nr < smin) {
-    k_spmv2<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, c1, c2, r, x, y, mode, lp);
+    k_spmv2<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, c1, c2, r, x, y, mode, nullptr);
     return false;
   }
-  if (!lidx && nr >= kNok2MinRows) {  // large operator, no long rows: two rows per lane group
+  if (nr >= kNok2MinRows) {  // large operator: two rows per lane group
     const int64_t half = (nr + 1) / 2;
     const Lanes ln = lanes_shape<T>(half, k);
     if (ln.sp == 4 && entry_split<T>(M, ln) == 1) {
@@ -2320,7 +2477,7 @@ bool spmv2_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const MatV<T
       return jz.u != nullptr;
     }
   }
-  GP_LANES_ES_DISPATCH(k_spmv2_sell, M, nr, k, M, c1, c2, r, x, y, mode, lidx, lp, jz);
+  GP_LANES_ES_DISPATCH(k_spmv2_sell, M, nr, k, M, c1, c2, r, x, y, mode, jz);
   return jz.u != nullptr;
 }
 
@@ -2335,6 +2492,48 @@ void long_pass(const MatV<T> &M, int k, const C2<T> *x, C2<T> *part, C2<T> *lp, 
   if (M.nlong <= 0) return;
   k_long_part<T><<<M.nchunk, 256, 0, s>>>(M, k, x, part);
   k_long_fin<T><<<M.nlong, 256, 0, s>>>(M, k, part, lp);
+}
+
+template <class T, int MODE>
+void aux_prod(int64_t nr, const VWork<T> &w, const SellV<T> &S, const MatV<T> &M, const C2<T> *x, const AuxEp<T> &ep,
+              hipStream_t s) {
+  if (nr == 0) return;
+  const int k = w.k;
+  if (nr < w.sell_min_rows) {
+    long_pass<T>(M, k, x, w.lpart, w.lp, s);
+    const unsigned g = blocks_for(nr * k);
+    if (MODE == AX_JAC)
+      k_node<T><<<g, 256, 0, s>>>(nr, k, M, w.c1, w.c2, ep.d0, ep.d1, ep.l0, ep.l1, ep.r, x, ep.y, (T)1, w.lp);
+    else if (MODE == AX_RES)
+      k_spmv2<T><<<g, 256, 0, s>>>(nr, k, M, w.c1, w.c2, ep.r, x, ep.y, 0, w.lp);
+    else
+      k_spmv_real<T><<<g, 256, 0, s>>>(nr, k, M, x, ep.y, ep.accumulate, w.lp);
+    if (MODE == AX_REAL && ep.z)
+      k_node<T><<<g, 256, 0, s>>>(nr, k, M, w.c1, w.c2, ep.d0, ep.d1, ep.l0, ep.l1, ep.y, nullptr, ep.z, (T)1, nullptr);
+    return;
+  }
+  const Lanes ln = lanes_shape<T>(nr, k);
+  const unsigned nbw = (unsigned)(((M.nchunk + 3) / 4 + 7) / 8 * 8);
+  const unsigned nbs = M.nlong == nr ? 0u : ln.grid.x;
+  const dim3 grid(nbw + nbs, ln.grid.y);
+  const unsigned nfin = (unsigned)(M.nlong - M.nsingle);
+  auto go = [&](auto sp_, auto lp_) {
+    constexpr int SP = decltype(sp_)::value, LP = decltype(lp_)::value;
+    k_aux<T, SP, LP, MODE><<<grid, 256, 0, s>>>(nr, k, nbw, S, M, w.c1, w.c2, x, ep, w.lpart);
+    if (nfin) k_aux_fin<T, SP, LP, MODE><<<dim3(nfin, grid.y), 256, 0, s>>>(k, M, w.c1, w.c2, x, ep, w.lpart);
+  };
+  auto lanes = [&](auto sp_) {
+    if (ln.lpr == 16) go(sp_, std::integral_constant<int, 16>());
+    else if (ln.lpr == 8) go(sp_, std::integral_constant<int, 8>());
+    else if (ln.lpr == 4) go(sp_, std::integral_constant<int, 4>());
+    else if (ln.lpr == 2) go(sp_, std::integral_constant<int, 2>());
+    else go(sp_, std::integral_constant<int, 1>());
+  };
+  if constexpr (sizeof(T) == 4) {
+    if (ln.sp == 4) { lanes(std::integral_constant<int, 4>()); return; }
+    if (ln.sp == 2) { lanes(std::integral_constant<int, 2>()); return; }
+  }
+  lanes(std::integral_constant<int, 1>());
 }
 
 }  // namespace
@@ -2437,10 +2636,10 @@ static gp_status vcycle_level(const Hierarchy &H, VWork<T> &w, hipStream_t s, in
   tb0();
   edge(r, u, nullptr, res, EdgeMode::RES, 0, damp, s);
   te0(EdgeMode::RES, 0);
-  spmv_real_sell<T>(nn, w.sell_min_rows, k, GTS, GT, res, rn, 0, nullptr, w.lp, s);
-  node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, nullptr, phi, damp, nullptr, w.lp, s);
+  spmv_real_sell<T>(nn, w.sell_min_rows, k, GTS, GT, res, rn, 0, s);
+  node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, nullptr, phi, damp, s);
   for (int it = 1; it < nu_pre; ++it) {
-    node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, phi, d2, damp, nullptr, w.lp, s);
+    node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, phi, d2, damp, s);
     std::swap(phi, d2);
   }
   // coarse-grid correction.  res holds r - K u for this u already, so only
@@ -2450,19 +2649,19 @@ static gp_status vcycle_level(const Hierarchy &H, VWork<T> &w, hipStream_t s, in
   edge(res, u, phi, tmp, EdgeMode::RES | EdgeMode::NOK, 1, damp, s);
   te0(EdgeMode::RES | EdgeMode::NOK, 1);
   const int64_t nec = H.L[l + 1].ne, nnc = H.L[l + 1].nn;
-  spmv_real_sell<T>(nec, w.sell_min_rows, k, PTS, PT, tmp, w.r[l + 1], 0, nullptr, w.lp, s);
+  spmv_real_sell<T>(nec, w.sell_min_rows, k, PTS, PT, tmp, w.r[l + 1], 0, s);
   GP_TRY(vcycle_level<T>(H, w, s, l + 1, nu_pre, nu_post));
-  spmv_real_sell<T>(ne, w.sell_min_rows, k, PS, P, w.u[l + 1], u, 1, nullptr, w.lp, s);
-  spmv_real_sell<T>(nn, w.sell_min_rows, k, PnS, Pn, w.phi[l + 1], phi, 1, nullptr, w.lp, s);
+  spmv_real_sell<T>(ne, w.sell_min_rows, k, PS, P, w.u[l + 1], u, 1, s);
+  spmv_real_sell<T>(nn, w.sell_min_rows, k, PnS, Pn, w.phi[l + 1], phi, 1, s);
   (void)nnc;
   // post-smoothing: nodal, then edges
   tb0();
   edge(r, u, phi, res, EdgeMode::RES, 1, damp, s);
   te0(EdgeMode::RES, 1);
-  spmv_real_sell<T>(nn, w.sell_min_rows, k, GTS, GT, res, rn, 0, nullptr, w.lp, s);
-  node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, nullptr, d1, damp, nullptr, w.lp, s);
+  spmv_real_sell<T>(nn, w.sell_min_rows, k, GTS, GT, res, rn, 0, s);
+  node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, nullptr, d1, damp, s);
   for (int it = 1; it < nu_post; ++it) {
-    node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, d1, d2, damp, nullptr, w.lp, s);
+    node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, d1, d2, damp, s);
     std::swap(d1, d2);
   }
   k_add<T><<<gn, 256, 0, s>>>(nn * k, phi, d1);
@@ -2486,7 +2685,24 @@ gp_status vcycle(const Hierarchy &H, VWork<T> &w, hipStream_t s, int nu_pre, int
   return vcycle_level<T>(H, w, s, 0, nu_pre, nu_post);
 }
 
-// Auxiliary AMG V-cycle on level l: input w.ar[l], output w.ax[l].
+// Epilogue of the product that forms level l's right-hand side: the level's
+// first sweep from zero with it (into the buffer aux_cycle starts from), except
+// on the coarsest level.
+template <class T>
+AuxEp<T> aux_first(const AuxAMG &X, const VWork<T> &w, int l) {
+  AuxEp<T> ep;
+  ep.y = w.ar[l];
+  if (l + 1 < (int)X.L.size()) {
+    const AuxLevel &L = X.L[l];
+    ep.z = w.at[l];
+    ep.d0 = arr<T>(L.nd[0], L.ndf[0]); ep.d1 = arr<T>(L.nd[1], L.ndf[1]);
+    ep.l0 = arr<T>(L.nl[0], L.nlf[0]); ep.l1 = arr<T>(L.nl[1], L.nlf[1]);
+  }
+  return ep;
+}
+
+// Auxiliary AMG V-cycle on level l: input w.ar[l] and its first sweep
+// (aux_first), output w.ax[l].
 template <class T>
 static gp_status aux_cycle(const Hierarchy &H, VWork<T> &w, hipStream_t s, int l) {
   const AuxAMG &X = H.aux;
@@ -2504,30 +2720,28 @@ static gp_status aux_cycle(const Hierarchy &H, VWork<T> &w, hipStream_t s, int l
   const SellV<T> NS = sv<T>(L.Ns, L.Nsf), PS = sv<T>(L.Ps, L.Psf), PTS = sv<T>(L.PTs, L.PTsf);
   const T *d0 = arr<T>(L.nd[0], L.ndf[0]), *d1 = arr<T>(L.nd[1], L.ndf[1]);
   const T *l0 = arr<T>(L.nl[0], L.nlf[0]), *l1 = arr<T>(L.nl[1], L.nlf[1]);
-  const unsigned gr = grid_rows(n, k);
   const int nu = w.nu_aux;
   // x and t trade places after every sweep but the first (2 nu - 1 swaps):
-  // start from t so that the last sweep writes the level's own x
+  // start from t so that the last sweep writes the level's own x.  The first
+  // sweep from zero came with r (aux_first, from the product that formed it)
   std::swap(x, t);
-  node_sell<T>(n, w.sell_min_rows, k, NS, N, w.c1, w.c2, d0, d1, l0, l1, r, nullptr, x, (T)1, L.N.lidx, w.lp, s);
-  for (int it = 1; it < nu; ++it) {
-    long_pass<T>(N, k, x, w.lpart, w.lp, s);
-    node_sell<T>(n, w.sell_min_rows, k, NS, N, w.c1, w.c2, d0, d1, l0, l1, r, x, t, (T)1, L.N.lidx, w.lp, s);
+  AuxEp<T> jac;
+  jac.r = r; jac.d0 = d0; jac.d1 = d1; jac.l0 = l0; jac.l1 = l1;
+  auto sweep = [&]() {
+    jac.y = t;
+    aux_prod<T, AX_JAC>(n, w, NS, N, x, jac, s);
     std::swap(x, t);
-  }
-  long_pass<T>(N, k, x, w.lpart, w.lp, s);
-  spmv2_sell<T>(n, w.sell_min_rows, k, NS, N, w.c1, w.c2, r, x, t, 0, L.N.lidx, w.lp, s);
-  const int64_t nc = X.L[l + 1].n;
-  long_pass<T>(PT, k, t, w.lpart, w.lp, s);
-  spmv_real_sell<T>(nc, w.sell_min_rows, k, PTS, PT, t, w.ar[l + 1], 0, L.PT.lidx, w.lp, s);
+  };
+  for (int it = 1; it < nu; ++it) sweep();
+  AuxEp<T> res;
+  res.r = r; res.y = t;
+  aux_prod<T, AX_RES>(n, w, NS, N, x, res, s);
+  aux_prod<T, AX_REAL>(X.L[l + 1].n, w, PTS, PT, t, aux_first<T>(X, w, l + 1), s);
   GP_TRY(aux_cycle<T>(H, w, s, l + 1));
-  long_pass<T>(P, k, w.ax[l + 1], w.lpart, w.lp, s);
-  spmv_real_sell<T>(n, w.sell_min_rows, k, PS, P, w.ax[l + 1], x, 1, L.P.lidx, w.lp, s);
-  for (int it = 0; it < nu; ++it) {
-    long_pass<T>(N, k, x, w.lpart, w.lp, s);
-    node_sell<T>(n, w.sell_min_rows, k, NS, N, w.c1, w.c2, d0, d1, l0, l1, r, x, t, (T)1, L.N.lidx, w.lp, s);
-    std::swap(x, t);
-  }
+  AuxEp<T> add;
+  add.y = x; add.accumulate = 1;
+  aux_prod<T, AX_REAL>(n, w, PS, P, w.ax[l + 1], add, s);
+  for (int it = 0; it < nu; ++it) sweep();
   if (x != w.ax[l]) GP_HIP(hipMemcpyAsync(w.ax[l], x, sizeof(C2<T>) * n * k, hipMemcpyDeviceToDevice, s));
   return GP_OK;
 }
@@ -2544,8 +2758,7 @@ gp_status precond(const Hierarchy &H, VWork<T> &w, hipStream_t s, int nu_pre, in
   const unsigned gn = grid_rows(n, k), ga = grid_rows(na, k);
   // auxiliary correction: a = AMG(Gx^T r), r <- r - Bx a
   if (w.aux_post) k_copy<T><<<blocks_for(n * k), 256, 0, s>>>(n * k, w.r[0], w.r0);
-  long_pass<T>(GxT, k, w.r[0], w.lpart, w.lp, s);
-  spmv_real_sell<T>(na, w.sell_min_rows, k, GxTS, GxT, w.r[0], w.ar[0], 0, X.GxT.lidx, w.lp, s);
+  aux_prod<T, AX_REAL>(na, w, GxTS, GxT, w.r[0], aux_first<T>(X, w, 0), s);
   if (w.aux_post) {
     GP_TRY(aux_cycle<T>(H, w, s, 0));
     k_copy<T><<<blocks_for(na * k), 256, 0, s>>>(na * k, w.ax[0], w.a);
@@ -2565,7 +2778,7 @@ gp_status precond(const Hierarchy &H, VWork<T> &w, hipStream_t s, int nu_pre, in
     jz.kl0 = arr<T>(L0.kl[0], L0.klf[0]); jz.kl1 = arr<T>(L0.kl[1], L0.klf[1]); jz.kl2 = arr<T>(L0.kl[2], L0.klf[2]);
     jz.u = (((nu_pre - 1) + nu_post) & 1) ? w.tmp[0] : w.u[0];
   }
-  w.u0_ready = spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, nullptr, w.a, w.r[0], 1, nullptr, w.lp, s, jz);
+  w.u0_ready = spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, nullptr, w.a, w.r[0], 1, s, jz);
   // edge V-cycle on the remaining residual
   GP_TRY(vcycle<T>(H, w, s, nu_pre, nu_post));
   // The second auxiliary correction (on r0 - K u - B phi - Bx a) makes the
@@ -2585,9 +2798,8 @@ gp_status precond(const Hierarchy &H, VWork<T> &w, hipStream_t s, int nu_pre, in
   if (!marched)
     edge_sell<T>(n, w.sell_min_rows, k, KS, BS, K, B, w.c1, w.c2, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                  w.r0, w.u[0], w.phi[0], w.res[0], EdgeMode::RES, 1, (T)1, s);
-  spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, nullptr, w.a, w.res[0], 1, nullptr, w.lp, s);
-  long_pass<T>(GxT, k, w.res[0], w.lpart, w.lp, s);
-  spmv_real_sell<T>(na, w.sell_min_rows, k, GxTS, GxT, w.res[0], w.ar[0], 0, X.GxT.lidx, w.lp, s);
+  spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, nullptr, w.a, w.res[0], 1, s);
+  aux_prod<T, AX_REAL>(na, w, GxTS, GxT, w.res[0], aux_first<T>(X, w, 0), s);
   GP_TRY(aux_cycle<T>(H, w, s, 0));
   k_add<T><<<blocks_for(na * k), 256, 0, s>>>(na * k, w.a, w.ax[0]);
   return GP_OK;

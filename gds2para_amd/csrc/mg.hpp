@@ -77,9 +77,9 @@ struct MatV {  // read-only view of a CSR in precision T
   const int32_t *ci = nullptr;
   const T *v[3] = {nullptr, nullptr, nullptr};
   int nv = 0;
-  int32_t nlong = 0;                 // rows reduced block-wise beforehand (kLongRow)
+  int32_t nlong = 0;                 // listed rows (kLongRow) and their chunks, as in Csr
   const int32_t *lrows = nullptr, *lidx = nullptr;
-  int32_t nchunk = 0;
+  int32_t nchunk = 0, nsingle = 0;
   const int64_t *lcb = nullptr, *lce = nullptr;
   const int32_t *lqp = nullptr;
   const T *dg[2] = {nullptr, nullptr};  // diagonal value blocks 1, 2 (then v[1], v[2] unused)
@@ -112,7 +112,7 @@ struct AuxLevel {
   int64_t n = 0;
   Csr N, P, PT;                  // N = [N_eps, N_sig]; P to the next coarser level
   CsrF Nf, Pf, PTf;
-  Sell Ns, Ps, PTs;              // SELL copies (long rows left to the long-row pass)
+  Sell Ns, Ps, PTs;              // SELL copies (listed rows left empty)
   SellF Nsf, Psf, PTsf;
   double *nd[2] = {}, *nl[2] = {};
   float *ndf[2] = {}, *nlf[2] = {};

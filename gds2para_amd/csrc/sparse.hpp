@@ -11,11 +11,16 @@
 namespace gp {
 
 // Rows with more than kLongRow entries (the per-conductor columns of the V0
-// basis couple to a whole conductor surface) are listed in lrows; lidx[i] is
-// the row's position in that list or -1.  Row-parallel kernels take those rows'
-// products from a block-per-row reduction instead of walking them serially.
-constexpr int64_t kLongRow = 256;
-constexpr int64_t kLongChunk = 256;   // entries per block of the long-row reduction
+// basis couple to a whole conductor surface, and nearly every row of the
+// coarse auxiliary operators is one) are listed in lrows; lidx[i] is the row's
+// position in that list or -1.  The SELL copies leave them empty.  kLongRow:
+// at 128x128x16 the level-0 auxiliary operator has 187 of 266,256 rows above
+// it, every other row holds 12 entries or fewer; a row of w entries walked by
+// one lane group takes w / 4 dependent rounds, so the few rows of up to 256
+// entries set the pace of every launch while the line was drawn there (45 us
+// for 28,812 rows against 14 us now).
+constexpr int64_t kLongRow = 24;
+constexpr int64_t kLongChunk = 256;   // entries of a listed row per wavefront
 
 struct Csr {
   int64_t nr = 0, nc = 0, nnz = 0;
@@ -26,8 +31,9 @@ struct Csr {
   int32_t nlong = 0;
   int32_t *lrows = nullptr, *lidx = nullptr;
   // the long rows cut into chunks of kLongChunk entries: chunk c spans
-  // [lcb[c], lce[c]); long row q owns chunks lqp[q] .. lqp[q+1]-1
-  int32_t nchunk = 0;
+  // [lcb[c], lce[c]); long row q owns chunks lqp[q] .. lqp[q+1]-1.  The
+  // nsingle rows of one chunk come first, so chunk q is row q for q < nsingle
+  int32_t nchunk = 0, nsingle = 0;
   int64_t *lcb = nullptr, *lce = nullptr;
   int32_t *lqp = nullptr;
   // when set, value blocks 1 and 2 are diagonal and live here (one per row)
@@ -47,7 +53,7 @@ struct CsrF {
   float *v[3] = {nullptr, nullptr, nullptr};
   int32_t nlong = 0;
   const int32_t *lrows = nullptr, *lidx = nullptr;
-  int32_t nchunk = 0;
+  int32_t nchunk = 0, nsingle = 0;
   const int64_t *lcb = nullptr, *lce = nullptr;
   const int32_t *lqp = nullptr;
   float *dg[2] = {nullptr, nullptr};
@@ -77,7 +83,7 @@ struct SellF {
   const int32_t *rows = nullptr;
 };
 // SELL copy of a CSR (all value arrays); rows listed as long in a (kLongRow)
-// are left empty, their products come from the long-row pass
+// are left empty: kernels take them from the CSR
 // order (device, nr entries, a permutation of the rows, or nullptr): slice
 // position p holds row order[p], so a launch over positions visits the rows in
 // that order; kernels map position -> row through Sell::rows

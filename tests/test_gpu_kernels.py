@@ -32,3 +32,27 @@ def test_coarsest_solve_alone(cells, slots, prec):
     assert st["status"] == capi.GP_OK and st["converged"] == slots
     assert max(st["iters"]) <= 16
     lay.close()
+
+
+@pytest.mark.parametrize("prec,slots", [(capi.GP_PREC_MIXED, 1), (capi.GP_PREC_MIXED, 2), (capi.GP_PREC_MIXED, 4),
+                                        (capi.GP_PREC_MIXED, 8), (capi.GP_PREC_MIXED, 16), (capi.GP_PREC_MIXED, 32),
+                                        (capi.GP_PREC_MIXED, 64), (capi.GP_PREC_FP64, 1), (capi.GP_PREC_FP64, 4)])
+def test_aux_products_match_csr_kernels(prec, slots):
+    """The auxiliary products of listed rows (a wavefront per chunk of 256
+    entries, the longest rows in several) and short rows against the (row,
+    slot) CSR kernels: 48x48x12 has rows of 1 to 11,924 entries on its finest
+    auxiliary level.  The two differ by rounding only, which moves an
+    application by 1e-7 (FP32) or 1e-16 of itself: the iteration counts agree
+    to one step in ten, and Z to 100 times the residual."""
+    m = M.Mesh(M.WORKLOADS["manhattan_48x48x12"]())
+    lay = Layout(m)
+    fs = np.geomspace(2e8, 4e9, max(1, slots // 4))
+    kw = dict(ports=list(range(min(slots, 4))), precision=prec, rtol=1e-10, batch=slots, max_iters=400)
+    Za, sa, _ = lay.solve(fs, **kw)
+    Zb, sb, _ = lay.solve(fs, sell_min_rows=1 << 40, **kw)
+    print(f"[kernels] aux products, {slots} slots, precision {prec}: iterations {max(sa['iters'])} / {max(sb['iters'])}, "
+          f"dZ {np.abs(Za - Zb).max() / np.abs(Zb).max():.2e}", flush=True)
+    assert sa["status"] == sb["status"] == capi.GP_OK
+    assert all(abs(a - b) <= 1 + b // 10 for a, b in zip(sa["iters"], sb["iters"]))
+    assert np.abs(Za - Zb).max() <= 1e-8 * np.abs(Zb).max()
+    lay.close()
