@@ -785,7 +785,7 @@ gp_status aux_coarse_inverse(const AuxAMG &X, double w, C2<double> *inv, hipStre
   k_blk_form<<<X.nblk, 256, 0, s>>>(X.perm, X.boff, X.aoff, X.nL, w, X.NLd[0], X.NLd[1], aug);
   const unsigned nsmall = (unsigned)X.small_h.size();
   if (nsmall) {
-    GP_TRY(gj_workgroup(X.small, X.boff, X.aoff, 0, (int)nsmall, aug, bad, s));
+    GP_TRY(gj_workgroup(X.small, X.boff, X.aoff, (int)nsmall, aug, bad, s));
     k_blk_extract<<<nsmall, 256, 0, s>>>(X.small, X.boff, X.aoff, X.ioff, aug, inv);
   }
   for (int32_t blk : X.big_h) {

@@ -373,16 +373,6 @@ __global__ void k_r_scal(int64_t n, double f, double *__restrict__ x) {
   if (i < n) x[i] *= f;
 }
 
-__global__ void k_r_to_c(int64_t n, const double *__restrict__ a, C2<double> *__restrict__ c) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) c[i] = {a[i], 0.};
-}
-
-__global__ void k_c_to_r(int64_t n, const C2<double> *__restrict__ c, double *__restrict__ a) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = c[i].x;
-}
-
 __global__ void k_csr_dense(int64_t n, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
                             const double *__restrict__ v, double *__restrict__ out) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -587,23 +577,12 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
   RLevel &C = G.L.back();
   const int64_t n = C.A.nr;
   if (n > 4096) return fail(GP_ERR_NOCONV, "real AMG coarsening stalled above 4096 unknowns");
-  double *dn = nullptr;
-  C2<double> *cm = nullptr;
-  Arena tmp;
-  gp_status st = GP_OK;
-  do {
-    if ((st = tmp.alloc(&dn, std::max<int64_t>(n * n, 1))) != GP_OK) break;
-    if ((st = tmp.alloc(&cm, std::max<int64_t>(n * n, 1))) != GP_OK) break;
-    if (hipMemsetAsync(dn, 0, sizeof(double) * n * n, s) != hipSuccess) { st = fail(GP_ERR_HIP, "memset"); break; }
-    k_csr_dense<<<blocks_for(n), 256, 0, s>>>(n, C.A.rp, C.A.ci, C.A.v[0], dn);
-    k_r_to_c<<<blocks_for(n * n), 256, 0, s>>>(n * n, dn, cm);
-    if ((st = dense_inverse_batched(cm, (int)n, 1, s)) != GP_OK) break;
-    if ((st = A.alloc(&G.inv, std::max<int64_t>(n * n, 1))) != GP_OK) break;
-    k_c_to_r<<<blocks_for(n * n), 256, 0, s>>>(n * n, cm, G.inv);
-    if (hipStreamSynchronize(s) != hipSuccess) { st = fail(GP_ERR_HIP, "coarse inverse"); break; }
-  } while (0);
-  tmp.free_all();
-  return st;
+  GP_TRY(A.alloc(&G.inv, std::max<int64_t>(n * n, 1)));
+  GP_HIP(hipMemsetAsync(G.inv, 0, sizeof(double) * n * n, s));
+  k_csr_dense<<<blocks_for(n), 256, 0, s>>>(n, C.A.rp, C.A.ci, C.A.v[0], G.inv);
+  GP_TRY(dense_inverse_real(G.inv, (int)n, s));
+  GP_HIP(hipStreamSynchronize(s));
+  return GP_OK;
 }
 
 void vcycle_real(const RealAMG &G, int l, hipStream_t s) {

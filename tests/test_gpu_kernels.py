@@ -56,3 +56,50 @@ def test_aux_products_match_csr_kernels(prec, slots):
     assert all(abs(a - b) <= 1 + b // 10 for a, b in zip(sa["iters"], sb["iters"]))
     assert np.abs(Za - Zb).max() <= 1e-8 * np.abs(Zb).max()
     lay.close()
+
+
+def _dense_coo(A):
+    r, c = np.nonzero(np.ones_like(A))
+    return r.astype(np.int64), c.astype(np.int64), A.ravel()
+
+
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 63, 64, 65, 250, 257, 511, 512])
+def test_dense_inverse_small(n):
+    """A real system of at most 512 unknowns is its own coarsest level: the
+    preconditioner is the dense inverse.  Random matrices whose diagonal is
+    zero, so that every step needs its pivot; partial pivoting's growth and a
+    condition number c leave an error of at most about n c eps per
+    application, and FGMRES takes two steps to 1e-12 at the most."""
+    from gds2para_amd.layout import solve_real
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n))
+    if n > 1:
+        np.fill_diagonal(A, 0.0)
+    A += 3.0 * np.sqrt(n) * np.eye(n)[rng.permutation(n)] * (1.0 if n > 2 else 0.0)
+    c = np.linalg.cond(A)
+    b = rng.standard_normal(n)
+    x, it, rr = solve_real(*_dense_coo(A), n, b, rtol=1e-12)
+    ref = np.linalg.solve(A, b)
+    print(f"[kernels] dense inverse n={n}: cond {c:.1e}, {it} steps, error {np.linalg.norm(x - ref) / np.linalg.norm(ref):.1e}",
+          flush=True)
+    assert c < 1e6 and it <= 2
+    assert np.linalg.norm(x - ref) <= 1e-11 * c * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n", [1000, 1900, 3800])
+def test_dense_inverse_of_stalled_coarsening(n):
+    """Rows coupled in pairs across the matrix with a zero diagonal: nothing
+    aggregates, so the dense inverse takes all n unknowns (narrower panels, and
+    above ~3700 rows a launch per step).  The inverse of each 2 x 2 pair is
+    exact to rounding: one step to 1e-12."""
+    from gds2para_amd.layout import solve_real
+    rng = np.random.default_rng(n)
+    i = np.arange(n, dtype=np.int64)
+    v = rng.uniform(0.5, 2.0, n)
+    b = rng.standard_normal(n)
+    print(f"[kernels] dense inverse of {n} unknowns", flush=True)
+    x, it, rr = solve_real(i, n - 1 - i, v, n, b, rtol=1e-12)
+    assert it <= 1
+    ref = np.empty(n)
+    ref[n - 1 - i] = b / v
+    assert np.linalg.norm(x - ref) <= 1e-12 * np.linalg.norm(ref)
