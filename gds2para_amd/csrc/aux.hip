@@ -76,17 +76,27 @@ __global__ void k_aux_class(int64_t naux, int64_t ndiel, int64_t nd, const int64
 // centroid of each conductor aggregate column (super node) from its V0d entries
 __global__ void k_super_centroid(int64_t nent, const int64_t *__restrict__ row, const int64_t *__restrict__ col,
                                  int64_t ndiel, Grid g, unsigned long long *__restrict__ acc) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nent) return;
-  const int64_t c = col[i];
-  if (c < ndiel) return;
-  int d; int64_t iz, ix, iy;
-  g.decode(row[i], d, iz, ix, iy);
-  unsigned long long *p = acc + 4 * (c - ndiel);
-  atomicAdd(p, (unsigned long long)iz);
-  atomicAdd(p + 1, (unsigned long long)ix);
-  atomicAdd(p + 2, (unsigned long long)iy);
-  atomicAdd(p + 3, 1ULL);
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t c = i < nent ? col[i] : -1;
+  const bool mine = c >= ndiel;
+  unsigned long long v[4] = {0, 0, 0, 0};
+  if (mine) {
+    int d; int64_t iz, ix, iy;
+    g.decode(row[i], d, iz, ix, iy);
+    v[0] = (unsigned long long)iz; v[1] = (unsigned long long)ix; v[2] = (unsigned long long)iy; v[3] = 1;
+  }
+  // entries come column by column: most wavefronts hold one column's
+  const unsigned long long m = __ballot(mine);
+  if (!m) return;
+  const int64_t c0 = __shfl(c, __ffsll(m) - 1);
+  if (__all(!mine || c == c0)) {
+    for (int k = 0; k < 4; ++k) {
+      for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+      if ((threadIdx.x & 63) == 0) atomicAdd(acc + 4 * (c0 - ndiel) + k, v[k]);
+    }
+  } else if (mine) {
+    for (int k = 0; k < 4; ++k) atomicAdd(acc + 4 * (c - ndiel) + k, v[k]);
+  }
 }
 
 __global__ void k_super_crd(int64_t nsup, int64_t ndiel, const unsigned long long *__restrict__ acc,
@@ -144,19 +154,37 @@ __global__ void k_cc_prop(int64_t n, const int64_t *__restrict__ rp, const int32
                           const double *__restrict__ ne, const double *__restrict__ ns, const int32_t *__restrict__ cls,
                           const int64_t *__restrict__ box, const int64_t *__restrict__ lin, int64_t *__restrict__ lout,
                           int *__restrict__ changed) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  int64_t b = 0, e = 0, own = 0, best = 0, bx = -1;
+  int32_t c = kSuperClass;
+  if (i < n) {
+    c = cls[i];
+    own = best = lin[i];
+    bx = box[i];
+    if (c != kSuperClass) { b = rp[i]; e = rp[i + 1]; }
+  }
+  auto label = [&](int64_t p, int64_t ii, int32_t cc, int64_t bb, int64_t cur) {
+    const int32_t j = ci[p];
+    if (j == (int32_t)ii || box[j] != bb || cls[j] != cc) return cur;
+    const double a = cc == 0 ? ne[p] : ns[p];
+    return a != 0. && lin[j] < cur ? lin[j] : cur;
+  };
+  if (e - b <= 32)
+    for (int64_t p = b; p < e; ++p) best = label(p, i, c, bx, best);
+  // longer rows by the whole wavefront, one after the other
+  for (unsigned long long m = __ballot(e - b > 32); m; m &= m - 1) {
+    const int l = __ffsll(m) - 1;
+    const int64_t bl = __shfl(b, l), el = __shfl(e, l), bxl = __shfl(bx, l);
+    const int32_t cl = __shfl(c, l);
+    int64_t cur = __shfl(own, l);
+    for (int64_t p = bl + lane; p < el; p += 64) cur = label(p, i - lane + l, cl, bxl, cur);
+    for (int o = 32; o > 0; o >>= 1) { const int64_t q = __shfl_xor(cur, o); if (q < cur) cur = q; }
+    if (lane == l) best = cur;
+  }
   if (i >= n) return;
-  const int32_t c = cls[i];
-  int64_t best = lin[i];
-  if (c != kSuperClass)
-    for (int64_t p = rp[i]; p < rp[i + 1]; ++p) {
-      const int32_t j = ci[p];
-      if (j == (int32_t)i || box[j] != box[i] || cls[j] != c) continue;
-      const double a = c == 0 ? ne[p] : ns[p];
-      if (a != 0. && lin[j] < best) best = lin[j];
-    }
   lout[i] = best;
-  if (best != lin[i]) atomicAdd(changed, 1);
+  if (best != own) *changed = 1;
 }
 
 __global__ void k_cc_keys(int64_t n, const int64_t *__restrict__ lab, uint64_t *__restrict__ key, int64_t *__restrict__ idx) {
@@ -196,29 +224,27 @@ __global__ void k_ptent(int64_t n, const int64_t *__restrict__ agg, int64_t *__r
 
 // class-filtered smoothing operator: omega/D_F * A_F, A_F from N_eps (dielectric
 // pairs) or N_sig (same-conductor pairs); super nodes and cross-class pairs dropped
-__global__ void k_filter(int64_t nr, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
+__global__ void k_filter(int64_t nr, int64_t nnz, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
                          const double *__restrict__ ne, const double *__restrict__ ns, const int32_t *__restrict__ cls,
                          double *__restrict__ out, double *__restrict__ dF) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nr) return;
-  const int32_t c = cls[i];
-  double d = 0.;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) {
-    const int32_t j = ci[p];
-    double a = 0.;
-    if (c != kSuperClass && cls[j] == c) a = c == 0 ? ne[p] : ns[p];
-    out[p] = a;
-    if (j == (int32_t)i) d = a;
-  }
-  dF[i] = d > 0 ? d : 0.;
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nnz) return;
+  const int64_t i = csr_row_of(rp, nr, p);
+  const int32_t c = cls[i], j = ci[p];
+  double a = 0.;
+  if (c != kSuperClass && cls[j] == c) a = c == 0 ? ne[p] : ns[p];
+  out[p] = a;
+  if (j == (int32_t)i) dF[i] = a > 0 ? a : 0.;  // dF starts at zero
 }
 
-__global__ void k_scale_rows_inv(int64_t nr, const int64_t *__restrict__ rp, const double *__restrict__ dF, double s,
-                                 double *__restrict__ v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nr) return;
-  const double f = dF[i] > 0 ? s / dF[i] : 0.;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) v[p] *= f;
+__global__ void k_scale_rows_inv(int64_t nr, int64_t nnz, const int64_t *__restrict__ rp, const double *__restrict__ dF,
+                                 double s, double *__restrict__ v) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nnz) return;
+  const double a = v[p];
+  if (a == 0.) return;
+  const double d = dF[csr_row_of(rp, nr, p)];
+  v[p] = a * (d > 0 ? s / d : 0.);
 }
 
 // power iteration step for lambda_max(D^-1 A): y = D^-1 A x, returns partial norms
@@ -239,20 +265,6 @@ __global__ void k_dinv_spmv(int64_t nr, const int64_t *__restrict__ rp, const in
 __global__ void k_fill_hash(int64_t n, double *__restrict__ x) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] = 0.5 + 0.5 * (double)((i * 2654435761ULL) % 1000) / 1000.0;
-}
-
-double dev_norm(const double *x, int64_t n, hipStream_t s) {
-  std::vector<double> h(n);
-  (void)hipMemcpyAsync(h.data(), x, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-  (void)hipStreamSynchronize(s);
-  double a = 0;
-  for (double v : h) a += v * v;
-  return std::sqrt(a);
-}
-
-__global__ void k_scal(int64_t n, double f, double *__restrict__ x) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] *= f;
 }
 
 gp_status dense_host_aux(const Csr &M, int which, int64_t n, std::vector<double> *out) {
@@ -380,20 +392,26 @@ gp_status build_aux(gp_layout *lay, Arena &A, Hierarchy *H) {
       if ((st = tmp.alloc(&dF, nf)) != GP_OK) break;
       if (hipMemcpyAsync(AF.rp, F.N.rp, sizeof(int64_t) * (nf + 1), hipMemcpyDeviceToDevice, s) != hipSuccess ||
           hipMemcpyAsync(AF.ci, F.N.ci, sizeof(int32_t) * F.N.nnz, hipMemcpyDeviceToDevice, s) != hipSuccess) { st = fail(GP_ERR_HIP, "copy"); break; }
-      k_filter<<<blocks_for(nf), 256, 0, s>>>(nf, F.N.rp, F.N.ci, F.N.v[0], F.N.v[1], cls, AF.v[0], dF);
-      double *x = nullptr, *y = nullptr;
+      if (hipMemsetAsync(dF, 0, sizeof(double) * nf, s) != hipSuccess) { st = fail(GP_ERR_HIP, "memset"); break; }
+      k_filter<<<blocks_for(F.N.nnz), 256, 0, s>>>(nf, F.N.nnz, F.N.rp, F.N.ci, F.N.v[0], F.N.v[1], cls, AF.v[0], dF);
+      double *x = nullptr, *y = nullptr, *part = nullptr, *nrm = nullptr;
       if ((st = tmp.alloc(&x, nf)) != GP_OK) break;
       if ((st = tmp.alloc(&y, nf)) != GP_OK) break;
+      if ((st = tmp.alloc(&part, kNormBlocks)) != GP_OK) break;
+      if ((st = tmp.alloc(&nrm, 1)) != GP_OK) break;
+      // lambda = |D^-1 A x| with |x| = 1; the norms stay on the device
       k_fill_hash<<<blocks_for(nf), 256, 0, s>>>(nf, x);
       double lam = 1.0;
-      for (int it = 0; it < 12; ++it) {
+      if ((st = dev_norm(x, nf, part, nrm, s)) != GP_OK || (st = dev_div(x, nf, nrm, s)) != GP_OK) break;
+      for (int it = 0; it < 12 && st == GP_OK; ++it) {
         k_dinv_spmv<<<blocks_for(nf * 64), 256, 0, s>>>(nf, AF.rp, AF.ci, AF.v[0], dF, x, y);
-        lam = dev_norm(y, nf, s) / std::max(dev_norm(x, nf, s), 1e-300);
-        k_scal<<<blocks_for(nf), 256, 0, s>>>(nf, 1.0 / std::max(dev_norm(y, nf, s), 1e-300), y);
+        if ((st = dev_norm(y, nf, part, nrm, s)) == GP_OK) st = dev_div(y, nf, nrm, s);
         std::swap(x, y);
       }
+      if (st != GP_OK) break;
+      if (hipMemcpyAsync(&lam, nrm, sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess) { st = fail(GP_ERR_HIP, "lambda"); break; }
       lam = std::max(lam, 1e-3);
-      k_scale_rows_inv<<<blocks_for(nf), 256, 0, s>>>(nf, AF.rp, dF, 4.0 / (3.0 * lam), AF.v[0]);
+      k_scale_rows_inv<<<blocks_for(F.N.nnz), 256, 0, s>>>(nf, F.N.nnz, AF.rp, dF, 4.0 / (3.0 * lam), AF.v[0]);
       Csr AFc, SP;
       if ((st = csr_drop_zeros(tmp, AF, &AFc, s)) != GP_OK) break;
       if ((st = spgemm(tmp, AFc, Pt, &SP, s)) != GP_OK) break;

@@ -185,12 +185,12 @@ __global__ void k_r_dinv_spmv(int64_t n, const int64_t *__restrict__ rp, const i
 }
 
 // rows of A scaled by f / d_i (the smoothing matrix of the prolongation)
-__global__ void k_r_scale_rows(int64_t n, const int64_t *__restrict__ rp, const double *__restrict__ v,
+__global__ void k_r_scale_rows(int64_t n, int64_t nnz, const int64_t *__restrict__ rp, const double *__restrict__ v,
                                const double *__restrict__ d, double f, double *__restrict__ out) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double s = d[i] != 0. ? f / d[i] : 0.;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) out[p] = s * v[p];
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nnz) return;
+  const double di = d[csr_row_of(rp, n, p)];
+  out[p] = (di != 0. ? f / di : 0.) * v[p];
 }
 
 // Row products split two ways: rows of at most kRLong entries take 8 lanes
@@ -373,11 +373,10 @@ __global__ void k_r_scal(int64_t n, double f, double *__restrict__ x) {
   if (i < n) x[i] *= f;
 }
 
-__global__ void k_csr_dense(int64_t n, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
+__global__ void k_csr_dense(int64_t n, int64_t nnz, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
                             const double *__restrict__ v, double *__restrict__ out) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) out[i * n + ci[p]] += v[p];
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < nnz) out[csr_row_of(rp, n, p) * n + ci[p]] = v[p];  // columns of a row are distinct
 }
 
 }  // namespace
@@ -493,27 +492,29 @@ gp_status match_pass(Arena &A, Arena &tmp, const Csr &M, const double *d, Csr *P
   return GP_OK;
 }
 
-double power_lambda(Arena &tmp, const Csr &M, const double *d, hipStream_t s) {
+__global__ void k_r_fill_hash(int64_t n, double *__restrict__ x) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) x[i] = 0.5 + 0.5 * (double)((i * 2654435761ULL) % 1000) / 1000.0;
+}
+
+// largest eigenvalue of D^-1 A by 12 power iterations, the norms kept on the
+// device (vectors went to the host and back at each before: 24 copies of n)
+gp_status power_lambda(Arena &tmp, const Csr &M, const double *d, double *lam, hipStream_t s) {
   const int64_t n = M.nr;
-  double *x = nullptr, *y = nullptr;
-  if (tmp.alloc(&x, n) != GP_OK || tmp.alloc(&y, n) != GP_OK) return 2.0;
-  std::vector<double> h(n);
-  for (int64_t i = 0; i < n; ++i) h[i] = 0.5 + 0.5 * (double)((i * 2654435761ULL) % 1000) / 1000.0;
-  (void)hipMemcpyAsync(x, h.data(), sizeof(double) * n, hipMemcpyHostToDevice, s);
-  double lam = 1.0;
+  double *x, *y, *part, *nrm;
+  GP_TRY(tmp.alloc(&x, n)); GP_TRY(tmp.alloc(&y, n)); GP_TRY(tmp.alloc(&part, kNormBlocks)); GP_TRY(tmp.alloc(&nrm, 1));
+  k_r_fill_hash<<<blocks_for(n), 256, 0, s>>>(n, x);
   for (int it = 0; it < 12; ++it) {
     k_r_dinv_spmv<<<wave_blocks(n), 256, 0, s>>>(n, M.rp, M.ci, M.v[0], d, x, y);
-    (void)hipMemcpyAsync(h.data(), y, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-    (void)hipStreamSynchronize(s);
-    double nr = 0;
-    for (double v : h) nr += v * v;
-    nr = std::sqrt(nr);
-    lam = nr;  // |D^-1 A x| with |x| = 1 after the first step
-    if (!(nr > 0)) break;
-    for (double &v : h) v /= nr;
-    (void)hipMemcpyAsync(x, h.data(), sizeof(double) * n, hipMemcpyHostToDevice, s);
+    GP_TRY(dev_norm(y, n, part, nrm, s));  // |D^-1 A x| with |x| = 1 after the first step
+    GP_TRY(dev_div(y, n, nrm, s));
+    std::swap(x, y);
   }
-  return std::max(lam, 1e-3);
+  double h = 0.;
+  GP_HIP(hipMemcpyAsync(&h, nrm, sizeof(double), hipMemcpyDeviceToHost, s));
+  GP_HIP(hipStreamSynchronize(s));
+  *lam = std::max(h, 1e-3);
+  return GP_OK;
 }
 
 gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
@@ -546,7 +547,8 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
       if ((st = spgemm(tmp, P1, P2, &Pt, s)) != GP_OK) break;
       if (Pt.nc > (int64_t)(0.8 * (double)n)) { st = GP_ERR_NOCONV; break; }  // stalled: stop coarsening
       // P = Pt - 4/(3 lambda) D^-1 A Pt
-      const double lam = power_lambda(tmp, F.A, F.d, s);
+      double lam = 2.0;
+      if ((st = power_lambda(tmp, F.A, F.d, &lam, s)) != GP_OK) break;
       if (G.smoother == GP_SMOOTH_CHEBYSHEV) {
         cheb_coeffs(lam, F.c1, F.c2);
         if ((st = A.alloc(&F.dd, n)) != GP_OK) break;
@@ -554,7 +556,7 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
       if ((st = csr_alloc(tmp, n, n, F.A.nnz, 1, &DA)) != GP_OK) break;
       if (hipMemcpyAsync(DA.rp, F.A.rp, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice, s) != hipSuccess ||
           hipMemcpyAsync(DA.ci, F.A.ci, sizeof(int32_t) * F.A.nnz, hipMemcpyDeviceToDevice, s) != hipSuccess) { st = fail(GP_ERR_HIP, "copy"); break; }
-      k_r_scale_rows<<<blocks_for(n), 256, 0, s>>>(n, F.A.rp, F.A.v[0], F.d, 4.0 / (3.0 * lam), DA.v[0]);
+      k_r_scale_rows<<<blocks_for(F.A.nnz), 256, 0, s>>>(n, F.A.nnz, F.A.rp, F.A.v[0], F.d, 4.0 / (3.0 * lam), DA.v[0]);
       if ((st = spgemm(tmp, DA, Pt, &DAP, s)) != GP_OK) break;
       if ((st = csr_add(tmp, Pt, -1.0, DAP, &Ps, s)) != GP_OK) break;
       if ((st = truncate_prolongation(A, tmp, Ps, Pt, kTrunc, &P, s)) != GP_OK) break;
@@ -579,7 +581,7 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
   if (n > 4096) return fail(GP_ERR_NOCONV, "real AMG coarsening stalled above 4096 unknowns");
   GP_TRY(A.alloc(&G.inv, std::max<int64_t>(n * n, 1)));
   GP_HIP(hipMemsetAsync(G.inv, 0, sizeof(double) * n * n, s));
-  k_csr_dense<<<blocks_for(n), 256, 0, s>>>(n, C.A.rp, C.A.ci, C.A.v[0], G.inv);
+  if (C.A.nnz) k_csr_dense<<<blocks_for(C.A.nnz), 256, 0, s>>>(n, C.A.nnz, C.A.rp, C.A.ci, C.A.v[0], G.inv);
   GP_TRY(dense_inverse_real(G.inv, (int)n, s));
   GP_HIP(hipStreamSynchronize(s));
   return GP_OK;

@@ -23,26 +23,48 @@ __global__ void k_expand_count(int64_t nr, const int64_t *__restrict__ arp, cons
   cnt[p] = brp[k + 1] - brp[k];
 }
 
-// row index of every nonzero of a CSR (binary search would also do; a scatter is simpler)
-__global__ void k_row_of(int64_t nr, const int64_t *__restrict__ rp, int32_t *__restrict__ row) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nr) return;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) row[p] = (int32_t)i;
+// row index of every nonzero of a CSR
+__global__ void k_row_of(int64_t nr, int64_t nnz, const int64_t *__restrict__ rp, int32_t *__restrict__ row) {
+  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < nnz) row[p] = (int32_t)csr_row_of(rp, nr, p);
 }
 
+// The products of A's entry p with row ci[p] of B.  Rows of B above kCoop
+// entries (a conductor aggregate's hold up to 1e5) are written by the whole
+// wavefront, one after the other: a thread that wrote one alone took 2 ms at
+// 128x128x16 (8.7 ms over a hierarchy, 4.4 now).
+constexpr int64_t kCoop = 32;
 __global__ void k_expand(int64_t annz, const int32_t *__restrict__ arow, const int32_t *__restrict__ aci,
                          const int64_t *__restrict__ brp, const int32_t *__restrict__ bci,
                          const int64_t *__restrict__ off, int64_t nc, uint64_t *__restrict__ key,
                          uint32_t *__restrict__ src_a, uint32_t *__restrict__ src_b) {
-  int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= annz) return;
-  int64_t o = off[p];
-  const int64_t i = arow[p];
-  const int32_t k = aci[p];
-  for (int64_t q = brp[k]; q < brp[k + 1]; ++q, ++o) {
-    key[o] = (uint64_t)i * (uint64_t)nc + (uint64_t)bci[q];
-    src_a[o] = (uint32_t)p;
-    src_b[o] = (uint32_t)q;
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  int64_t o = 0, b = 0, len = 0;
+  uint64_t base = 0;
+  if (p < annz) {
+    o = off[p];
+    const int32_t k = aci[p];
+    b = brp[k];
+    len = brp[k + 1] - b;
+    base = (uint64_t)arow[p] * (uint64_t)nc;
+  }
+  if (len <= kCoop)
+    for (int64_t t = 0; t < len; ++t) {
+      key[o + t] = base + (uint64_t)bci[b + t];
+      src_a[o + t] = (uint32_t)p;
+      src_b[o + t] = (uint32_t)(b + t);
+    }
+  for (unsigned long long m = __ballot(len > kCoop); m; m &= m - 1) {
+    const int l = __ffsll(m) - 1;
+    const int64_t ol = __shfl(o, l), bl = __shfl(b, l), ll = __shfl(len, l);
+    const uint64_t basel = __shfl(base, l);
+    const uint32_t pl = (uint32_t)(p - lane + l);
+    for (int64_t t = lane; t < ll; t += 64) {
+      key[ol + t] = basel + (uint64_t)bci[bl + t];
+      src_a[ol + t] = pl;
+      src_b[ol + t] = (uint32_t)(bl + t);
+    }
   }
 }
 
@@ -73,48 +95,119 @@ struct ValSrc {
 };
 
 // error-free transformations (Dekker/Knuth): a*b = p + e exactly, a+b = s + t exactly
-__device__ __forceinline__ void two_prod(double a, double b, double &p, double &e) { p = a * b; e = fma(a, b, -p); }
+__device__ __forceinline__ void two_prod(double a, double b, double &p, double &e) {
+#pragma clang fp contract(off)
+  p = a * b;
+  e = fma(a, b, -p);
+}
 __device__ __forceinline__ void two_sum(double a, double b, double &s, double &t) {
+#pragma clang fp contract(off)
   s = a + b;
   double bb = s - a;
   t = (a - (s - bb)) + (b - bb);
 }
 
+// Sums of runs of equal keys, entry by entry in run order.  A run of more than
+// kRunLong products goes on the list `longs` (longs[0] their number) for
+// k_reduce_long.
+constexpr int kRunLong = 48;
+constexpr int kRunChunk = 1024;
+
+struct RunSum {
+  double acc = 0., lo = 0.;
+  __device__ __forceinline__ void add(double va, double vb, int exact) {
+#pragma clang fp contract(off)  // two_sum must see the rounded product
+    if (exact) {
+      double p, pe, s2, t2;
+      two_prod(va, vb, p, pe);
+      two_sum(acc, p, s2, t2);
+      acc = s2;
+      lo += t2 + pe;
+    } else {
+      acc = fma(va, vb, acc);
+    }
+  }
+  __device__ __forceinline__ double value(int exact) const { return exact ? acc + lo : acc; }
+};
+
+__device__ __forceinline__ void run_factors(const ValSrc &vs, const uint32_t *src_a, const uint32_t *src_b, uint32_t t,
+                                            int c, double &va, double &vb) {
+  const uint32_t pa = src_a ? src_a[t] : t, pb = src_b ? src_b[t] : 0;
+  va = vs.a[vs.na > 1 ? c : 0][pa];
+  vb = vs.nb > 0 ? vs.b[vs.nb > 1 ? c : 0][pb] : 1.0;
+}
+
 __global__ void k_reduce(int64_t nseg, int64_t n, const int64_t *__restrict__ start, const uint64_t *__restrict__ key,
                          const uint32_t *__restrict__ perm, const uint32_t *__restrict__ src_a,
                          const uint32_t *__restrict__ src_b, ValSrc vs, int64_t nc, int32_t *__restrict__ ci,
-                         int64_t *__restrict__ rowcnt, double *__restrict__ o0, double *__restrict__ o1,
-                         double *__restrict__ o2) {
-  int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+                         double *__restrict__ o0, double *__restrict__ o1, double *__restrict__ o2,
+                         int32_t *__restrict__ longs) {
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nseg) return;
-  int64_t b = start[s], e = (s + 1 < nseg) ? start[s + 1] : n;
-  double acc[3] = {0., 0., 0.}, lo[3] = {0., 0., 0.};
+  const int64_t b = start[s], e = (s + 1 < nseg) ? start[s + 1] : n;
+  ci[s] = (int32_t)(key[b] % (uint64_t)nc);
+  if (e - b > kRunLong) { longs[1 + atomicAdd(longs, 1)] = (int32_t)s; return; }
+  RunSum acc[3];
   for (int64_t q = b; q < e; ++q) {
-    uint32_t t = perm[q];
-    uint32_t pa = src_a ? src_a[t] : t, pb = src_b ? src_b[t] : 0;
+    const uint32_t t = perm[q];
     for (int c = 0; c < vs.nout; ++c) {
-      double va = vs.a[vs.na > 1 ? c : 0][pa];
-      double vb = vs.nb > 0 ? vs.b[vs.nb > 1 ? c : 0][pb] : 1.0;
-      if (vs.exact) {
-        double p, pe, s2, t2;
-        two_prod(va, vb, p, pe);
-        two_sum(acc[c], p, s2, t2);
-        acc[c] = s2;
-        lo[c] += t2 + pe;
-      } else {
-        acc[c] += va * vb;
-      }
+      double va, vb;
+      run_factors(vs, src_a, src_b, t, c, va, vb);
+      acc[c].add(va, vb, vs.exact);
     }
   }
-  if (vs.exact)
-    for (int c = 0; c < vs.nout; ++c) acc[c] += lo[c];
-  uint64_t k = key[b];
-  int64_t row = (int64_t)(k / (uint64_t)nc);
-  ci[s] = (int32_t)(k % (uint64_t)nc);
-  atomicAdd((unsigned long long *)&rowcnt[row], 1ULL);
-  o0[s] = acc[0];
-  if (o1) o1[s] = acc[1];
-  if (o2) o2[s] = acc[2];
+  o0[s] = acc[0].value(vs.exact);
+  if (o1) o1[s] = acc[1].value(vs.exact);
+  if (o2) o2[s] = acc[2].value(vs.exact);
+}
+
+// The listed runs, a workgroup each: the factors of kRunChunk products at a
+// time come to LDS by all threads, one thread per value array sums them in run
+// order (the same bits as k_reduce).  The diagonal entries of the conductor
+// aggregates are sums of up to 1e5 products; a thread that gathered them alone
+// took 21 ms at 128x128x16, 2.4 now.
+__global__ void __launch_bounds__(256) k_reduce_long(int64_t nseg, int64_t n, const int64_t *__restrict__ start,
+                                                     const uint32_t *__restrict__ perm,
+                                                     const uint32_t *__restrict__ src_a,
+                                                     const uint32_t *__restrict__ src_b, ValSrc vs,
+                                                     double *__restrict__ o0, double *__restrict__ o1,
+                                                     double *__restrict__ o2, const int32_t *__restrict__ longs) {
+  __shared__ double A[3][kRunChunk], B[3][kRunChunk];
+  double *o[3] = {o0, o1, o2};
+  const int count = longs[0];
+  for (int r = blockIdx.x; r < count; r += gridDim.x) {
+    const int64_t s = longs[1 + r];
+    const int64_t b = start[s], e = (s + 1 < nseg) ? start[s + 1] : n;
+    RunSum acc;
+    for (int64_t q0 = b; q0 < e; q0 += kRunChunk) {
+      const int m = (int)min((int64_t)kRunChunk, e - q0);
+      __syncthreads();
+      for (int h = threadIdx.x; h < m; h += 256) {
+        const uint32_t t = perm[q0 + h];
+        for (int c = 0; c < vs.nout; ++c) run_factors(vs, src_a, src_b, t, c, A[c][h], B[c][h]);
+      }
+      __syncthreads();
+      // one thread in each of three wavefronts
+      const int c = threadIdx.x >> 6;
+      if ((threadIdx.x & 63) == 0 && c < vs.nout) {
+#pragma unroll 8
+        for (int h = 0; h < m; ++h) acc.add(A[c][h], B[c][h], vs.exact);
+      }
+    }
+    const int c = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0 && c < vs.nout) o[c][s] = acc.value(vs.exact);
+  }
+}
+
+// row pointers from the sorted runs: run s writes the pointers of the rows
+// after run s - 1's up to its own (s = nseg: of the rows after the last)
+__global__ void k_run_rows(int64_t nseg, int64_t nr, const int64_t *__restrict__ start, const uint64_t *__restrict__ key,
+                           int64_t nc, int64_t *__restrict__ rp) {
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s > nseg) return;
+  const int64_t lo = s == 0 ? -1 : (int64_t)(key[start[s - 1]] / (uint64_t)nc);
+  const int64_t hi = s == nseg ? nr : (int64_t)(key[start[s]] / (uint64_t)nc);
+  for (int64_t r = lo + 1; r <= hi; ++r) rp[r] = s;
 }
 
 int bits_for(uint64_t maxkey) {
@@ -130,7 +223,8 @@ gp_status sort_reduce(Arena &A, int64_t nr, int64_t nc, int64_t nprod, uint64_t 
   gp_status st = GP_OK;
   uint64_t *key2 = nullptr;
   uint32_t *perm = nullptr, *perm2 = nullptr;
-  int64_t *head = nullptr, *hscan = nullptr, *start = nullptr, *rowcnt = nullptr;
+  int64_t *head = nullptr, *hscan = nullptr, *start = nullptr;
+  int32_t *longs = nullptr;
   if (nprod > 2147483647LL) return fail(GP_ERR_NOMEM, "Galerkin expansion exceeds 2^31 products");
   do {
     if ((st = tmp.alloc(&key2, nprod)) != GP_OK) break;
@@ -155,12 +249,14 @@ gp_status sort_reduce(Arena &A, int64_t nr, int64_t nc, int64_t nprod, uint64_t 
     if ((st = tmp.alloc(&start, nseg)) != GP_OK) break;
     k_seg_start<<<blocks_for(nprod), 256, 0, s>>>(nprod, head, hscan, start);
     if ((st = csr_alloc(A, nr, nc, nseg, vs.nout, out)) != GP_OK) break;
-    if ((st = tmp.alloc(&rowcnt, nr)) != GP_OK) break;
-    if (hipMemsetAsync(rowcnt, 0, sizeof(int64_t) * nr, s) != hipSuccess) { st = fail(GP_ERR_HIP, "memset"); break; }
-    k_reduce<<<blocks_for(nseg), 256, 0, s>>>(nseg, nprod, start, key2, perm2, src_a, src_b, vs, nc, out->ci, rowcnt,
-                                               out->v[0], vs.nout > 1 ? out->v[1] : nullptr,
-                                               vs.nout > 2 ? out->v[2] : nullptr);
-    if ((st = exclusive_scan_i64(rowcnt, out->rp, nr, s, tmp)) != GP_OK) break;
+    // runs above kRunLong: fewer than nprod / kRunLong of them
+    if ((st = tmp.alloc(&longs, nprod / kRunLong + 2)) != GP_OK) break;
+    if (hipMemsetAsync(longs, 0, sizeof(int32_t), s) != hipSuccess) { st = fail(GP_ERR_HIP, "memset"); break; }
+    double *o1 = vs.nout > 1 ? out->v[1] : nullptr, *o2 = vs.nout > 2 ? out->v[2] : nullptr;
+    k_reduce<<<blocks_for(nseg), 256, 0, s>>>(nseg, nprod, start, key2, perm2, src_a, src_b, vs, nc, out->ci, out->v[0],
+                                              o1, o2, longs);
+    k_reduce_long<<<512, 256, 0, s>>>(nseg, nprod, start, perm2, src_a, src_b, vs, out->v[0], o1, o2, longs);
+    k_run_rows<<<blocks_for(nseg + 1), 256, 0, s>>>(nseg, nr, start, key2, nc, out->rp);
     if (hipStreamSynchronize(s) != hipSuccess || hipGetLastError() != hipSuccess) { st = fail(GP_ERR_HIP, "sort_reduce kernels"); break; }
   } while (0);
   (void)hipStreamSynchronize(s);
@@ -176,12 +272,14 @@ __global__ void k_coo_keys(int64_t n, const int64_t *__restrict__ r, const int64
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) key[i] = (uint64_t)r[i] * (uint64_t)nc + (uint64_t)c[i];
 }
-__global__ void k_csr_triplets(int64_t nr, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
+__global__ void k_csr_triplets(int64_t nr, int64_t nnz, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
                                const double *__restrict__ v, double alpha, int64_t base, int64_t *__restrict__ r,
                                int64_t *__restrict__ c, double *__restrict__ ov) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nr) return;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) { r[base + p] = i; c[base + p] = ci[p]; ov[base + p] = alpha * v[p]; }
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nnz) return;
+  r[base + p] = csr_row_of(rp, nr, p);
+  c[base + p] = ci[p];
+  ov[base + p] = alpha * v[p];
 }
 }  // namespace
 
@@ -217,8 +315,8 @@ gp_status csr_add(Arena &A, const Csr &a, double alpha, const Csr &b, Csr *c, hi
     if ((st = tmp.alloc(&r, std::max<int64_t>(n, 1))) != GP_OK) break;
     if ((st = tmp.alloc(&cc, std::max<int64_t>(n, 1))) != GP_OK) break;
     if ((st = tmp.alloc(&v, std::max<int64_t>(n, 1))) != GP_OK) break;
-    k_csr_triplets<<<blocks_for(a.nr), 256, 0, s>>>(a.nr, a.rp, a.ci, a.v[0], 1.0, 0, r, cc, v);
-    k_csr_triplets<<<blocks_for(b.nr), 256, 0, s>>>(b.nr, b.rp, b.ci, b.v[0], alpha, a.nnz, r, cc, v);
+    if (a.nnz) k_csr_triplets<<<blocks_for(a.nnz), 256, 0, s>>>(a.nr, a.nnz, a.rp, a.ci, a.v[0], 1.0, 0, r, cc, v);
+    if (b.nnz) k_csr_triplets<<<blocks_for(b.nnz), 256, 0, s>>>(b.nr, b.nnz, b.rp, b.ci, b.v[0], alpha, a.nnz, r, cc, v);
     const double *vals[1] = {v};
     st = csr_from_coo(A, a.nr, a.nc, n, r, cc, vals, 1, c, s);
   } while (0);
@@ -232,13 +330,15 @@ __global__ void k_nz_flags(int64_t nnz, const double *__restrict__ v, int64_t *_
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nnz) f[i] = v[i] != 0.0;
 }
-__global__ void k_nz_compact(int64_t nr, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
+__global__ void k_nz_compact(int64_t nr, int64_t nnz, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
                              const double *__restrict__ v, const int64_t *__restrict__ pos, int64_t *__restrict__ r,
                              int64_t *__restrict__ c, double *__restrict__ ov) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nr) return;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p)
-    if (v[p] != 0.0) { r[pos[p]] = i; c[pos[p]] = ci[p]; ov[pos[p]] = v[p]; }
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= nnz || v[p] == 0.0) return;
+  const int64_t q = pos[p];
+  r[q] = csr_row_of(rp, nr, p);
+  c[q] = ci[p];
+  ov[q] = v[p];
 }
 }  // namespace
 
@@ -257,7 +357,7 @@ gp_status csr_drop_zeros(Arena &A, const Csr &a, Csr *out, hipStream_t s) {
     if ((st = tmp.alloc(&r, std::max<int64_t>(nk, 1))) != GP_OK) break;
     if ((st = tmp.alloc(&c, std::max<int64_t>(nk, 1))) != GP_OK) break;
     if ((st = tmp.alloc(&v, std::max<int64_t>(nk, 1))) != GP_OK) break;
-    k_nz_compact<<<blocks_for(a.nr), 256, 0, s>>>(a.nr, a.rp, a.ci, a.v[0], pos, r, c, v);
+    if (a.nnz) k_nz_compact<<<blocks_for(a.nnz), 256, 0, s>>>(a.nr, a.nnz, a.rp, a.ci, a.v[0], pos, r, c, v);
     const double *vals[1] = {v};
     st = csr_from_coo(A, a.nr, a.nc, nk, r, c, vals, 1, out, s);
   } while (0);
@@ -312,7 +412,7 @@ gp_status spgemm_ex(Arena &A, const Csr &a, const Csr &b, Csr *c, hipStream_t s,
     if ((st = tmp.alloc(&cnt, a.nnz)) != GP_OK) break;
     if ((st = tmp.alloc(&off, a.nnz + 1)) != GP_OK) break;
     if ((st = tmp.alloc(&arow, a.nnz)) != GP_OK) break;
-    k_row_of<<<blocks_for(a.nr), 256, 0, s>>>(a.nr, a.rp, arow);
+    k_row_of<<<blocks_for(a.nnz), 256, 0, s>>>(a.nr, a.nnz, a.rp, arow);
     k_expand_count<<<blocks_for(a.nnz), 256, 0, s>>>(a.nr, a.rp, a.ci, b.rp, cnt);
     if ((st = exclusive_scan_i64(cnt, off, a.nnz, s, tmp)) != GP_OK) break;
     int64_t nprod = 0;
@@ -338,12 +438,10 @@ gp_status spgemm_ex(Arena &A, const Csr &a, const Csr &b, Csr *c, hipStream_t s,
 }
 
 namespace {
-__global__ void k_transpose_keys(int64_t nr, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                                 int64_t nrow_t, uint64_t *__restrict__ key) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nr) return;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) key[p] = (uint64_t)ci[p] * (uint64_t)nr + (uint64_t)i;
-  (void)nrow_t;
+__global__ void k_transpose_keys(int64_t nr, int64_t nnz, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
+                                 uint64_t *__restrict__ key) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < nnz) key[p] = (uint64_t)ci[p] * (uint64_t)nr + (uint64_t)csr_row_of(rp, nr, p);
 }
 }  // namespace
 
@@ -356,7 +454,7 @@ gp_status transpose(Arena &A, const Csr &a, Csr *t, hipStream_t s) {
       if (st == GP_OK && hipMemsetAsync(t->rp, 0, sizeof(int64_t) * (a.nc + 1), s) != hipSuccess) st = fail(GP_ERR_HIP, "memset");
       break; }
     if ((st = tmp.alloc(&key, a.nnz)) != GP_OK) break;
-    k_transpose_keys<<<blocks_for(a.nr), 256, 0, s>>>(a.nr, a.rp, a.ci, a.nc, key);
+    k_transpose_keys<<<blocks_for(a.nnz), 256, 0, s>>>(a.nr, a.nnz, a.rp, a.ci, key);
     ValSrc vs{};
     vs.na = a.nv; vs.nb = 0; vs.nout = a.nv;
     for (int k = 0; k < 3; ++k) vs.a[k] = a.v[k];
@@ -490,26 +588,17 @@ __global__ void k_sell_fill(int64_t nr, const int64_t *__restrict__ rp, const in
 }
 
 // bad[0] += 1 for every stored column index outside [0, nc); bad[1], bad[2]:
-// smallest and largest index seen.  Each wavefront reduces its 64 lanes
-// (a grid-stride loop of them) first and issues one atomic of each kind.
+// smallest and largest such index.  Only wavefronts that hold one touch the
+// counters (atomics of every wavefront, the form before, took 375 us a matrix).
 __global__ void __launch_bounds__(256) k_sell_check(int64_t n, int64_t nc, const int32_t *__restrict__ ci,
                                                     int *__restrict__ bad) {
-  int cnt = 0, lo = 2147483647, hi = -2147483647 - 1;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
     const int c = ci[e];
-    cnt += (c < 0 || (int64_t)c >= nc) ? 1 : 0;
-    lo = min(lo, c);
-    hi = max(hi, c);
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    cnt += __shfl_xor(cnt, off, 64);
-    lo = min(lo, __shfl_xor(lo, off, 64));
-    hi = max(hi, __shfl_xor(hi, off, 64));
-  }
-  if ((threadIdx.x & 63) == 0) {
-    if (cnt) atomicAdd(bad, cnt);
-    atomicMin(bad + 1, lo);
-    atomicMax(bad + 2, hi);
+    if (c < 0 || (int64_t)c >= nc) {
+      atomicAdd(bad, 1);
+      atomicMin(bad + 1, c);
+      atomicMax(bad + 2, c);
+    }
   }
 }
 
@@ -591,33 +680,54 @@ __device__ __forceinline__ int32_t own_col(const int64_t *trp, const int32_t *tc
 __device__ __forceinline__ bool keep_entry(double v, int32_t c, double cut, int32_t own) {
   return fabs(v) >= cut || c == own;
 }
-__global__ void k_trunc_count(int64_t n, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                              const double *__restrict__ v, const int64_t *__restrict__ trp,
-                              const int32_t *__restrict__ tci, double theta, int64_t *__restrict__ cnt) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// One wavefront per row (a few rows hold thousands of entries); the kept entries
+// stay in order.
+__global__ void __launch_bounds__(256) k_trunc_count(int64_t n, const int64_t *__restrict__ rp,
+                                                     const int32_t *__restrict__ ci, const double *__restrict__ v,
+                                                     const int64_t *__restrict__ trp, const int32_t *__restrict__ tci,
+                                                     double theta, int64_t *__restrict__ cnt) {
+  const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (i >= n) return;  // uniform across the wavefront
+  const int64_t b = rp[i], e = rp[i + 1];
   double mx = 0.;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) mx = fmax(mx, fabs(v[p]));
+  for (int64_t p = b + lane; p < e; p += 64) mx = fmax(mx, fabs(v[p]));
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o));
   const int32_t own = own_col(trp, tci, i);
-  int64_t c = 0;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) c += keep_entry(v[p], ci[p], theta * mx, own) ? 1 : 0;
-  cnt[i] = c;
+  int c = 0;
+  for (int64_t p = b + lane; p < e; p += 64) c += keep_entry(v[p], ci[p], theta * mx, own) ? 1 : 0;
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+  if (lane == 0) cnt[i] = c;
 }
-__global__ void k_trunc_fill(int64_t n, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                             const double *__restrict__ v, const int64_t *__restrict__ trp,
-                             const int32_t *__restrict__ tci, double theta, const int64_t *__restrict__ orp,
-                             int32_t *__restrict__ oci, double *__restrict__ ov) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+__global__ void __launch_bounds__(256) k_trunc_fill(int64_t n, const int64_t *__restrict__ rp,
+                                                    const int32_t *__restrict__ ci, const double *__restrict__ v,
+                                                    const int64_t *__restrict__ trp, const int32_t *__restrict__ tci,
+                                                    double theta, const int64_t *__restrict__ orp,
+                                                    int32_t *__restrict__ oci, double *__restrict__ ov) {
+  const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (i >= n) return;  // uniform across the wavefront
+  const int64_t b = rp[i], e = rp[i + 1];
   double mx = 0., rs = 0., rk = 0.;
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p) { mx = fmax(mx, fabs(v[p])); rs += v[p]; }
+  for (int64_t p = b + lane; p < e; p += 64) { mx = fmax(mx, fabs(v[p])); rs += v[p]; }
+  for (int o = 32; o > 0; o >>= 1) { mx = fmax(mx, __shfl_xor(mx, o)); rs += __shfl_xor(rs, o); }
   const int32_t own = own_col(trp, tci, i);
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p)
+  for (int64_t p = b + lane; p < e; p += 64)
     if (keep_entry(v[p], ci[p], theta * mx, own)) rk += v[p];
+  for (int o = 32; o > 0; o >>= 1) rk += __shfl_xor(rk, o);
   const double sc = rk != 0. ? rs / rk : 1.;
   int64_t q = orp[i];
-  for (int64_t p = rp[i]; p < rp[i + 1]; ++p)
-    if (keep_entry(v[p], ci[p], theta * mx, own)) { oci[q] = ci[p]; ov[q] = v[p] * sc; ++q; }
+  for (int64_t p0 = b; p0 < e; p0 += 64) {
+    const int64_t p = p0 + lane;
+    const bool k = p < e && keep_entry(v[p], ci[p], theta * mx, own);
+    const unsigned long long m = __ballot(k);
+    if (k) {
+      const int64_t at = q + __popcll(m & ((1ull << lane) - 1));
+      oci[at] = ci[p];
+      ov[at] = v[p] * sc;
+    }
+    q += __popcll(m);
+  }
 }
 }  // namespace
 
@@ -627,15 +737,55 @@ gp_status truncate_prolongation(Arena &A, Arena &tmp, const Csr &P, const Csr &P
   if (Pt.nr != n) return fail(GP_ERR_ARG, "truncate_prolongation: P and Pt differ in rows");
   int64_t *cnt, *off;
   GP_TRY(tmp.alloc(&cnt, std::max<int64_t>(n, 1))); GP_TRY(tmp.alloc(&off, n + 1));
-  k_trunc_count<<<blocks_for(n), 256, 0, s>>>(n, P.rp, P.ci, P.v[0], Pt.rp, Pt.ci, theta, cnt);
+  k_trunc_count<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(n, P.rp, P.ci, P.v[0], Pt.rp, Pt.ci, theta, cnt);
   GP_TRY(exclusive_scan_i64(cnt, off, n, s, tmp));
   int64_t nk = 0;
   GP_HIP(hipMemcpyAsync(&nk, off + n, sizeof(int64_t), hipMemcpyDeviceToHost, s));
   GP_HIP(hipStreamSynchronize(s));
   GP_TRY(csr_alloc(A, n, P.nc, nk, 1, out));
   GP_HIP(hipMemcpyAsync(out->rp, off, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice, s));
-  k_trunc_fill<<<blocks_for(n), 256, 0, s>>>(n, P.rp, P.ci, P.v[0], Pt.rp, Pt.ci, theta, off, out->ci, out->v[0]);
+  k_trunc_fill<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(n, P.rp, P.ci, P.v[0], Pt.rp, Pt.ci, theta, off, out->ci, out->v[0]);
   GP_HIP(hipStreamSynchronize(s));
+  return GP_OK;
+}
+
+namespace {
+__global__ void __launch_bounds__(256) k_norm_part(int64_t n, const double *__restrict__ x, double *__restrict__ part) {
+  __shared__ double sh[4];
+  double a = 0.;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) a += x[i] * x[i];
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = a;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+__global__ void __launch_bounds__(kNormBlocks) k_norm_fin(const double *__restrict__ part, double *__restrict__ out) {
+  __shared__ double sh[kNormBlocks];
+  sh[threadIdx.x] = part[threadIdx.x];
+  __syncthreads();
+  for (int h = kNormBlocks / 2; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *out = sqrt(sh[0]);
+}
+__global__ void k_div_by(int64_t n, const double *__restrict__ norm, double *__restrict__ x) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const double d = *norm;
+  if (i < n && d > 0.) x[i] /= d;
+}
+}  // namespace
+
+gp_status dev_norm(const double *x, int64_t n, double *part, double *out, hipStream_t s) {
+  k_norm_part<<<kNormBlocks, 256, 0, s>>>(n, x, part);
+  k_norm_fin<<<1, kNormBlocks, 0, s>>>(part, out);
+  GP_HIP(hipGetLastError());
+  return GP_OK;
+}
+
+gp_status dev_div(double *x, int64_t n, const double *norm, hipStream_t s) {
+  k_div_by<<<blocks_for(n), 256, 0, s>>>(n, norm, x);
+  GP_HIP(hipGetLastError());
   return GP_OK;
 }
 

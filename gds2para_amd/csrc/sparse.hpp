@@ -101,6 +101,26 @@ gp_status spgemm(Arena &A, const Csr &a, const Csr &b, Csr *c, hipStream_t s);
 // rounded once (the exact product of the FP64 inputs, to 1 ulp)
 gp_status spgemm_ex(Arena &A, const Csr &a, const Csr &b, Csr *c, hipStream_t s, int exact);
 gp_status transpose(Arena &A, const Csr &a, Csr *t, hipStream_t s);
+// Row of stored entry p of a CSR of nr rows (empty rows allowed): kernels over
+// entries take it by bisection, ~18 cached reads, so that no thread walks one
+// of the conductor aggregates' rows of up to 1e5 entries alone.
+__device__ __forceinline__ int64_t csr_row_of(const int64_t *__restrict__ rp, int64_t nr, int64_t p) {
+  int64_t lo = 0, hi = nr;  // rp[lo] <= p < rp[hi]
+  while (hi - lo > 1) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (rp[mid] <= p) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+
+// *out = sqrt(sum x^2) of a device vector, on the device (two launches, fixed
+// order); part holds kNormBlocks doubles.
+constexpr int kNormBlocks = 256;
+gp_status dev_norm(const double *x, int64_t n, double *part, double *out, hipStream_t s);
+// x /= *norm (device scalar; a norm of zero leaves x)
+gp_status dev_div(double *x, int64_t n, const double *norm, hipStream_t s);
+
 // copy of a single-valued CSR without its explicit zeros
 gp_status csr_drop_zeros(Arena &A, const Csr &a, Csr *out, hipStream_t s);
 // fill nlong / lrows / lidx (see kLongRow)

@@ -103,3 +103,35 @@ def test_dense_inverse_of_stalled_coarsening(n):
     ref = np.empty(n)
     ref[n - 1 - i] = b / v
     assert np.linalg.norm(x - ref) <= 1e-12 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("runs", [(1, 47, 48, 49), (1023, 1024, 1025, 5), (2047, 2049, 3500, 2)])
+def test_duplicate_sums(runs):
+    """Triplets of equal (row, column) are summed by one thread up to 48 of
+    them and by a workgroup, 1024 at a time, above: a diagonal matrix given as
+    runs of such triplets.  A sum of m terms of one sign is off by m eps at
+    most."""
+    from gds2para_amd.layout import solve_real
+    rng = np.random.default_rng(sum(runs))
+    n = len(runs)
+    row = np.repeat(np.arange(n, dtype=np.int64), runs)
+    val = rng.uniform(0.5, 1.5, len(row))
+    b = rng.standard_normal(n)
+    print(f"[kernels] sums of {runs} triplets", flush=True)
+    x, it, rr = solve_real(row, row, val, n, b, rtol=1e-10)
+    d = np.array([float(np.sum(val[row == i].astype(np.longdouble))) for i in range(n)])
+    assert np.all(np.abs(x - b / d) <= 4 * max(runs) * 2.3e-16 * np.abs(b / d))
+
+
+def test_ad_sums_in_order():
+    """Ad of 48x48x12, whose conductor aggregates sum up to 12,000 terms into
+    one entry: the same bits as the oracle's sums in the reference's order."""
+    import oracle
+    m = M.Mesh(M.WORKLOADS["manhattan_48x48x12"]())
+    lay = Layout(m)
+    lay.build_v0()
+    print("[kernels] Ad sums of 48x48x12", flush=True)
+    got, ref = lay.v0d(), oracle.v0d(m)
+    for k in ("ad_row", "ad_col", "ad_val"):
+        assert np.array_equal(got[k], ref[k]), k
+    lay.close()
