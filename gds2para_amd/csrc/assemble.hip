@@ -170,7 +170,7 @@ extern "C" gp_status gp_assemble_stiffness(gp_layout *lay) {
   CsrD &S = lay->S;
   S.n = n;
   GP_TRY(lay->arena.alloc(&S.rp, n + 1));
-  Arena tmp;
+  TmpArena tmp;
   int64_t *cnt = nullptr;
   gp_status st = tmp.alloc(&cnt, n);
   if (st == GP_OK) {

@@ -267,9 +267,9 @@ __global__ void k_fill_hash(int64_t n, double *__restrict__ x) {
   if (i < n) x[i] = 0.5 + 0.5 * (double)((i * 2654435761ULL) % 1000) / 1000.0;
 }
 
-gp_status dense_host_aux(const Csr &M, int which, int64_t n, std::vector<double> *out) {
+gp_status dense_host_aux(const Csr &M, int which, int64_t n, std::vector<double> *out, hipStream_t s) {
   HostCsr h;
-  GP_TRY(csr_host_copy(M, &h, which));
+  GP_TRY(csr_host_copy(M, &h, which, s));
   out->assign(n * n, 0.0);
   for (int64_t i = 0; i < n; ++i)
     for (int64_t p = h.rp[i]; p < h.rp[i + 1]; ++p) (*out)[i * n + h.ci[p]] += h.v[p];
@@ -287,7 +287,7 @@ gp_status build_aux(gp_layout *lay, Arena &A, Hierarchy *H) {
   const int64_t nd = V.v0d_cols, nc = V.v0c_cols, naux = nd + nc;
   X.naux = naux;
   X.ndiel = V.ndiel;
-  Arena tmp;
+  TmpArena tmp;
   gp_status st = GP_OK;
   do {
     // Gx = [V0d | V0c] on the kept edges
@@ -450,7 +450,7 @@ gp_status build_aux(gp_layout *lay, Arena &A, Hierarchy *H) {
     }
     const AuxLevel &C = X.L.back();
     X.nL = C.n;
-    for (int k = 0; k < 2; ++k) GP_TRY(dense_host_aux(C.N, k, C.n, &X.NL[k]));
+    for (int k = 0; k < 2; ++k) GP_TRY(dense_host_aux(C.N, k, C.n, &X.NL[k], s));
     if (hipStreamSynchronize(s) != hipSuccess || hipGetLastError() != hipSuccess) { st = fail(GP_ERR_HIP, "aux setup kernels"); break; }
   } while (0);
   (void)hipStreamSynchronize(s);

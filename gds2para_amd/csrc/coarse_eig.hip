@@ -122,7 +122,7 @@ gp_status aux_coarse_eigen(Arena &A, AuxAMG &X, hipStream_t s) {
   if (rocblas_create_handle(&h) != rocblas_status_success) return fail(GP_ERR_HIP, "rocblas_create_handle failed");
   struct HandleGuard { rocblas_handle h; ~HandleGuard() { rocblas_destroy_handle(h); } } hg{h};
   if (rocblas_set_stream(h, s) != rocblas_status_success) return fail(GP_ERR_HIP, "rocblas_set_stream failed");
-  Arena T;
+  TmpArena T;
   struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
   double *a = nullptr, *b = nullptr, *e = nullptr, *lam = nullptr;
   rocblas_int *info = nullptr;

@@ -298,7 +298,7 @@ namespace {
 template <class Z>
 gp_status inverse(Z *a, int n, int nb, hipStream_t s) {
   if (n <= 0 || nb <= 0) return GP_OK;
-  Arena T;
+  TmpArena T;
   struct Free { Arena &a; hipStream_t s; ~Free() { (void)hipStreamSynchronize(s); a.free_all(); } } fr{T, s};
   Z *t0 = nullptr, *t1 = nullptr;
   int32_t *rc = nullptr, *used = nullptr;

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <iterator>
+#include <map>
 #include <memory>
 #include <string>
 #include <vector>
@@ -35,7 +37,103 @@ inline unsigned blocks_for(int64_t n, int threads = 256) {
   return (unsigned)b;
 }
 
-// Device allocation with a byte counter (the layout's footprint).
+// Temporaries of one setup call (hierarchy, V0 basis, real AMG): those calls
+// make thousands of short-lived buffers, and hipMalloc / hipFree (which waits
+// for the device) took half of their time: 220 of 445 ms for the hierarchy at
+// 128x128x16.  A ScratchScope keeps the memory of the temporary arenas
+// (TmpArena) of its thread until it ends, carving buffers from a few chunks.
+// A freed range is handed out again at once, which is safe because everything
+// inside a scope runs on the scope's one stream; at its end the scope waits for
+// that stream and gives everything back, so nothing outlives the call and no
+// two threads share a pool.
+class ScratchPool {
+ public:
+  void *get(size_t bytes) {
+    bytes = (bytes + 511) & ~(size_t)511;
+    if (bytes > kDirect) return nullptr;
+    auto best = free_.end();
+    for (auto it = free_.begin(); it != free_.end(); ++it)
+      if (it->second >= bytes && (best == free_.end() || it->second < best->second)) best = it;
+    if (best == free_.end()) {
+      size_t c = next_ > bytes ? next_ : bytes;
+      void *p = nullptr;
+      if (hipMalloc(&p, c) != hipSuccess) {
+        (void)hipGetLastError();
+        c = bytes;
+        if (hipMalloc(&p, c) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+      }
+      if (next_ < kChunkMax) next_ *= 2;
+      chunk_[(char *)p] = c;
+      best = free_.emplace((char *)p, c).first;
+    }
+    char *p = best->first;
+    const size_t left = best->second - bytes;
+    free_.erase(best);
+    if (left) free_[p + bytes] = left;
+    used_[p] = bytes;
+    return p;
+  }
+  // false: not one of this pool's buffers
+  bool put(void *q) {
+    auto u = used_.find((char *)q);
+    if (u == used_.end()) return false;
+    char *p = u->first;
+    size_t n = u->second;
+    used_.erase(u);
+    auto next = free_.lower_bound(p);
+    if (next != free_.end() && next->first == p + n && !chunk_.count(next->first)) {
+      n += next->second;
+      next = free_.erase(next);
+    }
+    if (next != free_.begin() && !chunk_.count(p)) {
+      auto prev = std::prev(next);
+      if (prev->first + prev->second == p) { prev->second += n; return true; }
+    }
+    free_[p] = n;
+    return true;
+  }
+  bool empty() const { return chunk_.empty(); }
+  void drop() {
+    for (auto &c : chunk_) (void)hipFree(c.first);
+    chunk_.clear();
+    free_.clear();
+    used_.clear();
+  }
+
+ private:
+  static constexpr size_t kDirect = (size_t)512 << 20;    // larger buffers are allocated by themselves
+  static constexpr size_t kChunkMax = (size_t)256 << 20;
+  size_t next_ = (size_t)8 << 20;
+  std::map<char *, size_t> chunk_, free_, used_;
+};
+
+inline thread_local ScratchPool *t_scratch = nullptr;
+
+struct ScratchScope {
+  explicit ScratchScope(hipStream_t s) : s_(s), outer_(t_scratch != nullptr) {
+    if (!outer_) t_scratch = &pool_;
+  }
+  ~ScratchScope() {
+    if (outer_) return;
+    t_scratch = nullptr;
+    if (pool_.empty()) return;
+    (void)hipStreamSynchronize(s_);
+    pool_.drop();
+  }
+  ScratchScope(const ScratchScope &) = delete;
+  ScratchScope &operator=(const ScratchScope &) = delete;
+
+ private:
+  hipStream_t s_;
+  bool outer_;
+  ScratchPool pool_;
+};
+
+// Device allocation with a byte counter (the layout's footprint: the bytes asked
+// for).  Buffers up to kSmall bytes are cut from slabs that live until free_all:
+// a layout holds hundreds, and each hipMalloc / hipFree costs 40-200 us (38 of
+// 134 ms of a whole 48x48x12 run was hipFree).  Slabs double from 64 KB to
+// 32 MB, so the ends left unused stay below what the arena holds.
 struct Arena {
   int64_t bytes = 0;
   std::vector<void *> owned;
@@ -43,31 +141,81 @@ struct Arena {
   gp_status alloc(T **p, int64_t n) {
     *p = nullptr;
     if (n <= 0) return GP_OK;
-    hipError_t e = hipMalloc((void **)p, sizeof(T) * (size_t)n);
-    if (e != hipSuccess) {
-      *p = nullptr;
-      (void)hipGetLastError();
-      return fail(GP_ERR_NOMEM, "hipMalloc of " + std::to_string(sizeof(T) * (size_t)n) + " bytes failed");
+    const size_t b = sizeof(T) * (size_t)n;
+    void *q = nullptr;
+    if (tmp_ && t_scratch) q = t_scratch->get(b);
+    if (!tmp_ && b <= kSmall) {
+      const size_t need = (b + 255) & ~(size_t)255;
+      if (need > slab_left_) {
+        const size_t size = slab_next_ > need ? slab_next_ : need;
+        if (hipMalloc(&q, size) == hipSuccess) {
+          owned.push_back(q);
+          slab_ = (char *)q;
+          slab_left_ = size;
+          if (slab_next_ < ((size_t)32 << 20)) slab_next_ *= 2;
+        } else {
+          (void)hipGetLastError();
+        }
+        q = nullptr;
+      }
+      if (need <= slab_left_) {
+        *p = (T *)slab_;
+        slab_ += need;
+        slab_left_ -= need;
+        bytes += (int64_t)b;
+        return GP_OK;
+      }
     }
-    bytes += (int64_t)(sizeof(T) * (size_t)n);
-    owned.push_back(*p);
+    if (!q) {
+      const hipError_t e = hipMalloc(&q, b);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(GP_ERR_NOMEM, "hipMalloc of " + std::to_string(b) + " bytes failed");
+      }
+    }
+    *p = (T *)q;
+    bytes += (int64_t)b;
+    owned.push_back(q);
     return GP_OK;
   }
   template <class T>
   void release(T *&p, int64_t n) {
     if (!p) return;
-    for (auto &q : owned)
-      if (q == (void *)p) { q = nullptr; break; }
-    (void)hipFree(p);
     bytes -= (int64_t)(sizeof(T) * (size_t)n);
+    for (auto &q : owned)
+      if (q == (void *)p) {
+        // the first buffer of a slab shares the slab's address: it stays with the rest of it
+        if (tmp_ || sizeof(T) * (size_t)n > kSmall) { give_back(q); q = nullptr; }
+        break;
+      }
     p = nullptr;
   }
   void free_all() {
     for (void *q : owned)
-      if (q) (void)hipFree(q);
+      if (q) give_back(q);
     owned.clear();
     bytes = 0;
+    slab_ = nullptr;
+    slab_left_ = 0;
+    slab_next_ = kSlabFirst;
   }
+
+ protected:
+  bool tmp_ = false;
+
+ private:
+  static constexpr size_t kSmall = (size_t)8 << 20, kSlabFirst = (size_t)64 << 10;
+  char *slab_ = nullptr;
+  size_t slab_left_ = 0, slab_next_ = kSlabFirst;
+  void give_back(void *q) {
+    if (!(tmp_ && t_scratch && t_scratch->put(q))) (void)hipFree(q);
+  }
+};
+
+// Buffers that live for one function: from the thread's ScratchScope, if one is
+// open, else allocated as they are.
+struct TmpArena : Arena {
+  TmpArena() { tmp_ = true; }
 };
 
 // Deep host copy of a gp_mesh so the caller's arrays may be released.

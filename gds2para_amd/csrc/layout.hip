@@ -144,7 +144,7 @@ extern "C" gp_status gp_layout_create(const gp_mesh *mesh, gp_layout **out) {
   GP_HIP(hipMemcpyAsync(lay->mark_node, m.mark_node, sizeof(int32_t) * g.Nn, hipMemcpyHostToDevice, s));
   GP_HIP(hipMemsetAsync(lay->rm_edge, 0, g.Ne, s));
   GP_HIP(hipMemsetAsync(lay->bd_node, 0, g.Nn, s));
-  Arena tmp;
+  TmpArena tmp;
   int64_t *d_idx = nullptr, *cnt = nullptr, *before = nullptr;
   int64_t nb = std::max<int64_t>(m.num_bd_edges, m.num_bd_nodes);
   gp_status st = GP_OK;

@@ -139,9 +139,9 @@ gp_status d2f_copy(const double *src, float *dst, int64_t n, hipStream_t s) {
 
 namespace {
 
-gp_status dense_host(const Csr &M, int which, int64_t nr, int64_t nc, std::vector<double> *out) {
+gp_status dense_host(const Csr &M, int which, int64_t nr, int64_t nc, std::vector<double> *out, hipStream_t s) {
   HostCsr h;
-  GP_TRY(csr_host_copy(M, &h, which));
+  GP_TRY(csr_host_copy(M, &h, which, s));
   out->assign(nr * nc, 0.0);
   for (int64_t i = 0; i < nr; ++i)
     for (int64_t p = h.rp[i]; p < h.rp[i + 1]; ++p) (*out)[i * nc + h.ci[p]] += h.v[p];
@@ -174,7 +174,7 @@ __global__ void k_tile_keys(int64_t n, const int64_t *__restrict__ map_r, Grid g
 gp_status level0_order(gp_layout *lay, Arena &A, int32_t **order, hipStream_t s) {
   const int64_t n = lay->n;
   *order = nullptr;
-  Arena tmp;
+  TmpArena tmp;
   uint64_t *k1, *k2;
   int32_t *i1;
   GP_TRY(tmp.alloc(&k1, n)); GP_TRY(tmp.alloc(&k2, n)); GP_TRY(tmp.alloc(&i1, n));
@@ -271,7 +271,7 @@ gp_status build_edge_march(gp_layout *lay, Arena &A, Hierarchy *H, hipStream_t s
   M.nplane = (int32_t)(g.Nz + 1);
   M.nblk = M.ntile * M.nplane * 2;
   if (M.nblk >= ((int64_t)1 << 30)) return GP_OK;
-  Arena tmp;
+  TmpArena tmp;
   int32_t *blk, *inv, *bad;
   unsigned long long *outside;
   GP_TRY(tmp.alloc(&blk, n)); GP_TRY(tmp.alloc(&inv, n)); GP_TRY(tmp.alloc(&bad, 1));
@@ -444,6 +444,7 @@ gp_status build_hierarchy(gp_layout *lay, Arena &A, Hierarchy *H, bool want_f32,
   auto t0 = std::chrono::steady_clock::now();
   if (!lay->s_ready) GP_TRY(gp_assemble_stiffness(lay));
   hipStream_t s = lay->stream;
+  ScratchScope scratch(s);
   const gp_mesh &m = lay->hm.view;
   std::vector<LevelGrid> grids(1);
   level0_grid(m, &grids[0]);
@@ -511,16 +512,17 @@ gp_status build_hierarchy(gp_layout *lay, Arena &A, Hierarchy *H, bool want_f32,
     MgLevel Cl;
     Cl.ne = c.ne();
     Cl.nn = c.nn();
+    TmpArena tmp;
     Csr tmpc;
-    GP_TRY(spgemm(A, F.K, F.P, &tmpc, s));
+    GP_TRY(spgemm(tmp, F.K, F.P, &tmpc, s));
     GP_TRY(spgemm(A, F.PT, tmpc, &Cl.K, s));
-    csr_release(A, tmpc);
-    GP_TRY(spgemm(A, F.B, F.Pn, &tmpc, s));
+    csr_release(tmp, tmpc);
+    GP_TRY(spgemm(tmp, F.B, F.Pn, &tmpc, s));
     GP_TRY(spgemm(A, F.PT, tmpc, &Cl.B, s));
-    csr_release(A, tmpc);
-    GP_TRY(spgemm(A, F.N, F.Pn, &tmpc, s));
+    csr_release(tmp, tmpc);
+    GP_TRY(spgemm(tmp, F.N, F.Pn, &tmpc, s));
     GP_TRY(spgemm(A, F.PnT, tmpc, &Cl.N, s));
-    csr_release(A, tmpc);
+    csr_release(tmp, tmpc);
     GP_TRY(csr_upload(A, hg, &Cl.G, s));
     GP_TRY(transpose(A, Cl.G, &Cl.GT, s));
     grids.push_back(std::move(c));
@@ -555,7 +557,7 @@ gp_status build_hierarchy(gp_layout *lay, Arena &A, Hierarchy *H, bool want_f32,
     MgLevel &L = H->L[l];
     const int32_t *oe = l == 0 ? H->ord_e : nullptr, *on = l == 0 ? H->ord_n : nullptr;
     if (l == 0 && L.K.sdg) {  // level 0: the SELL copy of K holds the off-diagonal entries
-      Arena tmp;
+      TmpArena tmp;
       Csr K2 = L.K;
       K2.sdg = nullptr; K2.dg[0] = K2.dg[1] = nullptr;
       int64_t *cnt;
@@ -568,6 +570,7 @@ gp_status build_hierarchy(gp_layout *lay, Arena &A, Hierarchy *H, bool want_f32,
       k_offdiag_fill<<<blocks_for(L.K.nr), 256, 0, s>>>(L.K.nr, L.K.rp, L.K.ci, L.K.v[0], K2.rp, K2.ci, K2.v[0]);
       GP_TRY(sell_from_csr(A, K2, &L.Ks, s, "L.K off-diagonal", oe));
       GP_HIP(hipStreamSynchronize(s));
+      tmp.free_all();
       L.K.nsdg = L.K.nnz - K2.nnz;
     } else {
       GP_TRY(sell_from_csr(A, L.K, &L.Ks, s, "L.K", oe));
@@ -583,10 +586,10 @@ gp_status build_hierarchy(gp_layout *lay, Arena &A, Hierarchy *H, bool want_f32,
   const MgLevel &C = H->L.back();
   H->neL = C.ne;
   H->nnL = C.nn;
-  for (int k = 0; k < 3; ++k) GP_TRY(dense_host(C.K, k, C.ne, C.ne, &H->KL[k]));
-  for (int k = 0; k < 2; ++k) GP_TRY(dense_host(C.B, k, C.ne, C.nn, &H->BL[k]));
-  for (int k = 0; k < 2; ++k) GP_TRY(dense_host(C.N, k, C.nn, C.nn, &H->NL[k]));
-  GP_TRY(dense_host(C.GT, 0, C.nn, C.ne, &H->GTL));
+  for (int k = 0; k < 3; ++k) GP_TRY(dense_host(C.K, k, C.ne, C.ne, &H->KL[k], s));
+  for (int k = 0; k < 2; ++k) GP_TRY(dense_host(C.B, k, C.ne, C.nn, &H->BL[k], s));
+  for (int k = 0; k < 2; ++k) GP_TRY(dense_host(C.N, k, C.nn, C.nn, &H->NL[k], s));
+  GP_TRY(dense_host(C.GT, 0, C.nn, C.ne, &H->GTL, s));
   GP_HIP(hipStreamSynchronize(s));
   GP_TRY(build_aux(lay, A, H));
   GP_TRY(aux_coarse_blocks(A, H->aux, s));
@@ -775,7 +778,7 @@ gp_status coarse_make_room(CoarseCache &C, int64_t add, hipStream_t s) {
 // The auxiliary coarsest level's inverse at angular frequency w, block by
 // block (AuxAMG::nblk), packed into inv (block b at offset ioff[b]).
 gp_status aux_coarse_inverse(const AuxAMG &X, double w, C2<double> *inv, hipStream_t s) {
-  Arena T;
+  TmpArena T;
   struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
   C2<double> *aug = nullptr;
   int *bad = nullptr;
@@ -830,7 +833,7 @@ gp_status aux_coarse_dense(const Hierarchy &H, double w, std::vector<std::comple
       }
     return GP_OK;
   }
-  Arena T;
+  TmpArena T;
   struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
   C2<double> *d = nullptr;
   GP_TRY(T.alloc(&d, std::max<int64_t>(X.inv_len, 1)));
@@ -851,6 +854,7 @@ gp_status aux_coarse_dense(const Hierarchy &H, double w, std::vector<std::comple
 gp_status coarse_cache_lookup(const Hierarchy &H, CoarseCache &C, const std::vector<double> &omegas,
                               std::vector<int32_t> *slots, hipStream_t s, int pin) {
   const auto t0 = std::chrono::steady_clock::now();
+  ScratchScope scratch(s);
   slots->assign(omegas.size(), -1);
   const int64_t ne = H.neL, nn = H.nnL, na = H.aux.nL;
   const int64_t eb = coarse_entry_bytes(H);
@@ -861,7 +865,7 @@ gp_status coarse_cache_lookup(const Hierarchy &H, CoarseCache &C, const std::vec
     for (int32_t t = 0; t < (int32_t)C.e.size(); ++t)
       if (C.e[t].mem && C.e[t].omega == omegas[i]) { q = t; break; }
     if (q < 0) {
-      Arena T;
+      TmpArena T;
       struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
       C2<double> *nbuf = nullptr;
       GP_TRY(T.alloc(&nbuf, nn * nn));

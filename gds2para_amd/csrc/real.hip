@@ -531,7 +531,7 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
     GP_TRY(A.alloc(&F.r, n)); GP_TRY(A.alloc(&F.x, n)); GP_TRY(A.alloc(&F.t, n));
     GP_TRY(long_rows(A, F.A, &F.la, &F.nla, s));
     if (n <= kCoarsest || G.L.size() >= 24) break;
-    Arena tmp;
+    TmpArena tmp;
     gp_status st = GP_OK;
     Csr P1, M2, AP1, P2, Pt, DA, DAP, Ps, P, AP, Ac, R;
     do {
@@ -753,7 +753,8 @@ extern "C" gp_status gp_solve_real_ex(const int64_t *row, const int64_t *col, co
   hipStream_t s;
   GP_HIP(hipStreamCreate(&s));
   struct StreamGuard { hipStream_t s; ~StreamGuard() { (void)hipStreamSynchronize(s); (void)hipStreamDestroy(s); } } sg{s};
-  Arena tmp;
+  ScratchScope scratch(s);
+  TmpArena tmp;
   struct TGuard { Arena *a; hipStream_t s; ~TGuard() { (void)hipStreamSynchronize(s); a->free_all(); } } tg{&tmp, s};
   int64_t *dr, *dc;
   double *dv, *bd, *xd;

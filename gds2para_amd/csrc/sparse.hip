@@ -219,7 +219,7 @@ int bits_for(uint64_t maxkey) {
 // Sort (key, src) pairs and reduce equal keys into a CSR with nout value arrays.
 gp_status sort_reduce(Arena &A, int64_t nr, int64_t nc, int64_t nprod, uint64_t *key, const uint32_t *src_a,
                       const uint32_t *src_b, ValSrc vs, Csr *out, hipStream_t s) {
-  Arena tmp;
+  TmpArena tmp;
   gp_status st = GP_OK;
   uint64_t *key2 = nullptr;
   uint32_t *perm = nullptr, *perm2 = nullptr;
@@ -285,7 +285,7 @@ __global__ void k_csr_triplets(int64_t nr, int64_t nnz, const int64_t *__restric
 
 gp_status csr_from_coo(Arena &A, int64_t nr, int64_t nc, int64_t n, const int64_t *rows, const int64_t *cols,
                        const double *const *vals, int nv, Csr *out, hipStream_t s) {
-  Arena tmp;
+  TmpArena tmp;
   uint64_t *key = nullptr;
   gp_status st = GP_OK;
   do {
@@ -306,7 +306,7 @@ gp_status csr_from_coo(Arena &A, int64_t nr, int64_t nc, int64_t n, const int64_
 
 gp_status csr_add(Arena &A, const Csr &a, double alpha, const Csr &b, Csr *c, hipStream_t s) {
   if (a.nr != b.nr || a.nc != b.nc) return fail(GP_ERR_ARG, "csr_add shape mismatch");
-  Arena tmp;
+  TmpArena tmp;
   int64_t *r = nullptr, *cc = nullptr;
   double *v = nullptr;
   const int64_t n = a.nnz + b.nnz;
@@ -343,7 +343,7 @@ __global__ void k_nz_compact(int64_t nr, int64_t nnz, const int64_t *__restrict_
 }  // namespace
 
 gp_status csr_drop_zeros(Arena &A, const Csr &a, Csr *out, hipStream_t s) {
-  Arena tmp;
+  TmpArena tmp;
   gp_status st = GP_OK;
   int64_t *f = nullptr, *pos = nullptr, *r = nullptr, *c = nullptr;
   double *v = nullptr;
@@ -399,7 +399,7 @@ gp_status spgemm(Arena &A, const Csr &a, const Csr &b, Csr *c, hipStream_t s) { 
 gp_status spgemm_ex(Arena &A, const Csr &a, const Csr &b, Csr *c, hipStream_t s, int exact) {
   if (a.nc != b.nr) return fail(GP_ERR_ARG, "spgemm shape mismatch");
   if (a.nv > 1 && b.nv > 1 && a.nv != b.nv) return fail(GP_ERR_ARG, "spgemm value arrays mismatch");
-  Arena tmp;
+  TmpArena tmp;
   gp_status st = GP_OK;
   int64_t *cnt = nullptr, *off = nullptr;
   int32_t *arow = nullptr;
@@ -446,7 +446,7 @@ __global__ void k_transpose_keys(int64_t nr, int64_t nnz, const int64_t *__restr
 }  // namespace
 
 gp_status transpose(Arena &A, const Csr &a, Csr *t, hipStream_t s) {
-  Arena tmp;
+  TmpArena tmp;
   uint64_t *key = nullptr;
   gp_status st = GP_OK;
   do {
@@ -525,16 +525,17 @@ gp_status csr_mark_long(Arena &A, Csr &a, hipStream_t s) {
   return GP_OK;
 }
 
-gp_status csr_host_copy(const Csr &a, HostCsr *h, int which) {
+gp_status csr_host_copy(const Csr &a, HostCsr *h, int which, hipStream_t s) {
   h->nr = a.nr; h->nc = a.nc;
   h->rp.resize(a.nr + 1);
   h->ci.resize(a.nnz);
   h->v.resize(a.nnz);
-  GP_HIP(hipMemcpy(h->rp.data(), a.rp, sizeof(int64_t) * (a.nr + 1), hipMemcpyDeviceToHost));
+  GP_HIP(hipMemcpyAsync(h->rp.data(), a.rp, sizeof(int64_t) * (a.nr + 1), hipMemcpyDeviceToHost, s));
   if (a.nnz) {
-    GP_HIP(hipMemcpy(h->ci.data(), a.ci, sizeof(int32_t) * a.nnz, hipMemcpyDeviceToHost));
-    GP_HIP(hipMemcpy(h->v.data(), a.v[which], sizeof(double) * a.nnz, hipMemcpyDeviceToHost));
+    GP_HIP(hipMemcpyAsync(h->ci.data(), a.ci, sizeof(int32_t) * a.nnz, hipMemcpyDeviceToHost, s));
+    GP_HIP(hipMemcpyAsync(h->v.data(), a.v[which], sizeof(double) * a.nnz, hipMemcpyDeviceToHost, s));
   }
+  GP_HIP(hipStreamSynchronize(s));
   return GP_OK;
 }
 
@@ -615,7 +616,7 @@ gp_status sell_from_csr(Arena &A, const Csr &a, Sell *out, hipStream_t s, const 
   out->nv = a.nv;
   out->nslice = (a.nr + 63) / 64;
   if (a.nr == 0) return GP_OK;
-  Arena tmp;
+  TmpArena tmp;
   gp_status st = GP_OK;
   do {
     int64_t *cnt = nullptr;

@@ -138,7 +138,8 @@ gp_status csr_add(Arena &A, const Csr &a, double alpha, const Csr &b, Csr *c, hi
 // scaled so that every row keeps its sum.
 gp_status truncate_prolongation(Arena &A, Arena &tmp, const Csr &P, const Csr &Pt, double theta, Csr *out,
                                 hipStream_t s);
-// host copy of value array `which` of a
-gp_status csr_host_copy(const Csr &a, HostCsr *h, int which);
+// host copy of value array `which` of a, on stream s (a copy on the legacy stream
+// fails while another thread's solve captures its preconditioner)
+gp_status csr_host_copy(const Csr &a, HostCsr *h, int which, hipStream_t s);
 
 }  // namespace gp

@@ -336,7 +336,7 @@ __global__ void k_rank(int64_t ncn, const int64_t *__restrict__ nodes, const int
 static gp_status galerkin(gp_layout *lay, const Geo &G, const V0Coo &V, int64_t ncols, const int64_t *map,
                           int sigma_mode, int filter, V0Coo *out, int64_t *len_unfiltered, Arena &A) {
   hipStream_t s = lay->stream;
-  Arena tmp;
+  TmpArena tmp;
   gp_status st = GP_OK;
   int64_t *ncon = nullptr, *off = nullptr;
   uint64_t *key = nullptr, *key2 = nullptr;
@@ -408,8 +408,9 @@ gp_status build_v0(gp_layout *lay) {
   hipStream_t s = lay->stream;
   Arena &A = lay->arena;
   Geo G{lay->xn, lay->yn, lay->zn, g, m.nx, m.ny, m.nz};
+  ScratchScope scratch(s);
   auto *V = new V0Data();
-  Arena tmp;
+  TmpArena tmp;
   gp_status st = GP_OK;
   const int32_t ncdt = m.num_cdt;
   do {

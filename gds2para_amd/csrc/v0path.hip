@@ -102,6 +102,7 @@ unsigned wave_blocks(int64_t nr) { return (unsigned)((nr + 3) / 4); }
 gp_status setup(gp_layout *lay, V0Path **out) {
   auto t0 = std::chrono::steady_clock::now();
   hipStream_t s = lay->stream;
+  ScratchScope scratch(s);
   const V0Data &V = *lay->v0;
   V0Path *P = new V0Path();
   P->nd = V.v0d_cols;
@@ -260,7 +261,7 @@ extern "C" gp_status gp_solve_v0(gp_layout *lay, double rtol, double *Z0, double
     for (int64_t q = m.side_edge_ptr[s0]; q < m.side_edge_ptr[s0 + 1]; ++q) redge.push_back(m.side_edges[q]);
     rptr[p + 1] = (int64_t)redge.size();
   }
-  Arena tmp;
+  TmpArena tmp;
   struct TGuard { Arena *a; hipStream_t s; ~TGuard() { (void)hipStreamSynchronize(s); a->free_all(); } } tg{&tmp, s};
   const int64_t ne = P.ne, nd = P.nd, nc = P.nc;
   const int64_t nr = std::max<int64_t>((int64_t)redge.size(), 1);
@@ -350,7 +351,7 @@ extern "C" gp_status gp_v0_vh_inputs(gp_layout *lay, int32_t src, double rtol, d
   const double tol = rtol > 0 ? rtol : 1e-4;
   const double w0 = 2 * kPi * m.freq_start * m.freq_unit;
   const int64_t ne = P.ne, nd = P.nd, nc = P.nc, n = lay->n;
-  Arena tmp;
+  TmpArena tmp;
   struct TGuard { Arena *a; hipStream_t s; ~TGuard() { (void)hipStreamSynchronize(s); a->free_all(); } } tg{&tmp, s};
   PortBufs b;
   GP_TRY(tmp.alloc(&b.J, ne)); GP_TRY(tmp.alloc(&b.t, ne)); GP_TRY(tmp.alloc(&b.yd1, ne));

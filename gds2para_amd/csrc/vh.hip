@@ -285,7 +285,7 @@ extern "C" gp_status gp_find_vh(gp_layout *lay, int32_t k, double scale, double 
   if (k > len) return fail(GP_ERR_ARG, "gp_find_vh: more Arnoldi steps than the operator's dimension 2n");
   hipStream_t s = lay->stream;
   const auto t0 = std::chrono::steady_clock::now();
-  Arena T;
+  TmpArena T;
   struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
   double *V = nullptr, *w = nullptr, *h = nullptr, *h2 = nullptr;
   GP_TRY(T.alloc(&V, (int64_t)(k + 1) * len));

@@ -133,7 +133,7 @@ extern "C" gp_status gp_solve_vh(gp_layout *lay, const double *vh, int64_t leng_
   if (rocblas_create_handle(&h) != rocblas_status_success) return fail(GP_ERR_HIP, "rocblas_create_handle failed");
   struct HandleGuard { rocblas_handle h; ~HandleGuard() { rocblas_destroy_handle(h); } } hg{h};
   RB_TRY(rocblas_set_stream(h, s));
-  Arena T;
+  TmpArena T;
   struct Free { Arena &a; hipStream_t s; ~Free() { (void)hipStreamSynchronize(s); a.free_all(); } } fr{T, s};
   double2 *dVh, *dVp, *dT, *dU, *dUa, *dDU, *dY, *dM, *dYd, *dYw, *dR, *dRh, *d4;
   double *dEps, *dSig;
