@@ -21,6 +21,9 @@
 //     BoomerAMG's relaxation with HYPRE_BoomerAMGSetRelaxType,
 //     src/hypreSolve.cpp:230); dense FP64 inverse on the coarsest level
 //     (<= 512 unknowns).
+// A solve takes 1, 2, 4 or 8 right-hand sides side by side (vectors
+// interleaved, row i column j at i*K + j): every matrix entry and every launch
+// serves all of them, while each column keeps its own recurrence.
 #include <algorithm>
 #include <cmath>
 #include <complex>
@@ -193,184 +196,293 @@ __global__ void k_r_scale_rows(int64_t n, int64_t nnz, const int64_t *__restrict
   out[p] = (di != 0. ? f / di : 0.) * v[p];
 }
 
-// Row products split two ways: rows of at most kRLong entries take 8 lanes
-// each (k_r_spmv, k_r_jacobi), longer rows -- the conductor aggregate
-// columns of V0d couple to every dielectric node around a conductor -- take a
-// 256-thread block each (the *_long kernels), listed per matrix at setup.
-constexpr int kRLong = 64;
-constexpr int kRLanes = 8;
+// ---------------------------------------------------------------- products of K columns
 
-__device__ __forceinline__ double row_dot8(int64_t b, int64_t e, int lane, const int32_t *__restrict__ ci,
-                                           const double *__restrict__ v, const double *__restrict__ x) {
-  double s = 0.;
-  for (int64_t p = b + lane; p < e; p += kRLanes) s += v[p] * x[ci[p]];
-  for (int off = kRLanes / 2; off > 0; off >>= 1) s += __shfl_down(s, off, kRLanes);
-  return s;
-}
+// One row product s = sum a x of K columns and what is done with it:
+//   R_MUL:  y = alpha s (+ y); with z also the first sweep of y's level from
+//           zero, z = q, dd = q (if given) with q = zc y / zd
+//   R_RES:  y = r - s
+//   R_JAC:  y = x + (r - s) / d                      (l1-Jacobi, d = l1 diagonal)
+//   R_CHEB: q = c2 (r - s) / d + c1 dd;  dd = q;  y = x + q
+// (Chebyshev smoothing, the three-term recurrence written with a direction
+// vector dd, Saad, Iterative Methods for Sparse Linear Systems, 2nd ed., Alg.
+// 12.1, preconditioned with D^-1; c1 = 0 starts the recurrence from a nonzero
+// x, dd is then not read).  y may be r.
+enum RMode { R_MUL = 0, R_RES = 1, R_JAC = 2, R_CHEB = 3 };
 
-__device__ __forceinline__ double row_dot_block(int64_t b, int64_t e, const int32_t *__restrict__ ci,
-                                                const double *__restrict__ v, const double *__restrict__ x) {
-  __shared__ double sh[256];
-  double s = 0.;
-  for (int64_t p = b + threadIdx.x; p < e; p += blockDim.x) s += v[p] * x[ci[p]];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int st = blockDim.x / 2; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
+struct REp {
+  double *y = nullptr;
+  const double *r = nullptr;
+  double alpha = 1.;
+  int acc = 0;
+  const double *d = nullptr;
+  double c1 = 0., c2 = 0.;
+  double *dd = nullptr;
+  double *z = nullptr;
+  const double *zd = nullptr;
+  double zc = 0.;
+};
+
+template <int K, int MODE>
+__device__ __forceinline__ void r_row(const REp &ep, const double *x, int64_t i, int c, double s) {
+  const int64_t q = i * K + c;
+  if (MODE == R_MUL) {
+    double v = ep.alpha * s;
+    if (ep.acc) v = ep.y[q] + v;
+    ep.y[q] = v;
+    if (ep.z) {
+      const double d = ep.zd[i], f = d != 0. ? ep.zc * v / d : 0.;
+      ep.z[q] = f;
+      if (ep.dd) ep.dd[q] = f;
+    }
+  } else if (MODE == R_RES) {
+    ep.y[q] = ep.r[q] - s;
+  } else if (MODE == R_JAC) {
+    ep.y[q] = x[q] + (ep.r[q] - s) / ep.d[i];
+  } else {
+    const double d = ep.d[i];
+    double f = d != 0. ? ep.c2 * (ep.r[q] - s) / d : 0.;
+    if (ep.c1 != 0.) f += ep.c1 * ep.dd[q];
+    ep.dd[q] = f;
+    ep.y[q] = x[q] + f;
   }
-  return sh[0];
 }
 
-// y = A x (mode 0), y = r - A x (mode 1), y = y + A x (mode 2)
-__global__ void k_r_spmv(int64_t n, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                         const double *__restrict__ v, const double *__restrict__ x, const double *__restrict__ r,
-                         double *__restrict__ y, int mode) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kRLanes;
-  const int lane = threadIdx.x & (kRLanes - 1);
-  if (i >= n) return;
+template <int K>
+__device__ __forceinline__ void r_load(const double *__restrict__ p, double (&v)[K]) {
+  if constexpr (K == 1) {
+    v[0] = p[0];
+  } else {
+#pragma unroll
+    for (int h = 0; h < K / 2; ++h) {
+      const double2 t = reinterpret_cast<const double2 *>(p)[h];
+      v[2 * h] = t.x;
+      v[2 * h + 1] = t.y;
+    }
+  }
+}
+
+// Sums the K columns over W lanes: each exchange halves the columns a lane
+// carries until it carries one (col), then halves the lanes.  Lanes whose
+// low W / K bits are zero hold column col's sum.
+template <int K, int W>
+__device__ __forceinline__ double r_reduce(const double (&a)[K], int lane, int &col) {
+  if constexpr (W == 1) {
+    return a[0];
+  } else if constexpr (K == 1) {
+    const double b[1] = {a[0] + __shfl_xor(a[0], W / 2)};
+    return r_reduce<1, W / 2>(b, lane, col);
+  } else {
+    constexpr int H = K / 2;
+    const bool up = (lane & (W / 2)) != 0;
+    double b[H];
+#pragma unroll
+    for (int q = 0; q < H; ++q) {
+      const double keep = up ? a[H + q] : a[q], send = up ? a[q] : a[H + q];
+      b[q] = keep + __shfl_xor(send, W / 2);
+    }
+    if (up) col += H;
+    return r_reduce<H, W / 2>(b, lane, col);
+  }
+}
+
+// The first nbw workgroups give every chunk of a listed row (kLongRow) a
+// wavefront, a lane per entry and K columns a lane; rows of several chunks
+// leave partial sums to k_rm_fin.  The rest take the short rows, 8 lanes each.
+// One workgroup per row above 64 entries, in a launch of its own (the layout
+// before), took 28 us a product at 200x200x24, whose longest rows hold 1e5
+// entries, and served one column.
+template <int K, int MODE>
+__global__ void __launch_bounds__(256) k_rm(int64_t nr, unsigned nbw, const int64_t *__restrict__ rp,
+                                            const int32_t *__restrict__ ci, const double *__restrict__ v,
+                                            const int32_t *__restrict__ lidx, const int32_t *__restrict__ lrows,
+                                            const int64_t *__restrict__ lcb, const int64_t *__restrict__ lce, int nchunk,
+                                            int nsingle, const double *x, REp ep, double *__restrict__ part) {
+  double a[K];
+#pragma unroll
+  for (int q = 0; q < K; ++q) a[q] = 0.;
+  if (blockIdx.x < nbw) {
+    const int c = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (c >= nchunk) return;  // uniform across the wavefront
+    const int lane = threadIdx.x & 63;
+    const int64_t b = lcb[c], e = lce[c];
+    constexpr int NB = (int)(kLongChunk / 64);
+    int32_t cc[NB];
+    double av[NB];
+#pragma unroll
+    for (int h = 0; h < NB; ++h) {  // past the end: the last entry's column with value 0
+      const int64_t p = b + h * 64 + lane, pp = p < e ? p : e - 1;
+      cc[h] = ci[pp];
+      av[h] = p < e ? v[pp] : 0.;
+    }
+#pragma unroll
+    for (int h = 0; h < NB; ++h) {
+      if (b + h * 64 >= e) break;
+      double xv[K];
+      r_load<K>(x + (int64_t)cc[h] * K, xv);
+#pragma unroll
+      for (int q = 0; q < K; ++q) a[q] += av[h] * xv[q];
+    }
+    int col = 0;
+    const double s = r_reduce<K, 64>(a, lane, col);
+    if (lane & (64 / K - 1)) return;
+    if (c < nsingle) r_row<K, MODE>(ep, x, lrows[c], col, s);
+    else part[(int64_t)(c - nsingle) * K + col] = s;
+    return;
+  }
+  const int64_t i = ((int64_t)(blockIdx.x - nbw) * 256 + threadIdx.x) >> 3;
+  const int lane = threadIdx.x & 7;
+  if (i >= nr || (lidx && lidx[i] >= 0)) return;  // the same on a row's 8 lanes
   const int64_t b = rp[i], e = rp[i + 1];
-  if (e - b > kRLong) return;
-  const double s = row_dot8(b, e, lane, ci, v, x);
-  if (lane == 0) y[i] = mode == 0 ? s : mode == 1 ? r[i] - s : y[i] + s;
+  constexpr int NB = (int)(kLongRow / 8);
+  int32_t cc[NB];
+  double av[NB];
+#pragma unroll
+  for (int h = 0; h < NB; ++h) {
+    const int64_t p = b + h * 8 + lane;
+    cc[h] = 0;
+    av[h] = 0.;
+    if (p < e) { cc[h] = ci[p]; av[h] = v[p]; }
+  }
+#pragma unroll
+  for (int h = 0; h < NB; ++h)
+    if (b + h * 8 + lane < e) {
+      double xv[K];
+      r_load<K>(x + (int64_t)cc[h] * K, xv);
+#pragma unroll
+      for (int q = 0; q < K; ++q) a[q] += av[h] * xv[q];
+    }
+  int col = 0;
+  const double s = r_reduce<K, 8>(a, lane, col);
+  if ((lane & (8 / K - 1)) == 0) r_row<K, MODE>(ep, x, i, col, s);
 }
+static_assert(kLongRow % 8 == 0 && kLongChunk % 64 == 0, "rounds of the row walks");
 
-__global__ void k_r_spmv_long(const int32_t *__restrict__ lrows, const int64_t *__restrict__ rp,
-                              const int32_t *__restrict__ ci, const double *__restrict__ v,
-                              const double *__restrict__ x, const double *__restrict__ r, double *__restrict__ y,
-                              int mode) {
-  const int64_t i = lrows[blockIdx.x];
-  const double s = row_dot_block(rp[i], rp[i + 1], ci, v, x);
-  if (threadIdx.x == 0) y[i] = mode == 0 ? s : mode == 1 ? r[i] - s : y[i] + s;
-}
-
-// l1-Jacobi, first sweep: xo = r / d
-__global__ void k_r_jacobi0(int64_t n, const double *__restrict__ dl1, const double *__restrict__ r,
-                            double *__restrict__ xo) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) xo[i] = 0. + r[i] / dl1[i];
-}
-
-// l1-Jacobi, later sweeps: xo = x + (r - A x) / d
-__global__ void k_r_jacobi(int64_t n, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                           const double *__restrict__ v, const double *__restrict__ dl1, const double *__restrict__ r,
-                           const double *__restrict__ x, double *__restrict__ xo) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kRLanes;
-  const int lane = threadIdx.x & (kRLanes - 1);
-  if (i >= n) return;
-  const int64_t b = rp[i], e = rp[i + 1];
-  if (e - b > kRLong) return;
-  const double s = row_dot8(b, e, lane, ci, v, x);
-  if (lane == 0) xo[i] = x[i] + (r[i] - s) / dl1[i];
-}
-
-__global__ void k_r_jacobi_long(const int32_t *__restrict__ lrows, const int64_t *__restrict__ rp,
-                                const int32_t *__restrict__ ci, const double *__restrict__ v,
-                                const double *__restrict__ dl1, const double *__restrict__ r,
-                                const double *__restrict__ x, double *__restrict__ xo) {
-  const int64_t i = lrows[blockIdx.x];
-  const double s = row_dot_block(rp[i], rp[i + 1], ci, v, x);
-  if (threadIdx.x == 0) xo[i] = x[i] + (r[i] - s) / dl1[i];
-}
-
-// Chebyshev smoothing (the three-term recurrence written with a direction
-// vector dd, Saad, Iterative Methods for Sparse Linear Systems, 2nd ed.,
-// Alg. 12.1, preconditioned with D^-1), first step from x = 0:
-// dd = c2 D^-1 r, xo = dd
-__global__ void k_r_cheb0(int64_t n, const double *__restrict__ dg, const double *__restrict__ r, double c2,
-                          double *__restrict__ dd, double *__restrict__ xo) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double q = dg[i] != 0. ? c2 * r[i] / dg[i] : 0.;
-  dd[i] = q;
-  xo[i] = q;
-}
-
-// later steps: dd = c1 dd + c2 D^-1 (r - A x), xo = x + dd (c1 = 0 starts the
-// recurrence from a nonzero x; dd is then not read)
-__device__ __forceinline__ void cheb_row(int64_t i, double s, const double *__restrict__ dg,
-                                         const double *__restrict__ r, const double *__restrict__ x, double c1,
-                                         double c2, double *__restrict__ dd, double *__restrict__ xo) {
-  double q = dg[i] != 0. ? c2 * (r[i] - s) / dg[i] : 0.;
-  if (c1 != 0.) q += c1 * dd[i];
-  dd[i] = q;
-  xo[i] = x[i] + q;
-}
-
-__global__ void k_r_cheb(int64_t n, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                         const double *__restrict__ v, const double *__restrict__ dg, const double *__restrict__ r,
-                         const double *__restrict__ x, double c1, double c2, double *__restrict__ dd,
-                         double *__restrict__ xo) {
-  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kRLanes;
-  const int lane = threadIdx.x & (kRLanes - 1);
-  if (i >= n) return;
-  const int64_t b = rp[i], e = rp[i + 1];
-  if (e - b > kRLong) return;
-  const double s = row_dot8(b, e, lane, ci, v, x);
-  if (lane == 0) cheb_row(i, s, dg, r, x, c1, c2, dd, xo);
-}
-
-__global__ void k_r_cheb_long(const int32_t *__restrict__ lrows, const int64_t *__restrict__ rp,
-                              const int32_t *__restrict__ ci, const double *__restrict__ v,
-                              const double *__restrict__ dg, const double *__restrict__ r,
-                              const double *__restrict__ x, double c1, double c2, double *__restrict__ dd,
-                              double *__restrict__ xo) {
-  const int64_t i = lrows[blockIdx.x];
-  const double s = row_dot_block(rp[i], rp[i + 1], ci, v, x);
-  if (threadIdx.x == 0) cheb_row(i, s, dg, r, x, c1, c2, dd, xo);
+// rows of several chunks: a wavefront per row sums the partial sums
+template <int K, int MODE>
+__global__ void __launch_bounds__(256) k_rm_fin(int nmulti, int nsingle, const int32_t *__restrict__ lrows,
+                                                const int32_t *__restrict__ lqp, const double *x, REp ep,
+                                                const double *__restrict__ part) {
+  const int r = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+  if (r >= nmulti) return;  // uniform across the wavefront
+  const int lane = threadIdx.x & 63;
+  double a[K];
+#pragma unroll
+  for (int q = 0; q < K; ++q) a[q] = 0.;
+  for (int c = lqp[nsingle + r] + lane; c < lqp[nsingle + r + 1]; c += 64) {
+    double t[K];
+    r_load<K>(part + (int64_t)(c - nsingle) * K, t);
+#pragma unroll
+    for (int q = 0; q < K; ++q) a[q] += t[q];
+  }
+  int col = 0;
+  const double s = r_reduce<K, 64>(a, lane, col);
+  if ((lane & (64 / K - 1)) == 0) r_row<K, MODE>(ep, x, lrows[nsingle + r], col, s);
 }
 
 // x = inv r on the coarsest level, one wavefront per row (coalesced rows)
+template <int K>
 __global__ void k_r_dense(int64_t n, const double *__restrict__ inv, const double *__restrict__ r, double *__restrict__ x) {
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64;
   const int lane = threadIdx.x & 63;
   if (i >= n) return;
-  double s = 0.;
-  for (int64_t j = lane; j < n; j += 64) s += inv[i * n + j] * r[j];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if (lane == 0) x[i] = s;
+  double a[K];
+#pragma unroll
+  for (int q = 0; q < K; ++q) a[q] = 0.;
+#pragma unroll 4
+  for (int64_t j = lane; j < n; j += 64) {
+    const double m = inv[i * n + j];
+    double t[K];
+    r_load<K>(r + j * K, t);
+#pragma unroll
+    for (int q = 0; q < K; ++q) a[q] += m * t[q];
+  }
+  int col = 0;
+  const double s = r_reduce<K, 64>(a, lane, col);
+  if ((lane & (64 / K - 1)) == 0) x[i * K + col] = s;
 }
 
-// partial[t * nb + blk] = sum over the block's rows of V_t . w
-__global__ void k_r_dots(int64_t n, const double *__restrict__ V, int64_t vstride, int nvec, const double *__restrict__ w,
-                         double *__restrict__ partial) {
+// ---------------------------------------------------------------- Krylov kernels of K columns
+
+// partial[(blk * nvec + t) * K + j] = sum over the block's rows of V_t w, four
+// vectors per grid row
+constexpr int kRDotBlocks = 256, kRDotChunk = 4;
+template <int K>
+__global__ void __launch_bounds__(256) k_rm_dots(int64_t n, const double *__restrict__ V, int64_t vstride, int nvec,
+                                                 const double *__restrict__ w, double *__restrict__ partial) {
   __shared__ double sh[256];
-  const int t = blockIdx.y;
-  double acc = 0.;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    acc += V[(int64_t)t * vstride + i] * w[i];
-  sh[threadIdx.x] = acc;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+  const int t0 = blockIdx.y * kRDotChunk, nt = min(kRDotChunk, nvec - t0);
+  double acc[kRDotChunk] = {0., 0., 0., 0.};
+  for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < n * K; q += (int64_t)gridDim.x * 256) {  // 256 % K == 0
+    const double b = w[q];
+#pragma unroll
+    for (int t = 0; t < kRDotChunk; ++t)
+      if (t < nt) acc[t] += V[(int64_t)(t0 + t) * vstride + q] * b;
+  }
+  for (int t = 0; t < nt; ++t) {
+    sh[threadIdx.x] = acc[t];
+    __syncthreads();
+    for (int h = 128; h >= K; h >>= 1) {
+      if ((int)threadIdx.x < h) sh[threadIdx.x] += sh[threadIdx.x + h];
+      __syncthreads();
+    }
+    if ((int)threadIdx.x < K) partial[((int64_t)blockIdx.x * nvec + t0 + t) * K + threadIdx.x] = sh[threadIdx.x];
     __syncthreads();
   }
-  if (threadIdx.x == 0) partial[(int64_t)t * gridDim.x + blockIdx.x] = sh[0];
 }
 
-// w = (w - sum_t V_t h_t) * sc
-__global__ void k_r_gs(int64_t n, const double *__restrict__ V, int64_t vstride, int nvec, const double *__restrict__ h,
-                       double sc, double *__restrict__ w) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double a = w[i];
-  for (int t = 0; t < nvec; ++t) a -= V[(int64_t)t * vstride + i] * h[t];
-  w[i] = a * sc;
+// h[q] = the sum of the blocks' partial sums of output q, a wavefront each
+__global__ void k_rm_dots_fin(int nout, int nb, const double *__restrict__ partial, double *__restrict__ h) {
+  const int q = (int)(blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64), lane = threadIdx.x & 63;
+  if (q >= nout) return;  // uniform across the wavefront
+  double a = 0.;
+  for (int b = lane; b < nb; b += 64) a += partial[(int64_t)b * nout + q];
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
+  if (lane == 0) h[q] = a;
+}
+
+// w -= sum_t V_t h_t
+template <int K>
+__global__ void k_rm_gs(int64_t n, const double *__restrict__ V, int64_t vstride, int nvec, const double *__restrict__ h,
+                        double *__restrict__ w) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n * K) return;
+  const int j = (int)(q % K);
+  double a = w[q];
+#pragma unroll 4
+  for (int t = 0; t < nvec; ++t) a -= V[(int64_t)t * vstride + q] * h[t * K + j];
+  w[q] = a;
+}
+
+// w *= sc_j, or (sc null) divided by sqrt(nn_j) where that is positive; with z
+// also the finest level's first sweep from zero, z = dd = zc w / d
+template <int K>
+__global__ void k_rm_scale(int64_t n, const double *__restrict__ sc, const double *__restrict__ nn,
+                           double *__restrict__ w, const double *__restrict__ d, double zc, double *__restrict__ z,
+                           double *__restrict__ dd) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n * K) return;
+  const int j = (int)(q % K);
+  const double f = sc ? sc[j] : nn[j] > 0. ? 1.0 / sqrt(nn[j]) : 1.0;
+  const double v = w[q] * f;
+  w[q] = v;
+  if (!z) return;
+  const double di = d[q / K], g = di != 0. ? zc * v / di : 0.;
+  z[q] = g;
+  if (dd) dd[q] = g;
 }
 
 // x += sum_t Z_t y_t
-__global__ void k_r_xup(int64_t n, const double *__restrict__ Z, int64_t zstride, int nvec, const double *__restrict__ y,
-                        double *__restrict__ x) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double a = x[i];
-  for (int t = 0; t < nvec; ++t) a += Z[(int64_t)t * zstride + i] * y[t];
-  x[i] = a;
-}
-
-__global__ void k_r_scal(int64_t n, double f, double *__restrict__ x) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] *= f;
+template <int K>
+__global__ void k_rm_xup(int64_t n, const double *__restrict__ Z, int64_t zstride, int nvec, const double *__restrict__ y,
+                         double *__restrict__ x) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n * K) return;
+  const int j = (int)(q % K);
+  double a = x[q];
+#pragma unroll 4
+  for (int t = 0; t < nvec; ++t) a += Z[(int64_t)t * zstride + q] * y[t * K + j];
+  x[q] = a;
 }
 
 __global__ void k_csr_dense(int64_t n, int64_t nnz, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
@@ -382,61 +494,33 @@ __global__ void k_csr_dense(int64_t n, int64_t nnz, const int64_t *__restrict__ 
 }  // namespace
 
 struct RLevel {
-  Csr A, P, R;
+  Csr A, P, R;              // rows above kLongRow listed
   double *d = nullptr, *dl1 = nullptr;
-  double *r = nullptr, *x = nullptr, *t = nullptr;
-  // Chebyshev smoothing: direction vector and the coefficients of each step
-  double *dd = nullptr;
-  double c1[kChebSteps] = {}, c2[kChebSteps] = {};
-  // rows longer than kRLong of A, P and R (device lists) and their counts
-  int32_t *la = nullptr, *lp = nullptr, *lr = nullptr;
-  int64_t nla = 0, nlp = 0, nlr = 0;
+  double c1[kChebSteps] = {}, c2[kChebSteps] = {};  // Chebyshev coefficients of each step
+};
+
+constexpr int kRestart = 30;
+
+// Vectors of a solve of K columns, kept for the next one of as many or fewer.
+struct RWork {
+  int K = 0;
+  Arena A;
+  std::vector<double *> r, x, t, dd;  // per level (r: from level 1 on)
+  double *part = nullptr;             // partial sums of the longest rows
+  // FGMRES: basis V (m+1 vectors), preconditioned basis Z (m), partial sums of
+  // the dot products, their results, per-column factors
+  double *V = nullptr, *Zb = nullptr, *dpart = nullptr, *h = nullptr, *y = nullptr;
 };
 
 struct RealAMG {
   int smoother = GP_SMOOTH_L1_JACOBI;
   std::vector<RLevel> L;
   double *inv = nullptr;  // coarsest, dense n x n
-  // FGMRES workspace: basis V (m+1 vectors), preconditioned basis Z (m),
-  // block partial sums of the dot products, Hessenberg coefficients
-  double *V = nullptr, *Zb = nullptr, *partial = nullptr, *hd = nullptr;
   Arena A;
+  RWork W;
 };
 
 namespace {
-
-// rows of M longer than kRLong, as a device list
-gp_status long_rows(Arena &A, const Csr &M, int32_t **out, int64_t *nl, hipStream_t s) {
-  *out = nullptr;
-  *nl = 0;
-  if (M.nr == 0) return GP_OK;
-  std::vector<int64_t> rp((size_t)M.nr + 1);
-  GP_HIP(hipMemcpyAsync(rp.data(), M.rp, sizeof(int64_t) * rp.size(), hipMemcpyDeviceToHost, s));
-  GP_HIP(hipStreamSynchronize(s));
-  std::vector<int32_t> l;
-  for (int64_t i = 0; i < M.nr; ++i)
-    if (rp[i + 1] - rp[i] > kRLong) l.push_back((int32_t)i);
-  if (l.empty()) return GP_OK;
-  GP_TRY(A.alloc(out, (int64_t)l.size()));
-  GP_HIP(hipMemcpyAsync(*out, l.data(), sizeof(int32_t) * l.size(), hipMemcpyHostToDevice, s));
-  GP_HIP(hipStreamSynchronize(s));
-  *nl = (int64_t)l.size();
-  return GP_OK;
-}
-
-void spmv_r(const Csr &M, const int32_t *lr, int64_t nl, const double *x, const double *r, double *y, int mode,
-            hipStream_t s) {
-  if (M.nr == 0) return;
-  k_r_spmv<<<blocks_for(M.nr * kRLanes), 256, 0, s>>>(M.nr, M.rp, M.ci, M.v[0], x, r, y, mode);
-  if (nl) k_r_spmv_long<<<(unsigned)nl, 256, 0, s>>>(lr, M.rp, M.ci, M.v[0], x, r, y, mode);
-}
-
-void jacobi_r(const RLevel &L, const double *x, double *xo, hipStream_t s) {
-  const int64_t n = L.A.nr;
-  if (!x) { k_r_jacobi0<<<blocks_for(n), 256, 0, s>>>(n, L.dl1, L.r, xo); return; }
-  k_r_jacobi<<<blocks_for(n * kRLanes), 256, 0, s>>>(n, L.A.rp, L.A.ci, L.A.v[0], L.dl1, L.r, x, xo);
-  if (L.nla) k_r_jacobi_long<<<(unsigned)L.nla, 256, 0, s>>>(L.la, L.A.rp, L.A.ci, L.A.v[0], L.dl1, L.r, x, xo);
-}
 
 // the Chebyshev coefficients for lambda, the estimate of D^-1 A's largest
 // eigenvalue: interval [alpha, beta], theta its centre, delta its half width,
@@ -455,15 +539,6 @@ void cheb_coeffs(double lam, double *c1, double *c2) {
     c2[k] = 2.0 * rn / delta;
     rho = rn;
   }
-}
-
-// step k of the Chebyshev smoother from x (null: x = 0, step 0 only) into xo
-void cheb_r(const RLevel &L, int k, const double *x, double *xo, hipStream_t s) {
-  const int64_t n = L.A.nr;
-  if (!x) { k_r_cheb0<<<blocks_for(n), 256, 0, s>>>(n, L.d, L.r, L.c2[0], L.dd, xo); return; }
-  k_r_cheb<<<blocks_for(n * kRLanes), 256, 0, s>>>(n, L.A.rp, L.A.ci, L.A.v[0], L.d, L.r, x, L.c1[k], L.c2[k], L.dd, xo);
-  if (L.nla)
-    k_r_cheb_long<<<(unsigned)L.nla, 256, 0, s>>>(L.la, L.A.rp, L.A.ci, L.A.v[0], L.d, L.r, x, L.c1[k], L.c2[k], L.dd, xo);
 }
 
 // one pairwise matching pass on M: tentative P (n x ncoarse)
@@ -528,8 +603,7 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
     const int64_t n = F.A.nr;
     GP_TRY(A.alloc(&F.d, n)); GP_TRY(A.alloc(&F.dl1, n));
     k_r_diag<<<wave_blocks(n), 256, 0, s>>>(n, F.A.rp, F.A.ci, F.A.v[0], F.d, F.dl1);
-    GP_TRY(A.alloc(&F.r, n)); GP_TRY(A.alloc(&F.x, n)); GP_TRY(A.alloc(&F.t, n));
-    GP_TRY(long_rows(A, F.A, &F.la, &F.nla, s));
+    GP_TRY(csr_mark_long(A, F.A, s));
     if (n <= kCoarsest || G.L.size() >= 24) break;
     TmpArena tmp;
     gp_status st = GP_OK;
@@ -549,10 +623,7 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
       // P = Pt - 4/(3 lambda) D^-1 A Pt
       double lam = 2.0;
       if ((st = power_lambda(tmp, F.A, F.d, &lam, s)) != GP_OK) break;
-      if (G.smoother == GP_SMOOTH_CHEBYSHEV) {
-        cheb_coeffs(lam, F.c1, F.c2);
-        if ((st = A.alloc(&F.dd, n)) != GP_OK) break;
-      }
+      if (G.smoother == GP_SMOOTH_CHEBYSHEV) cheb_coeffs(lam, F.c1, F.c2);
       if ((st = csr_alloc(tmp, n, n, F.A.nnz, 1, &DA)) != GP_OK) break;
       if (hipMemcpyAsync(DA.rp, F.A.rp, sizeof(int64_t) * (n + 1), hipMemcpyDeviceToDevice, s) != hipSuccess ||
           hipMemcpyAsync(DA.ci, F.A.ci, sizeof(int32_t) * F.A.nnz, hipMemcpyDeviceToDevice, s) != hipSuccess) { st = fail(GP_ERR_HIP, "copy"); break; }
@@ -569,8 +640,8 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
     if (st != GP_OK) return st;
     F.P = P;
     F.R = R;
-    GP_TRY(long_rows(A, F.P, &F.lp, &F.nlp, s));
-    GP_TRY(long_rows(A, F.R, &F.lr, &F.nlr, s));
+    GP_TRY(csr_mark_long(A, F.P, s));
+    GP_TRY(csr_mark_long(A, F.R, s));
     RLevel C;
     C.A = Ac;
     G.L.push_back(C);
@@ -587,41 +658,217 @@ gp_status build_real_amg(RealAMG &G, Csr A0, hipStream_t s) {
   return GP_OK;
 }
 
-void vcycle_real(const RealAMG &G, int l, hipStream_t s) {
-  const RLevel &L = G.L[l];
-  const int64_t n = L.A.nr;
-  if (l + 1 == (int)G.L.size()) {
-    k_r_dense<<<blocks_for(n * 64), 256, 0, s>>>(n, G.inv, L.r, L.x);
-    return;
-  }
-  static_assert(kChebSteps == 2, "the smoothing steps alternate between x and t twice");
-  const bool cheb = G.smoother == GP_SMOOTH_CHEBYSHEV;
-  if (cheb) { cheb_r(L, 0, nullptr, L.x, s); cheb_r(L, 1, L.x, L.t, s); }
-  else { jacobi_r(L, nullptr, L.x, s); jacobi_r(L, L.x, L.t, s); }
-  spmv_r(L.A, L.la, L.nla, L.t, L.r, L.x, 1, s);      // x <- r - A t
-  const RLevel &C = G.L[l + 1];
-  spmv_r(L.R, L.lr, L.nlr, L.x, nullptr, C.r, 0, s);
-  vcycle_real(G, l + 1, s);
-  spmv_r(L.P, L.lp, L.nlp, C.x, nullptr, L.t, 2, s);  // t += P xc
-  if (cheb) { cheb_r(L, 0, L.t, L.x, s); cheb_r(L, 1, L.x, L.t, s); }
-  else { jacobi_r(L, L.t, L.x, s); jacobi_r(L, L.x, L.t, s); }
-  (void)hipMemcpyAsync(L.x, L.t, sizeof(double) * n, hipMemcpyDeviceToDevice, s);
+template <int K, int MODE>
+void rm(const Csr &M, const double *v, const double *x, const REp &ep, double *part, hipStream_t s) {
+  if (M.nr == 0) return;
+  const unsigned nbw = (unsigned)((M.nchunk + 3) / 4);
+  const unsigned nbs = M.nlong == M.nr ? 0u : (unsigned)((M.nr * 8 + 255) / 256);
+  k_rm<K, MODE><<<nbw + nbs, 256, 0, s>>>(M.nr, nbw, M.rp, M.ci, v, M.lidx, M.lrows, M.lcb, M.lce, M.nchunk, M.nsingle, x,
+                                          ep, part);
+  const int nmulti = M.nlong - M.nsingle;
+  if (nmulti)
+    k_rm_fin<K, MODE><<<(unsigned)((nmulti + 3) / 4), 256, 0, s>>>(nmulti, M.nsingle, M.lrows, M.lqp, x, ep, part);
 }
 
-gp_status rdots(hipStream_t s, int64_t n, const double *V, int64_t vstride, int nvec, const double *w, double *partial,
-                std::vector<double> &h) {
-  const int nb = 256;
-  k_r_dots<<<dim3(nb, nvec), 256, 0, s>>>(n, V, vstride, nvec, w, partial);
-  std::vector<double> p((size_t)nb * nvec);
-  GP_HIP(hipMemcpyAsync(p.data(), partial, sizeof(double) * p.size(), hipMemcpyDeviceToHost, s));
-  GP_HIP(hipStreamSynchronize(s));
-  h.assign(nvec, 0.);
-  for (int t = 0; t < nvec; ++t)
-    for (int b = 0; b < nb; ++b) h[t] += p[(size_t)t * nb + b];
+template <int K>
+struct RCycle {
+  const RealAMG &G;
+  RWork &W;
+  hipStream_t s;
+  bool cheb() const { return G.smoother == GP_SMOOTH_CHEBYSHEV; }
+  double first_c(int l) const { return cheb() ? G.L[l].c2[0] : 1.0; }
+  const double *first_d(int l) const { return cheb() ? G.L[l].d : G.L[l].dl1; }
+  // step k of the smoother (k = 0: from a nonzero x)
+  void smooth(int l, int k, const double *r, const double *x, double *y) {
+    const RLevel &L = G.L[l];
+    REp ep;
+    ep.r = r; ep.y = y;
+    if (cheb()) {
+      ep.d = L.d; ep.c1 = L.c1[k]; ep.c2 = L.c2[k]; ep.dd = W.dd[l];
+      rm<K, R_CHEB>(L.A, L.A.v[0], x, ep, W.part, s);
+    } else {
+      ep.d = L.dl1;
+      rm<K, R_JAC>(L.A, L.A.v[0], x, ep, W.part, s);
+    }
+  }
+  // One V-cycle on level l for the right-hand side r, whose first sweep from
+  // zero is in W.x[l] (and W.dd[l]) already; the result goes to out.
+  void run(int l, const double *r, double *out) {
+    const RLevel &L = G.L[l];
+    if (l + 1 == (int)G.L.size()) {
+      k_r_dense<K><<<blocks_for(L.A.nr * 64), 256, 0, s>>>(L.A.nr, G.inv, r, out);
+      return;
+    }
+    static_assert(kChebSteps == 2, "the smoothing steps alternate between x and t twice");
+    double *x = W.x[l], *t = W.t[l];
+    smooth(l, 1, r, x, t);
+    REp res;
+    res.r = r; res.y = x;                       // x <- r - A t
+    rm<K, R_RES>(L.A, L.A.v[0], t, res, W.part, s);
+    REp down;
+    down.y = W.r[l + 1];
+    if (l + 2 < (int)G.L.size()) {
+      down.z = W.x[l + 1]; down.zd = first_d(l + 1); down.zc = first_c(l + 1);
+      if (cheb()) down.dd = W.dd[l + 1];
+    }
+    rm<K, R_MUL>(L.R, L.R.v[0], x, down, W.part, s);
+    run(l + 1, W.r[l + 1], W.t[l + 1]);
+    REp up;
+    up.y = t; up.acc = 1;                       // t += P xc
+    rm<K, R_MUL>(L.P, L.P.v[0], W.t[l + 1], up, W.part, s);
+    smooth(l, 0, r, t, x);
+    smooth(l, 1, r, x, out);
+  }
+};
+
+gp_status work(RealAMG &G, int K) {
+  RWork &W = G.W;
+  if (W.K >= K) return GP_OK;
+  W.A.free_all();
+  W.K = 0;
+  const size_t nl = G.L.size();
+  const int64_t n = G.L[0].A.nr;
+  W.r.assign(nl, nullptr); W.x.assign(nl, nullptr); W.t.assign(nl, nullptr); W.dd.assign(nl, nullptr);
+  int64_t chunks = 0;
+  for (size_t l = 0; l < nl; ++l) {
+    const RLevel &L = G.L[l];
+    if (l) GP_TRY(W.A.alloc(&W.r[l], L.A.nr * K));
+    GP_TRY(W.A.alloc(&W.x[l], L.A.nr * K)); GP_TRY(W.A.alloc(&W.t[l], L.A.nr * K));
+    if (G.smoother == GP_SMOOTH_CHEBYSHEV) GP_TRY(W.A.alloc(&W.dd[l], L.A.nr * K));
+    for (const Csr *M : {&L.A, &L.P, &L.R}) chunks = std::max<int64_t>(chunks, M->nchunk);
+  }
+  GP_TRY(W.A.alloc(&W.part, std::max<int64_t>(chunks, 1) * K));
+  GP_TRY(W.A.alloc(&W.V, (int64_t)(kRestart + 1) * n * K));
+  GP_TRY(W.A.alloc(&W.Zb, (int64_t)kRestart * n * K));
+  GP_TRY(W.A.alloc(&W.dpart, (int64_t)kRDotBlocks * (kRestart + 1) * K));
+  GP_TRY(W.A.alloc(&W.h, (int64_t)(2 * kRestart + 1) * K));
+  GP_TRY(W.A.alloc(&W.y, (int64_t)kRestart * K));
+  W.K = K;
   return GP_OK;
 }
 
-constexpr int kRestart = 30;
+template <int K>
+void rdots(const RWork &W, int64_t n, const double *V, int nvec, const double *w, double *h, hipStream_t s) {
+  k_rm_dots<K><<<dim3(kRDotBlocks, (nvec + kRDotChunk - 1) / kRDotChunk), 256, 0, s>>>(n, V, n * K, nvec, w, W.dpart);
+  k_rm_dots_fin<<<(unsigned)((nvec * K + 3) / 4), 256, 0, s>>>(nvec * K, kRDotBlocks, W.dpart, h);
+}
+
+// Flexible GMRES(m) per column, FP64, classical Gram-Schmidt with one
+// reorthogonalization pass, Givens rotations on the host: the coefficients of
+// both passes and the norm stay on the device and reach the host once per step.
+template <int K>
+gp_status solve_cols(RealAMG &G, const double *bd, double *xd, double tol, int maxit, int32_t *iters, double *relres,
+                     hipStream_t s) {
+  const int m = kRestart;
+  RWork &W = G.W;
+  const RLevel &L0 = G.L[0];
+  const int64_t n = L0.A.nr, nk = n * K;
+  RCycle<K> cyc{G, W, s};
+  const bool one = G.L.size() == 1;
+  const unsigned gk = blocks_for(nk);
+  GP_HIP(hipMemsetAsync(xd, 0, sizeof(double) * nk, s));
+  std::vector<double> hh((size_t)(2 * m + 1) * K);
+  auto fetch = [&](const double *dv, int cnt) -> gp_status {
+    GP_HIP(hipMemcpyAsync(hh.data(), dv, sizeof(double) * cnt, hipMemcpyDeviceToHost, s));
+    GP_HIP(hipStreamSynchronize(s));
+    return GP_OK;
+  };
+  rdots<K>(W, n, bd, 1, bd, W.h, s);
+  GP_TRY(fetch(W.h, K));
+  double bn[K], rel[K], beta[K], sc[K];
+  bool active[K];
+  for (int j = 0; j < K; ++j) { bn[j] = std::sqrt(hh[j]); rel[j] = 0.; iters[j] = 0; }
+  std::vector<double> H((size_t)(m + 1) * m * K), cs((size_t)m * K), sn((size_t)m * K), g((size_t)(m + 1) * K),
+      y((size_t)m * K);
+  for (;;) {
+    REp res;
+    res.r = bd; res.y = W.V;
+    rm<K, R_RES>(L0.A, L0.A.v[0], xd, res, W.part, s);
+    rdots<K>(W, n, W.V, 1, W.V, W.h, s);
+    GP_TRY(fetch(W.h, K));
+    bool any = false;
+    for (int j = 0; j < K; ++j) {
+      beta[j] = std::sqrt(hh[j]);
+      active[j] = false;
+      if (bn[j] > 0.) {
+        rel[j] = beta[j] / bn[j];
+        active[j] = rel[j] > tol && iters[j] < maxit;
+      }
+      sc[j] = active[j] ? 1.0 / beta[j] : 0.;
+      any = any || active[j];
+    }
+    if (!any) break;
+    // columns that are done carry zero vectors
+    GP_HIP(hipMemcpyAsync(W.y, sc, sizeof(double) * K, hipMemcpyHostToDevice, s));
+    auto scale = [&](const double *scp, double *v) {
+      k_rm_scale<K><<<gk, 256, 0, s>>>(n, scp, W.h + (int64_t)2 * m * K, v, cyc.first_d(0), cyc.first_c(0),
+                                       one ? nullptr : W.x[0], W.dd[0]);
+    };
+    scale(W.y, W.V);
+    std::fill(g.begin(), g.end(), 0.);
+    for (int j = 0; j < K; ++j) g[j] = active[j] ? beta[j] : 0.;
+    int used[K] = {}, steps = 0;
+    bool open[K];
+    for (int j = 0; j < K; ++j) open[j] = active[j];
+    for (int i = 0; i < m; ++i) {
+      double *Vi = W.V + (int64_t)i * nk, *Vn = Vi + nk, *Zi = W.Zb + (int64_t)i * nk;
+      cyc.run(0, Vi, Zi);
+      REp mul;
+      mul.y = Vn;
+      rm<K, R_MUL>(L0.A, L0.A.v[0], Zi, mul, W.part, s);
+      double *h1 = W.h, *h2 = W.h + (int64_t)(i + 1) * K, *nn = W.h + (int64_t)2 * m * K;
+      for (double *h : {h1, h2}) {
+        rdots<K>(W, n, W.V, i + 1, Vn, h, s);
+        k_rm_gs<K><<<gk, 256, 0, s>>>(n, W.V, nk, i + 1, h, Vn);
+      }
+      rdots<K>(W, n, Vn, 1, Vn, nn, s);
+      scale(nullptr, Vn);
+      GP_TRY(fetch(W.h, (2 * m + 1) * K));
+      steps = i + 1;
+      bool more = false;
+      for (int j = 0; j < K; ++j) {
+        if (!open[j]) continue;
+        double *Hj = &H[(size_t)j * (m + 1) * m], *cj = &cs[(size_t)j * m], *sj = &sn[(size_t)j * m];
+        for (int t = 0; t <= i; ++t) Hj[t * m + i] = hh[t * K + j] + hh[(i + 1 + t) * K + j];
+        Hj[(i + 1) * m + i] = std::sqrt(std::max(hh[(size_t)2 * m * K + j], 0.));
+        for (int t = 0; t < i; ++t) {
+          const double a = Hj[t * m + i], bq = Hj[(t + 1) * m + i];
+          Hj[t * m + i] = cj[t] * a + sj[t] * bq;
+          Hj[(t + 1) * m + i] = -sj[t] * a + cj[t] * bq;
+        }
+        const double a = Hj[i * m + i], bq = Hj[(i + 1) * m + i];
+        const double den = std::sqrt(a * a + bq * bq);
+        cj[i] = den > 0 ? a / den : 1.;
+        sj[i] = den > 0 ? bq / den : 0.;
+        Hj[i * m + i] = cj[i] * a + sj[i] * bq;
+        Hj[(i + 1) * m + i] = 0.;
+        g[(i + 1) * K + j] = -sj[i] * g[i * K + j];
+        g[i * K + j] = cj[i] * g[i * K + j];
+        ++iters[j];
+        used[j] = i + 1;
+        if (std::fabs(g[(i + 1) * K + j]) <= tol * bn[j] || iters[j] >= maxit) open[j] = false;
+        more = more || open[j];
+      }
+      if (!more) break;
+    }
+    std::fill(y.begin(), y.end(), 0.);
+    for (int j = 0; j < K; ++j) {
+      const double *Hj = &H[(size_t)j * (m + 1) * m];
+      for (int t = used[j] - 1; t >= 0; --t) {
+        double acc = g[t * K + j];
+        for (int q = t + 1; q < used[j]; ++q) acc -= Hj[t * m + q] * y[q * K + j];
+        y[t * K + j] = Hj[t * m + t] != 0. ? acc / Hj[t * m + t] : 0.;
+      }
+    }
+    GP_HIP(hipMemcpyAsync(W.y, y.data(), sizeof(double) * steps * K, hipMemcpyHostToDevice, s));
+    k_rm_xup<K><<<gk, 256, 0, s>>>(n, W.Zb, nk, steps, W.y, xd);
+  }
+  GP_HIP(hipStreamSynchronize(s));
+  GP_HIP(hipGetLastError());
+  bool ok = true;
+  for (int j = 0; j < K; ++j) { relres[j] = rel[j]; ok = ok && rel[j] <= tol; }
+  return ok ? GP_OK : fail(GP_ERR_NOCONV, "real solve stopped above the tolerance");
+}
 
 }  // namespace
 
@@ -637,10 +884,6 @@ gp_status real_amg_create(int64_t n, int64_t nnz, const int64_t *rows, const int
   const double *vv[1] = {vals};
   gp_status st = csr_from_coo(G->A, n, n, nnz, rows, cols, vv, 1, &A0, s);
   if (st == GP_OK) st = build_real_amg(*G, A0, s);
-  if (st == GP_OK) st = G->A.alloc(&G->V, (int64_t)(kRestart + 1) * n);
-  if (st == GP_OK) st = G->A.alloc(&G->Zb, (int64_t)kRestart * n);
-  if (st == GP_OK) st = G->A.alloc(&G->partial, (int64_t)256 * (kRestart + 1));
-  if (st == GP_OK) st = G->A.alloc(&G->hd, kRestart + 1);
   if (st != GP_OK) { real_amg_destroy(G); return st; }
   *out = G;
   return GP_OK;
@@ -648,87 +891,42 @@ gp_status real_amg_create(int64_t n, int64_t nnz, const int64_t *rows, const int
 
 int64_t real_amg_rows(const RealAMG *G) { return G->L[0].A.nr; }
 int32_t real_amg_levels(const RealAMG *G) { return (int32_t)G->L.size(); }
-int64_t real_amg_bytes(const RealAMG *G) { return G->A.bytes; }
+int64_t real_amg_column_bytes(const RealAMG *G) {
+  int64_t rows = (2 * kRestart + 1) * G->L[0].A.nr;
+  for (const RLevel &L : G->L) rows += 4 * L.A.nr;
+  return (int64_t)sizeof(double) * rows;
+}
+int64_t real_amg_work_bytes(const RealAMG *G) { return G->W.A.bytes; }
+int64_t real_amg_bytes(const RealAMG *G) { return G->A.bytes + G->W.A.bytes; }
 
 void real_amg_destroy(RealAMG *G) {
   if (!G) return;
+  G->W.A.free_all();
   G->A.free_all();
   delete G;
 }
 
-// flexible GMRES(m), FP64, classical Gram-Schmidt with one
-// reorthogonalization pass, Givens rotations on the host
-gp_status real_amg_solve(RealAMG *G, const double *bd, double *xd, double tol, int maxit, int32_t *iters_out,
-                         double *relres_out, hipStream_t s) {
-  const int m = kRestart;
-  const RLevel &L0 = G->L[0];
-  const int64_t n = L0.A.nr;
-  double *V = G->V, *Zb = G->Zb, *partial = G->partial, *hd = G->hd;
-  GP_HIP(hipMemsetAsync(xd, 0, sizeof(double) * n, s));
-  const unsigned gb = blocks_for(n);
-  std::vector<double> h, h2;
-  GP_TRY(rdots(s, n, bd, 0, 1, bd, partial, h));
-  const double bn = std::sqrt(h[0]);
-  int iters = 0;
-  double rel = 0.;
-  if (bn > 0.) {
-    std::vector<double> H((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m);
-    for (;;) {
-      spmv_r(L0.A, L0.la, L0.nla, xd, bd, V, 1, s);
-      GP_TRY(rdots(s, n, V, 0, 1, V, partial, h));
-      const double beta = std::sqrt(h[0]);
-      rel = beta / bn;
-      if (rel <= tol || iters >= maxit) break;
-      k_r_scal<<<gb, 256, 0, s>>>(n, 1.0 / beta, V);
-      std::fill(g.begin(), g.end(), 0.);
-      g[0] = beta;
-      int used = 0;
-      for (int i = 0; i < m && iters < maxit; ++i) {
-        double *Vi = V + (int64_t)i * n, *Vn = V + (int64_t)(i + 1) * n, *Zi = Zb + (int64_t)i * n;
-        GP_HIP(hipMemcpyAsync(L0.r, Vi, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-        vcycle_real(*G, 0, s);
-        GP_HIP(hipMemcpyAsync(Zi, L0.x, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-        spmv_r(L0.A, L0.la, L0.nla, Zi, nullptr, Vn, 0, s);
-        for (int pass = 0; pass < 2; ++pass) {
-          GP_TRY(rdots(s, n, V, n, i + 1, Vn, partial, h2));
-          GP_HIP(hipMemcpyAsync(hd, h2.data(), sizeof(double) * (i + 1), hipMemcpyHostToDevice, s));
-          k_r_gs<<<gb, 256, 0, s>>>(n, V, n, i + 1, hd, 1.0, Vn);
-          for (int t = 0; t <= i; ++t) H[t * m + i] = (pass ? H[t * m + i] : 0.) + h2[t];
-        }
-        GP_TRY(rdots(s, n, Vn, 0, 1, Vn, partial, h));
-        const double hn = std::sqrt(std::max(h[0], 0.));
-        H[(i + 1) * m + i] = hn;
-        if (hn > 0) k_r_scal<<<gb, 256, 0, s>>>(n, 1.0 / hn, Vn);
-        for (int t = 0; t < i; ++t) {
-          const double a = H[t * m + i], bq = H[(t + 1) * m + i];
-          H[t * m + i] = cs[t] * a + sn[t] * bq;
-          H[(t + 1) * m + i] = -sn[t] * a + cs[t] * bq;
-        }
-        const double a = H[i * m + i], bq = H[(i + 1) * m + i];
-        const double den = std::sqrt(a * a + bq * bq);
-        cs[i] = den > 0 ? a / den : 1.;
-        sn[i] = den > 0 ? bq / den : 0.;
-        H[i * m + i] = cs[i] * a + sn[i] * bq;
-        H[(i + 1) * m + i] = 0.;
-        g[i + 1] = -sn[i] * g[i];
-        g[i] = cs[i] * g[i];
-        ++iters;
-        used = i + 1;
-        if (std::fabs(g[i + 1]) <= tol * bn) break;
-      }
-      for (int t = used - 1; t >= 0; --t) {
-        double acc = g[t];
-        for (int q = t + 1; q < used; ++q) acc -= H[t * m + q] * y[q];
-        y[t] = H[t * m + t] != 0. ? acc / H[t * m + t] : 0.;
-      }
-      GP_HIP(hipMemcpyAsync(hd, y.data(), sizeof(double) * used, hipMemcpyHostToDevice, s));
-      k_r_xup<<<gb, 256, 0, s>>>(n, Zb, n, used, hd, xd);
-    }
-  }
-  GP_HIP(hipStreamSynchronize(s));
-  if (iters_out) *iters_out = iters;
-  if (relres_out) *relres_out = rel;
-  return rel <= tol ? GP_OK : fail(GP_ERR_NOCONV, "real solve stopped above the tolerance");
+gp_status real_amg_solve(RealAMG *G, int k, const double *b, double *x, double tol, int maxit, int32_t *iters,
+                         double *relres, hipStream_t s) {
+  if (k != 1 && k != 2 && k != 4 && k != 8) return fail(GP_ERR_ARG, "real solves take 1, 2, 4 or 8 columns");
+  GP_TRY(work(*G, k));
+  if (k == 1) return solve_cols<1>(*G, b, x, tol, maxit, iters, relres, s);
+  if (k == 2) return solve_cols<2>(*G, b, x, tol, maxit, iters, relres, s);
+  if (k == 4) return solve_cols<4>(*G, b, x, tol, maxit, iters, relres, s);
+  return solve_cols<8>(*G, b, x, tol, maxit, iters, relres, s);
+}
+
+gp_status real_mv(const Csr &M, int which, int k, double alpha, int acc, const double *x, double *y, double *part,
+                  hipStream_t s) {
+  REp ep;
+  ep.y = y; ep.alpha = alpha; ep.acc = acc;
+  if (k == 1) rm<1, R_MUL>(M, M.v[which], x, ep, part, s);
+  else if (k == 2) rm<2, R_MUL>(M, M.v[which], x, ep, part, s);
+  else if (k == 4) rm<4, R_MUL>(M, M.v[which], x, ep, part, s);
+  else if (k == 8) rm<8, R_MUL>(M, M.v[which], x, ep, part, s);
+  else return fail(GP_ERR_ARG, "real products take 1, 2, 4 or 8 columns");
+  GP_HIP(hipGetLastError());
+  return GP_OK;
 }
 
 }  // namespace gp
@@ -767,7 +965,11 @@ extern "C" gp_status gp_solve_real_ex(const int64_t *row, const int64_t *col, co
   RealAMG *G = nullptr;
   GP_TRY(real_amg_create(n, nnz, dr, dc, dv, smoother, &G, s));
   struct GGuard { RealAMG *g; ~GGuard() { real_amg_destroy(g); } } gg{G};
-  gp_status st = real_amg_solve(G, bd, xd, tol, 1000, iters_out, relres_out, s);
+  int32_t it = 0;
+  double rel = 0.;
+  gp_status st = real_amg_solve(G, 1, bd, xd, tol, 1000, &it, &rel, s);
+  if (iters_out) *iters_out = it;
+  if (relres_out) *relres_out = rel;
   if (st != GP_OK && st != GP_ERR_NOCONV) return st;
   GP_HIP(hipMemcpyAsync(x, xd, sizeof(double) * n, hipMemcpyDeviceToHost, s));
   GP_HIP(hipStreamSynchronize(s));

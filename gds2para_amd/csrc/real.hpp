@@ -14,14 +14,24 @@ struct RealAMG;
 // solver owns its copy of the matrix.
 gp_status real_amg_create(int64_t n, int64_t nnz, const int64_t *rows, const int64_t *cols, const double *vals,
                           int smoother, RealAMG **out, hipStream_t s);
-// x = A^-1 b (device vectors of n) by FGMRES(30) preconditioned with one
-// V-cycle, from x = 0, until ||b - A x|| <= tol ||b|| or maxit iterations.
-// Returns GP_ERR_NOCONV when the tolerance is not met (x holds the last iterate).
-gp_status real_amg_solve(RealAMG *G, const double *b, double *x, double tol, int maxit, int32_t *iters,
+// x = A^-1 b for k = 1, 2, 4 or 8 columns (device vectors, row i column j at
+// i*k + j) by FGMRES(30) preconditioned with one V-cycle, from x = 0, until
+// ||b - A x|| <= tol ||b|| or maxit iterations in every column; iters and relres
+// have k entries.  Returns GP_ERR_NOCONV when a column misses the tolerance (x
+// holds the last iterate).  The vectors it works on stay with the solver.
+gp_status real_amg_solve(RealAMG *G, int k, const double *b, double *x, double tol, int maxit, int32_t *iters,
                          double *relres, hipStream_t s);
+// y = alpha M x, or y += alpha M x, for k columns as above and value array
+// `which` of M, whose rows above kLongRow must be listed (csr_mark_long); part
+// holds M.nchunk * k doubles.
+gp_status real_mv(const Csr &M, int which, int k, double alpha, int acc, const double *x, double *y, double *part,
+                  hipStream_t s);
 int64_t real_amg_rows(const RealAMG *G);
 int32_t real_amg_levels(const RealAMG *G);
 int64_t real_amg_bytes(const RealAMG *G);
+// device bytes of a solve's vectors per column, and those held now
+int64_t real_amg_column_bytes(const RealAMG *G);
+int64_t real_amg_work_bytes(const RealAMG *G);
 void real_amg_destroy(RealAMG *G);
 
 }  // namespace gp

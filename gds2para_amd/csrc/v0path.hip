@@ -17,6 +17,7 @@
 // hold (v0d1valo / v0d1avalo / v0cvalo / v0cavalo, :104-108, :316-322).
 #pragma clang fp contract(off)
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <functional>
@@ -31,6 +32,7 @@ namespace gp {
 struct V0Path {
   Arena A;
   Csr Vd, VdT, Vc, VcT;            // v[0] = V0 values, v[1] = the test ("a") values
+  double *part = nullptr;          // partial sums of their longest rows, kPortCols columns
   RealAMG *ad = nullptr, *ac = nullptr;
   int smoother = GP_SMOOTH_CHEBYSHEV;  // of ad and ac
   int64_t nd = 0, nc = 0, ne = 0;
@@ -47,19 +49,12 @@ int64_t v0path_bytes(const V0Path *p);
 
 namespace {
 
-// y = A x (mode 0), y = -(A x) (mode 1), y = y + A x (mode 2); one wavefront
-// per row, so the long rows of V0d^T (the conductor aggregate columns of V0d)
-// are split over 64 lanes
-__global__ void k_mv_wave(int64_t nr, const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                          const double *__restrict__ v, const double *__restrict__ x, double *__restrict__ y, int mode) {
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-  const int lane = threadIdx.x & 63;
-  if (row >= nr) return;
-  double s = 0.;
-  for (int64_t p = rp[row] + lane; p < rp[row + 1]; p += 64) s += v[p] * x[ci[p]];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if (lane == 0) y[row] = mode == 0 ? s : mode == 1 ? -s : y[row] + s;
-}
+// Ports solved side by side: their vectors are interleaved (row i, port column j
+// at i*k + j), so the V0 matrices, the Ad and Ac hierarchies and every launch
+// serve all of them.  One port after the other (the layout before) left the 24
+// solves of 8 ports bound by launches and by the longest rows' latency: 820 ms
+// at 200x200x24 (2,900,000 edges), 56 ms now.
+constexpr int kPortCols = 8;
 
 // y0d /= (2 pi freqStart freqUnit)
 __global__ void k_div(int64_t n, double w, double *__restrict__ x) {
@@ -68,17 +63,17 @@ __global__ void k_div(int64_t n, double w, double *__restrict__ x) {
 }
 
 // t[e] = yd1[e] * (-1.0 * w0 * stackEpsn[e / El] * EPSILON0)   (src/matrixCon.cpp:442)
-__global__ void k_scale_eps_w(int64_t ne, int64_t El, const double *__restrict__ epsn, double w0,
+__global__ void k_scale_eps_w(int64_t nq, int k, int64_t El, const double *__restrict__ epsn, double w0,
                               const double *__restrict__ yd1, double *__restrict__ t) {
-  int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < ne) t[e] = yd1[e] * (-1.0 * w0 * epsn[e / El] * kEps0);
+  int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < nq) t[q] = yd1[q] * (-1.0 * w0 * epsn[q / k / El] * kEps0);
 }
 
 // t[e] = -yc[e] * stackEpsn[e / El] * EPSILON0   (src/matrixCon.cpp:536-538)
-__global__ void k_neg_eps(int64_t ne, int64_t El, const double *__restrict__ epsn, const double *__restrict__ yc,
+__global__ void k_neg_eps(int64_t nq, int k, int64_t El, const double *__restrict__ epsn, const double *__restrict__ yc,
                           double *__restrict__ t) {
-  int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < ne) t[e] = -yc[e] * epsn[e / El] * kEps0;
+  int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < nq) t[q] = -yc[q] * epsn[q / k / El] * kEps0;
 }
 
 __global__ void k_scatter(int64_t n, const int64_t *__restrict__ idx, const double *__restrict__ val,
@@ -87,17 +82,15 @@ __global__ void k_scatter(int64_t n, const int64_t *__restrict__ idx, const doub
   if (i < n) J[idx[i]] = val[i];
 }
 
-// yd = (yd2 - i yd1) + yc at the response edges only
-__global__ void k_gather_yd(int64_t n, const int64_t *__restrict__ idx, const double *__restrict__ yd2,
+// yd = (yd2 - i yd1) + yc at the response edges only, every port column
+__global__ void k_gather_yd(int64_t n, int k, const int64_t *__restrict__ idx, const double *__restrict__ yd2,
                             const double *__restrict__ yd1, const double *__restrict__ yc, double *__restrict__ out) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t e = idx[i];
-  out[2 * i] = (yd2[e] - 0. * yd1[e]) + (yc ? yc[e] : 0.);
-  out[2 * i + 1] = -yd1[e];
+  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n * k) return;
+  const int64_t q = idx[t / k] * k + t % k;
+  out[2 * t] = (yd2[q] - 0. * yd1[q]) + (yc ? yc[q] : 0.);
+  out[2 * t + 1] = -yd1[q];
 }
-
-unsigned wave_blocks(int64_t nr) { return (unsigned)((nr + 3) / 4); }
 
 gp_status setup(gp_layout *lay, V0Path **out) {
   auto t0 = std::chrono::steady_clock::now();
@@ -119,6 +112,12 @@ gp_status setup(gp_layout *lay, V0Path **out) {
       if ((st = csr_from_coo(P->A, P->ne, P->nc, V.v0c.n, V.v0c.row, V.v0c.col, cv, 2, &P->Vc, s)) != GP_OK) break;
       if ((st = csr_from_coo(P->A, P->nc, P->ne, V.v0c.n, V.v0c.col, V.v0c.row, cv, 2, &P->VcT, s)) != GP_OK) break;
     }
+    int64_t chunks = 1;
+    for (Csr *M : {&P->Vd, &P->VdT, &P->Vc, &P->VcT}) {
+      if ((st = csr_mark_long(P->A, *M, s)) != GP_OK) break;
+      chunks = std::max<int64_t>(chunks, M->nchunk);
+    }
+    if (st != GP_OK || (st = P->A.alloc(&P->part, chunks * kPortCols)) != GP_OK) break;
     // Ad: the kept entries only; the reference's trailing (0, 0, 0) slots are
     // never read by hypreSolve's row-by-row insertion (src/hypreSolve.cpp:47-59)
     if ((st = real_amg_create(P->nd, V.ad.n, V.ad.row, V.ad.col, V.ad.val, P->smoother, &P->ad, s)) != GP_OK) break;
@@ -139,75 +138,99 @@ double edge_len(const gp_mesh &m, const Grid &g, int64_t e) {
 }
 
 
-// Device buffers of one port's V0 solves (N_edge-long unless noted).  The
+// Device buffers of k ports' V0 solves (N_edge-long columns unless noted).  The
 // last three are optional: the test-value ("a") products that find_Vh's
 // per-frequency solve needs (src/matrixCon.cpp:412, :529, :553).
 struct PortBufs {
   double *J = nullptr, *t = nullptr, *yd1 = nullptr, *yc = nullptr, *yd2 = nullptr;
   double *bd = nullptr, *xd = nullptr, *bc = nullptr, *xc = nullptr;  // nd / nc long
   double *ydat = nullptr, *yca = nullptr, *yd2a = nullptr;
+  int64_t *jidx = nullptr;  // the ports' edges, at most maxj per port
+  double *jv = nullptr;
+  gp_status alloc(Arena &A, const gp_mesh &m, const V0Path &P, int k, bool test_values) {
+    const int64_t ne = P.ne * k, nd = P.nd * k, nc = P.nc * k;
+    int64_t maxj = 1;
+    for (int32_t p = 0; p < m.num_ports; ++p) {
+      int64_t c = 0;
+      for (int32_t sd = m.port_side_ptr[p]; sd < m.port_side_ptr[p + 1]; ++sd) c += m.side_edge_ptr[sd + 1] - m.side_edge_ptr[sd];
+      maxj = std::max(maxj, c);
+    }
+    GP_TRY(A.alloc(&J, ne)); GP_TRY(A.alloc(&t, ne)); GP_TRY(A.alloc(&yd1, ne));
+    GP_TRY(A.alloc(&yc, ne)); GP_TRY(A.alloc(&yd2, ne));
+    GP_TRY(A.alloc(&bd, nd)); GP_TRY(A.alloc(&xd, nd));
+    if (nc > 0) { GP_TRY(A.alloc(&bc, nc)); GP_TRY(A.alloc(&xc, nc)); }
+    if (test_values) { GP_TRY(A.alloc(&ydat, ne)); GP_TRY(A.alloc(&yca, ne)); GP_TRY(A.alloc(&yd2a, ne)); }
+    GP_TRY(A.alloc(&jidx, maxj * k)); GP_TRY(A.alloc(&jv, maxj * k));
+    return GP_OK;
+  }
 };
 
 typedef std::function<gp_status(RealAMG *, const double *, double *)> RealRun;
 
-// paraGenerator's V0 section for source port src (src/matrixCon.cpp:367-587):
+// paraGenerator's V0 section (src/matrixCon.cpp:367-587) for the source ports
+// src .. src + np - 1 in the first np of k columns (the others stay zero):
 // J, then
 //   y0d  = Ad^-1 (-V0da^T J) / w0,               yd1 = V0d y0d   (ydat = V0da y0d)
 //   y0c  = Ac^-1 (-V0ca^T J + V0ca^T (-w0 D_eps yd1)), yc = V0c y0c (yca = V0ca y0c)
 //   y0d2 = Ad^-1 (V0da^T (-D_eps yc)),           yd2 = V0d y0d2  (yd2a = V0da y0d2)
-gp_status port_solves(gp_layout *lay, V0Path &P, int32_t src, double w0, PortBufs &b, Arena &tmp,
+gp_status port_solves(gp_layout *lay, V0Path &P, int32_t src, int np, int k, double w0, PortBufs &b,
                       const RealRun &run) {
   hipStream_t s = lay->stream;
   const gp_mesh &m = lay->hm.view;
-  const int64_t ne = P.ne, nd = P.nd, nc = P.nc;
+  const int64_t ne = P.ne * k, nc = P.nc;
   const unsigned ge = blocks_for(ne);
+  auto mv = [&](const Csr &M, int which, double alpha, int acc, const double *x, double *y) {
+    return real_mv(M, which, k, alpha, acc, x, y, P.part, s);
+  };
   // J: portDirection of each side, assigned side by side (last assignment wins)
-  std::unordered_map<int64_t, size_t> jm;
   std::vector<int64_t> ji;
   std::vector<double> jvh;
-  for (int32_t sd = m.port_side_ptr[src]; sd < m.port_side_ptr[src + 1]; ++sd)
-    for (int64_t q = m.side_edge_ptr[sd]; q < m.side_edge_ptr[sd + 1]; ++q) {
-      auto it = jm.find(m.side_edges[q]);
-      if (it == jm.end()) { jm.emplace(m.side_edges[q], ji.size()); ji.push_back(m.side_edges[q]); jvh.push_back(m.side_dir[sd]); }
-      else jvh[it->second] = m.side_dir[sd];
-    }
+  for (int j = 0; j < np; ++j) {
+    std::unordered_map<int64_t, size_t> jm;
+    for (int32_t sd = m.port_side_ptr[src + j]; sd < m.port_side_ptr[src + j + 1]; ++sd)
+      for (int64_t q = m.side_edge_ptr[sd]; q < m.side_edge_ptr[sd + 1]; ++q) {
+        auto it = jm.find(m.side_edges[q]);
+        if (it == jm.end()) {
+          jm.emplace(m.side_edges[q], ji.size());
+          ji.push_back(m.side_edges[q] * k + j);
+          jvh.push_back(m.side_dir[sd]);
+        } else {
+          jvh[it->second] = m.side_dir[sd];
+        }
+      }
+  }
   const int64_t nj = (int64_t)ji.size();
   GP_HIP(hipMemsetAsync(b.J, 0, sizeof(double) * ne, s));
   if (nj > 0) {
-    int64_t *jidx = nullptr;
-    double *jv = nullptr;
-    GP_TRY(tmp.alloc(&jidx, nj)); GP_TRY(tmp.alloc(&jv, nj));
-    GP_HIP(hipMemcpyAsync(jidx, ji.data(), sizeof(int64_t) * nj, hipMemcpyHostToDevice, s));
-    GP_HIP(hipMemcpyAsync(jv, jvh.data(), sizeof(double) * nj, hipMemcpyHostToDevice, s));
-    k_scatter<<<blocks_for(nj), 256, 0, s>>>(nj, jidx, jv, b.J);
-    GP_HIP(hipStreamSynchronize(s));
-    tmp.release(jidx, nj);
-    tmp.release(jv, nj);
+    GP_HIP(hipMemcpyAsync(b.jidx, ji.data(), sizeof(int64_t) * nj, hipMemcpyHostToDevice, s));
+    GP_HIP(hipMemcpyAsync(b.jv, jvh.data(), sizeof(double) * nj, hipMemcpyHostToDevice, s));
+    k_scatter<<<blocks_for(nj), 256, 0, s>>>(nj, b.jidx, b.jv, b.J);
+    GP_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
   }
   // y0d = Ad^-1 (-V0da^T J) / w0 ; yd1 = V0d y0d
-  k_mv_wave<<<wave_blocks(nd), 256, 0, s>>>(nd, P.VdT.rp, P.VdT.ci, P.VdT.v[1], b.J, b.bd, 1);
+  GP_TRY(mv(P.VdT, 1, -1., 0, b.J, b.bd));
   GP_TRY(run(P.ad, b.bd, b.xd));
-  k_div<<<blocks_for(nd), 256, 0, s>>>(nd, w0, b.xd);
-  k_mv_wave<<<wave_blocks(ne), 256, 0, s>>>(ne, P.Vd.rp, P.Vd.ci, P.Vd.v[0], b.xd, b.yd1, 0);
-  if (b.ydat) k_mv_wave<<<wave_blocks(ne), 256, 0, s>>>(ne, P.Vd.rp, P.Vd.ci, P.Vd.v[1], b.xd, b.ydat, 0);
+  k_div<<<blocks_for(P.nd * k), 256, 0, s>>>(P.nd * k, w0, b.xd);
+  GP_TRY(mv(P.Vd, 0, 1., 0, b.xd, b.yd1));
+  if (b.ydat) GP_TRY(mv(P.Vd, 1, 1., 0, b.xd, b.ydat));
   if (nc > 0) {
     // y0c = Ac^-1 (-V0ca^T J + V0ca^T (yd1 * (-w0 D_eps))) ; yc = V0c y0c
-    k_scale_eps_w<<<ge, 256, 0, s>>>(ne, lay->g.El, lay->epsn, w0, b.yd1, b.t);
-    k_mv_wave<<<wave_blocks(nc), 256, 0, s>>>(nc, P.VcT.rp, P.VcT.ci, P.VcT.v[1], b.J, b.bc, 1);
-    k_mv_wave<<<wave_blocks(nc), 256, 0, s>>>(nc, P.VcT.rp, P.VcT.ci, P.VcT.v[1], b.t, b.bc, 2);
+    k_scale_eps_w<<<ge, 256, 0, s>>>(ne, k, lay->g.El, lay->epsn, w0, b.yd1, b.t);
+    GP_TRY(mv(P.VcT, 1, -1., 0, b.J, b.bc));
+    GP_TRY(mv(P.VcT, 1, 1., 1, b.t, b.bc));
     GP_TRY(run(P.ac, b.bc, b.xc));
-    k_mv_wave<<<wave_blocks(ne), 256, 0, s>>>(ne, P.Vc.rp, P.Vc.ci, P.Vc.v[0], b.xc, b.yc, 0);
-    if (b.yca) k_mv_wave<<<wave_blocks(ne), 256, 0, s>>>(ne, P.Vc.rp, P.Vc.ci, P.Vc.v[1], b.xc, b.yca, 0);
+    GP_TRY(mv(P.Vc, 0, 1., 0, b.xc, b.yc));
+    if (b.yca) GP_TRY(mv(P.Vc, 1, 1., 0, b.xc, b.yca));
   } else {
     GP_HIP(hipMemsetAsync(b.yc, 0, sizeof(double) * ne, s));
     if (b.yca) GP_HIP(hipMemsetAsync(b.yca, 0, sizeof(double) * ne, s));
   }
   // y0d2 = Ad^-1 (V0da^T (-yc D_eps)) ; yd2 = V0d y0d2
-  k_neg_eps<<<ge, 256, 0, s>>>(ne, lay->g.El, lay->epsn, b.yc, b.t);
-  k_mv_wave<<<wave_blocks(nd), 256, 0, s>>>(nd, P.VdT.rp, P.VdT.ci, P.VdT.v[1], b.t, b.bd, 0);
+  k_neg_eps<<<ge, 256, 0, s>>>(ne, k, lay->g.El, lay->epsn, b.yc, b.t);
+  GP_TRY(mv(P.VdT, 1, 1., 0, b.t, b.bd));
   GP_TRY(run(P.ad, b.bd, b.xd));
-  k_mv_wave<<<wave_blocks(ne), 256, 0, s>>>(ne, P.Vd.rp, P.Vd.ci, P.Vd.v[0], b.xd, b.yd2, 0);
-  if (b.yd2a) k_mv_wave<<<wave_blocks(ne), 256, 0, s>>>(ne, P.Vd.rp, P.Vd.ci, P.Vd.v[1], b.xd, b.yd2a, 0);
+  GP_TRY(mv(P.Vd, 0, 1., 0, b.xd, b.yd2));
+  if (b.yd2a) GP_TRY(mv(P.Vd, 1, 1., 0, b.xd, b.yd2a));
   return GP_OK;
 }
 
@@ -263,56 +286,72 @@ extern "C" gp_status gp_solve_v0(gp_layout *lay, double rtol, double *Z0, double
   }
   TmpArena tmp;
   struct TGuard { Arena *a; hipStream_t s; ~TGuard() { (void)hipStreamSynchronize(s); a->free_all(); } } tg{&tmp, s};
-  const int64_t ne = P.ne, nd = P.nd, nc = P.nc;
+  const int64_t nd = P.nd, nc = P.nc;
   const int64_t nr = std::max<int64_t>((int64_t)redge.size(), 1);
-  double *J, *t, *yd1, *yc, *yd2, *bd, *xd, *bc = nullptr, *xc = nullptr, *gat;
-  int64_t *ridx;
-  GP_TRY(tmp.alloc(&J, ne)); GP_TRY(tmp.alloc(&t, ne)); GP_TRY(tmp.alloc(&yd1, ne));
-  GP_TRY(tmp.alloc(&yc, ne)); GP_TRY(tmp.alloc(&yd2, ne));
-  GP_TRY(tmp.alloc(&bd, nd)); GP_TRY(tmp.alloc(&xd, nd));
-  if (nc > 0) { GP_TRY(tmp.alloc(&bc, nc)); GP_TRY(tmp.alloc(&xc, nc)); }
-  GP_TRY(tmp.alloc(&ridx, nr)); GP_TRY(tmp.alloc(&gat, 2 * nr));
+  // columns side by side: the ports, in steps of up to kPortCols, fewer where
+  // the solver's vectors and the buffers below would take a quarter of the
+  // free memory (what it holds from an earlier call counts as free)
+  int k = 1;
+  {
+    size_t fre = 0, tot = 0;
+    GP_HIP(hipMemGetInfo(&fre, &tot));
+    const int64_t per = real_amg_column_bytes(P.ad) + (P.ac ? real_amg_column_bytes(P.ac) : 0) +
+                        (int64_t)sizeof(double) * (5 * P.ne + 2 * nd + 2 * nc);
+    const int64_t avail = (int64_t)fre + real_amg_work_bytes(P.ad) + (P.ac ? real_amg_work_bytes(P.ac) : 0);
+    while (k < kPortCols && k < np && 2 * k * per <= avail / 4) k *= 2;
+  }
+  PortBufs pb;
+  double *gat = nullptr;
+  int64_t *ridx = nullptr;
+  GP_TRY(pb.alloc(tmp, m, P, k, false));
+  GP_TRY(tmp.alloc(&ridx, nr)); GP_TRY(tmp.alloc(&gat, 2 * nr * k));
   if (!redge.empty())
     GP_HIP(hipMemcpyAsync(ridx, redge.data(), sizeof(int64_t) * redge.size(), hipMemcpyHostToDevice, s));
 
-  std::vector<double> Zh(2 * (size_t)np * np, 0.), yh(2 * nr);
+  std::vector<double> Zh(2 * (size_t)np * np, 0.), yh(2 * nr * k);
   int32_t solves = 0, maxit = 0;
   double maxrel = 0.;
   gp_status result = GP_OK;
+  int ports_now = 0;
   RealRun run = [&](RealAMG *G, const double *b, double *x) -> gp_status {
-    int32_t it = 0;
-    double rel = 0.;
-    gp_status st = real_amg_solve(G, b, x, tol, 1000, &it, &rel, s);
-    ++solves;
-    maxit = std::max(maxit, it);
-    maxrel = std::max(maxrel, rel);
+    int32_t it[kPortCols] = {};
+    double rel[kPortCols] = {};
+    gp_status st = real_amg_solve(G, k, b, x, tol, 1000, it, rel, s);
+    solves += ports_now;
+    for (int j = 0; j < ports_now; ++j) {
+      maxit = std::max(maxit, it[j]);
+      maxrel = std::max(maxrel, rel[j]);
+    }
     if (st == GP_ERR_NOCONV) { result = GP_ERR_NOCONV; return GP_OK; }  // reported, x kept (as hypreSolve)
     return st;
   };
-  PortBufs pb;
-  pb.J = J; pb.t = t; pb.yd1 = yd1; pb.yc = yc; pb.yd2 = yd2; pb.bd = bd; pb.xd = xd; pb.bc = bc; pb.xc = xc;
-  for (int32_t src = 0; src < np; ++src) {
-    GP_TRY(port_solves(lay, P, src, w0, pb, tmp, run));
+  for (int32_t src0 = 0; src0 < np; src0 += k) {
+    ports_now = std::min<int32_t>(k, np - src0);
+    GP_TRY(port_solves(lay, P, src0, ports_now, k, w0, pb, run));
     // yd at the response edges, then Construct_Z_V0 on the host
     if (!redge.empty()) {
-      k_gather_yd<<<blocks_for((int64_t)redge.size()), 256, 0, s>>>((int64_t)redge.size(), ridx, yd2, yd1, yc, gat);
-      GP_HIP(hipMemcpyAsync(yh.data(), gat, sizeof(double) * 2 * redge.size(), hipMemcpyDeviceToHost, s));
+      const int64_t cnt = (int64_t)redge.size();
+      k_gather_yd<<<blocks_for(cnt * k), 256, 0, s>>>(cnt, k, ridx, pb.yd2, pb.yd1, pb.yc, gat);
+      GP_HIP(hipMemcpyAsync(yh.data(), gat, sizeof(double) * 2 * cnt * k, hipMemcpyDeviceToHost, s));
     }
     GP_HIP(hipStreamSynchronize(s));
-    double cur = 0.;
-    for (int32_t sd = m.port_side_ptr[src]; sd < m.port_side_ptr[src + 1]; ++sd) cur += m.side_area[sd];
-    for (int32_t p = 0; p < np; ++p) {
-      const size_t zi = (size_t)p + (size_t)np * src;
-      double zr = Zh[2 * zi], zim = Zh[2 * zi + 1];
-      const double dir = m.side_dir[m.port_side_ptr[p]] * 1.0;
-      for (int64_t q = rptr[p]; q < rptr[p + 1]; ++q) {
-        const double leng = edge_len(m, lay->g, redge[q]);
-        double tr = yh[2 * q] * leng, ti = yh[2 * q + 1] * leng;
-        tr = tr * dir; ti = ti * dir;
-        zr -= tr; zim -= ti;
+    for (int32_t src = src0; src < src0 + ports_now; ++src) {
+      double cur = 0.;
+      for (int32_t sd = m.port_side_ptr[src]; sd < m.port_side_ptr[src + 1]; ++sd) cur += m.side_area[sd];
+      for (int32_t p = 0; p < np; ++p) {
+        const size_t zi = (size_t)p + (size_t)np * src;
+        double zr = Zh[2 * zi], zim = Zh[2 * zi + 1];
+        const double dir = m.side_dir[m.port_side_ptr[p]] * 1.0;
+        for (int64_t q = rptr[p]; q < rptr[p + 1]; ++q) {
+          const double leng = edge_len(m, lay->g, redge[q]);
+          const size_t at = 2 * ((size_t)q * k + (src - src0));
+          double tr = yh[at] * leng, ti = yh[at + 1] * leng;
+          tr = tr * dir; ti = ti * dir;
+          zr -= tr; zim -= ti;
+        }
+        Zh[2 * zi] = zr / cur;
+        Zh[2 * zi + 1] = zim / cur;
       }
-      Zh[2 * zi] = zr / cur;
-      Zh[2 * zi + 1] = zim / cur;
     }
   }
   std::copy(Zh.begin(), Zh.end(), Z0);
@@ -350,24 +389,20 @@ extern "C" gp_status gp_v0_vh_inputs(gp_layout *lay, int32_t src, double rtol, d
   const gp_mesh &m = lay->hm.view;
   const double tol = rtol > 0 ? rtol : 1e-4;
   const double w0 = 2 * kPi * m.freq_start * m.freq_unit;
-  const int64_t ne = P.ne, nd = P.nd, nc = P.nc, n = lay->n;
+  const int64_t ne = P.ne, n = lay->n;
   TmpArena tmp;
   struct TGuard { Arena *a; hipStream_t s; ~TGuard() { (void)hipStreamSynchronize(s); a->free_all(); } } tg{&tmp, s};
   PortBufs b;
-  GP_TRY(tmp.alloc(&b.J, ne)); GP_TRY(tmp.alloc(&b.t, ne)); GP_TRY(tmp.alloc(&b.yd1, ne));
-  GP_TRY(tmp.alloc(&b.yc, ne)); GP_TRY(tmp.alloc(&b.yd2, ne));
-  GP_TRY(tmp.alloc(&b.ydat, ne)); GP_TRY(tmp.alloc(&b.yca, ne)); GP_TRY(tmp.alloc(&b.yd2a, ne));
-  GP_TRY(tmp.alloc(&b.bd, nd)); GP_TRY(tmp.alloc(&b.xd, nd));
-  if (nc > 0) { GP_TRY(tmp.alloc(&b.bc, nc)); GP_TRY(tmp.alloc(&b.xc, nc)); }
+  GP_TRY(b.alloc(tmp, m, P, 1, true));
   bool noconv = false;
   RealRun run = [&](RealAMG *G, const double *rhs, double *x) -> gp_status {
     int32_t it = 0;
     double rel = 0.;
-    gp_status st = real_amg_solve(G, rhs, x, tol, 1000, &it, &rel, s);
+    gp_status st = real_amg_solve(G, 1, rhs, x, tol, 1000, &it, &rel, s);
     if (st == GP_ERR_NOCONV) { noconv = true; return GP_OK; }
     return st;
   };
-  GP_TRY(port_solves(lay, P, src, w0, b, tmp, run));
+  GP_TRY(port_solves(lay, P, src, 1, 1, w0, b, run));
   std::vector<double> yd1(ne), ydat(ne), yd2(ne), yd2a(ne), yc(ne), yca(ne);
   std::vector<int64_t> mr(n);
   GP_HIP(hipMemcpyAsync(yd1.data(), b.yd1, sizeof(double) * ne, hipMemcpyDeviceToHost, s));

@@ -135,3 +135,42 @@ def test_ad_sums_in_order():
     for k in ("ad_row", "ad_col", "ad_val"):
         assert np.array_equal(got[k], ref[k]), k
     lay.close()
+
+
+def _z_from_yd(m, yd, src):
+    """Construct_Z_V0's column of source port src from the field yd."""
+    c, n = m.c, m.num_ports
+    psp = np.ctypeslib.as_array(c.port_side_ptr, shape=(n + 1,))
+    sep = np.ctypeslib.as_array(c.side_edge_ptr, shape=(int(psp[-1]) + 1,))
+    edges = np.ctypeslib.as_array(c.side_edges, shape=(int(sep[-1]),))
+    area = np.ctypeslib.as_array(c.side_area, shape=(int(psp[-1]),))
+    sdir = np.ctypeslib.as_array(c.side_dir, shape=(int(psp[-1]),))
+    zn = np.ctypeslib.as_array(c.zn, shape=(c.nz,))
+    es, ev = int(m.sizes.n_edge_s), int(m.sizes.n_edge_v)
+    z = np.zeros(n, complex)
+    for p in range(n):
+        s0 = psp[p]
+        e = edges[sep[s0]:sep[s0 + 1]]
+        iz = e // (es + ev)
+        z[p] = -np.sum(yd[e] * (zn[iz + 1] - zn[iz])) * sdir[s0]
+    return z / area[psp[src]:psp[src + 1]].sum()
+
+
+@pytest.mark.parametrize("smoother", [capi.GP_SMOOTH_CHEBYSHEV, capi.GP_SMOOTH_L1_JACOBI])
+@pytest.mark.parametrize("ports", [1, 2, 3, 8, 9])
+def test_v0_ports_side_by_side(ports, smoother):
+    """Z0 with the ports solved side by side (1, 2, 4 or 8 columns, the last
+    group partly empty) against each port's field solved alone.  Both reach a
+    relative residual of 1e-10, which leaves the responses alike to 1e-8 of the
+    column's largest."""
+    m = M.Mesh(M.manhattan_spec((30, 26, 11), n_ports=ports, nfreq=2, f_range=(1e8, 1e10), seed=21))
+    lay = Layout(m)
+    lay.set_v0_smoother(smoother)
+    Z0, _, st = lay.solve_v0(1e-10)
+    print(f"[kernels] V0 with {ports} ports, smoother {smoother}: {st['solves']} solves, {st['max_iters']} iterations", flush=True)
+    assert st["solves"] == 3 * ports and st["max_rel_residual"] <= 1e-10
+    Z0 = Z0.reshape(ports, ports)
+    for src in range(ports):
+        ref = _z_from_yd(m, lay.v0_vh_inputs(src, 1e-10)[2], src)
+        assert np.abs(Z0[src] - ref).max() <= 1e-8 * np.abs(ref).max(), src
+    lay.close()
