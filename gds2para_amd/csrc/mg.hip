@@ -1156,11 +1156,14 @@ __device__ __forceinline__ void sell_batch(const SellV<T> &M, int64_t b0, int t0
 #pragma unroll
   for (int h = 0; h < NB; ++h) {
     const int64_t e = b0 + (int64_t)(t0 + h * ES) * 64 + lane;
-    // the matrix is streamed once per launch: non-temporal, so it does not
-    // push the gathered rows of x out of the caches
-    c[h] = __builtin_nontemporal_load(M.ci + e);
+    // plain loads: a small operator then stays in L2 from one launch to the next
+    // (edge launches of a 60x20x8 layout 7.0 us with non-temporal loads, 5.4 with
+    // these; 9.0 and 7.2 at 48x48x12 in FP64), and where the operator streams
+    // the gathered rows of x keep their places all the same (level 0 at
+    // 200x200x24 224 us either way, a 400x400x32 solve 2286 and 2267 ms)
+    c[h] = M.ci[e];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) a[v][h] = __builtin_nontemporal_load(M.v[v] + e);
+    for (int v = 0; v < NV; ++v) a[v][h] = M.v[v][e];
   }
   C2<T> xv[NB][KS];
 #pragma unroll

@@ -171,9 +171,9 @@ __device__ __forceinline__ void outer_batch(const SellV<double> &SS, int64_t b0,
 #pragma unroll
   for (int h = 0; h < NB; ++h) {
     const int64_t e = b0 + (int64_t)(t0 + h) * 64 + lane;
-    // streamed once per launch: non-temporal, keeping the caches for x
-    c[h] = __builtin_nontemporal_load(SS.ci + e);
-    m[h] = __builtin_nontemporal_load(SS.v[0] + e);
+    // plain loads, as in the preconditioner's walks (sell_batch)
+    c[h] = SS.ci[e];
+    m[h] = SS.v[0][e];
   }
   C2<TZ> x[NB][KS];
 #pragma unroll
