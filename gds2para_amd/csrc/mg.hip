@@ -1622,7 +1622,7 @@ bool edge_march(const Hierarchy &H, int k, const SellV<float> &K, const SellV<fl
   return true;
 }
 
-// SELL nodal l1-Jacobi (contract of k_node) of an operator without listed rows
+// SELL nodal l1-Jacobi sweep (contract of k_node, d given) of an operator without listed rows
 template <class T, int SPL, int LPR, int ES>
 __global__ void __launch_bounds__(256) k_node_sell(int64_t nr, int k, SellV<T> N, const T *__restrict__ c1v,
                                                    const T *__restrict__ c2v, const T *__restrict__ nd0,
@@ -1645,42 +1645,81 @@ __global__ void __launch_bounds__(256) k_node_sell(int64_t nr, int k, SellV<T> N
   else
 #pragma unroll
     for (int q = 0; q < KS; ++q) acc[q] = {0, 0};
-  if (d) {
-      const int64_t sl = pos >> 6;
-      const int lane = (int)(pos & 63);
-      const int64_t b0 = N.base[sl];
-      const int wd = N.w[sl];
-      sell_row_es<T, KS, 2, ES>(N, b0, wd, lane, es, d, k, j0, [&](T a0, T a1, T, const C2<T>(&x)[KS]) {
+  {
+    const int64_t sl = pos >> 6;
+    const int lane = (int)(pos & 63);
+    const int64_t b0 = N.base[sl];
+    const int wd = N.w[sl];
+    sell_row_es<T, KS, 2, ES>(N, b0, wd, lane, es, d, k, j0, [&](T a0, T a1, T, const C2<T>(&x)[KS]) {
 #pragma unroll
-        for (int q = 0; q < KS; ++q) {
-          const T ar = c1[q] * a0, ai = c2[q] * a1;
-          acc[q].x -= ar * x[q].x - ai * x[q].y;
-          acc[q].y -= ar * x[q].y + ai * x[q].x;
-        }
-      });
+      for (int q = 0; q < KS; ++q) {
+        const T ar = c1[q] * a0, ai = c2[q] * a1;
+        acc[q].x -= ar * x[q].x - ai * x[q].y;
+        acc[q].y -= ar * x[q].y + ai * x[q].x;
+      }
+    });
   }
   es_reduce<T, KS, LPR, ES>(acc);
   if (es != 0) return;
   const T e0 = nd0[i], e1 = nd1[i], m0 = nl0[i], m1 = nl1[i];
   C2<T> o[KS];
-  if (d) load_slots<T, KS>(d + i * k + j0, o);
+  load_slots<T, KS>(d + i * k + j0, o);
 #pragma unroll
   for (int q = 0; q < KS; ++q) {
     const C2<T> dg = l1diag<T>({c1[q] * e0, c2[q] * e1}, fabs(c1[q]) * m0 + c2[q] * m1);
     const C2<T> z = cdiv(acc[q], dg);
-    if (d) o[q] = {o[q].x + damp * z.x, o[q].y + damp * z.y};
-    else o[q] = {damp * z.x, damp * z.y};
+    o[q] = {o[q].x + damp * z.x, o[q].y + damp * z.y};
   }
   store_slots<T, KS>(dout + i * k + j0, o);
 }
 
-// SELL y = M x (real M) or y += M x, an operator without listed rows
-template <class T, int SPL, int LPR, int ES>
-__global__ void __launch_bounds__(256) k_spmv_real_sell(int64_t nr, int k, SellV<T> M, const C2<T> *__restrict__ x,
-                                                        C2<T> *__restrict__ y, int accumulate) {
+// Optional epilogues of the products that form a right-hand side, taken while it
+// is in registers instead of by a pass of its own.  Jac0, over edge rows y:
+// u = damp y / d_l1, the edge smoother's first sweep from zero.
+template <class T>
+struct Jac0 {
+  const T *kd0 = nullptr, *kd1 = nullptr, *kd2 = nullptr, *kl0 = nullptr, *kl1 = nullptr, *kl2 = nullptr;
+  C2<T> *u = nullptr;
+  T damp = (T)1;
+};
+template <class T, int KS>
+__device__ __forceinline__ void jac0_store(const Jac0<T> &jz, int64_t i, int k, int j0, const T (&c1)[KS], const T (&c2)[KS],
+                                           const C2<T> (&o)[KS]) {
+  const T d0 = jz.kd0[i], d1 = jz.kd1[i], d2 = jz.kd2[i], l0 = jz.kl0[i], l1 = jz.kl1[i], l2 = jz.kl2[i];
+  C2<T> uo[KS];
+#pragma unroll
+  for (int q = 0; q < KS; ++q) {
+    const C2<T> dq = l1diag<T>({d0 + c1[q] * d1, c2[q] * d2}, l0 + fabs(c1[q]) * l1 + c2[q] * l2);
+    const C2<T> z = cdiv(o[q], dq);
+    uo[q] = {jz.damp * z.x, jz.damp * z.y};
+  }
+  store_slots<T, KS>(jz.u + i * k + j0, uo);
+}
+// Nod0, over nodal rows y = G^T res: d = damp y / d_n, the nodal smoother's first
+// sweep from zero, and with sum also sum += d.  y itself is stored only where a
+// second sweep reads it.
+template <class T>
+struct Nod0 {
+  const T *nd0 = nullptr, *nd1 = nullptr, *nl0 = nullptr, *nl1 = nullptr;
+  C2<T> *d = nullptr, *sum = nullptr;
+  T damp = (T)1;
+};
+
+// SELL y = M x (real M) or y += M x, an operator without listed rows; EP names
+// the epilogue.  One level's edge and nodal prolongations share a launch
+// (k_prolong_sell).  Most of a small level's launch is the launch (2.5-6 us at
+// 48x48x12), and a level of the edge V-cycle takes 9 of them now instead of 14;
+// on large levels the passes over rn and phi go.  Solve of a 60x20x8 layout 10.1
+// -> 9.2 ms, 48x48x12 in FP64 18.2 -> 16.8, 8 ports at 128x128x16 164.0 -> 157.5,
+// at 200x200x24 333.3 -> 324.9.
+enum SpmvEp { SPMV_PLAIN = 0, SPMV_JAC0 = 1, SPMV_NOD0 = 2 };
+
+template <class T, int SPL, int LPR, int ES, int EP>
+__device__ __forceinline__ void spmv_real_row(int64_t t_, int64_t nr, int k, const SellV<T> &M, const C2<T> *__restrict__ x,
+                                              C2<T> *__restrict__ y, int accumulate, const T *__restrict__ c1v,
+                                              const T *__restrict__ c2v, const Jac0<T> &jz, const Nod0<T> &nz) {
   constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each;
                            // ES such groups split the row's entries
-  const int64_t t_ = xcd_block_id() * blockDim.x + threadIdx.x;
   const int64_t pos = t_ / (LPR * ES);
   if (pos >= nr) return;
   const int sub = (int)(t_ - pos * (LPR * ES)), es = sub / LPR;
@@ -1701,13 +1740,55 @@ __global__ void __launch_bounds__(256) k_spmv_real_sell(int64_t nr, int k, SellV
   }
   es_reduce<T, KS, LPR, ES>(acc);
   if (es != 0) return;
-  if (accumulate) {
+  if (EP == SPMV_PLAIN && accumulate) {
     C2<T> o[KS];
     load_slots<T, KS>(y + i * k + j0, o);
 #pragma unroll
     for (int q = 0; q < KS; ++q) { acc[q].x += o[q].x; acc[q].y += o[q].y; }
   }
-  store_slots<T, KS>(y + i * k + j0, acc);
+  if (EP != SPMV_NOD0 || y) store_slots<T, KS>(y + i * k + j0, acc);
+  if constexpr (EP != SPMV_PLAIN) {
+    T c1[KS], c2[KS];
+#pragma unroll
+    for (int q = 0; q < KS; ++q) { c1[q] = c1v[j0 + q]; c2[q] = c2v[j0 + q]; }
+    if constexpr (EP == SPMV_JAC0) {
+      jac0_store<T, KS>(jz, i, k, j0, c1, c2, acc);
+    } else {
+      const T e0 = nz.nd0[i], e1 = nz.nd1[i], m0 = nz.nl0[i], m1 = nz.nl1[i];
+      C2<T> o[KS], sm[KS];
+      if (nz.sum) load_slots<T, KS>(nz.sum + i * k + j0, sm);
+#pragma unroll
+      for (int q = 0; q < KS; ++q) {
+        const C2<T> dg = l1diag<T>({c1[q] * e0, c2[q] * e1}, fabs(c1[q]) * m0 + c2[q] * m1);
+        const C2<T> z = cdiv(acc[q], dg);
+        o[q] = {nz.damp * z.x, nz.damp * z.y};
+        if (nz.sum) sm[q] = {sm[q].x + o[q].x, sm[q].y + o[q].y};
+      }
+      store_slots<T, KS>(nz.d + i * k + j0, o);
+      if (nz.sum) store_slots<T, KS>(nz.sum + i * k + j0, sm);
+    }
+  }
+}
+
+template <class T, int SPL, int LPR, int ES, int EP>
+__global__ void __launch_bounds__(256) k_spmv_real_sell(int64_t nr, int k, SellV<T> M, const C2<T> *__restrict__ x,
+                                                        C2<T> *__restrict__ y, int accumulate,
+                                                        const T *__restrict__ c1v, const T *__restrict__ c2v, Jac0<T> jz,
+                                                        Nod0<T> nz) {
+  spmv_real_row<T, SPL, LPR, ES, EP>(xcd_block_id() * blockDim.x + threadIdx.x, nr, k, M, x, y, accumulate, c1v, c2v, jz, nz);
+}
+
+// y += M x and y2 += M2 x2: workgroups below nb take the first, the others the second
+template <class T, int SPL, int LPR>
+__global__ void __launch_bounds__(256) k_prolong_sell(unsigned nb, int64_t nr, int64_t nr2, int k, SellV<T> M, SellV<T> M2,
+                                                      const C2<T> *__restrict__ x, C2<T> *__restrict__ y,
+                                                      const C2<T> *__restrict__ x2, C2<T> *__restrict__ y2) {
+  const int64_t b = xcd_block_id();
+  if (b < (int64_t)nb)
+    spmv_real_row<T, SPL, LPR, 1, SPMV_PLAIN>(b * 256 + threadIdx.x, nr, k, M, x, y, 1, nullptr, nullptr, Jac0<T>(), Nod0<T>());
+  else
+    spmv_real_row<T, SPL, LPR, 1, SPMV_PLAIN>((b - nb) * 256 + threadIdx.x, nr2, k, M2, x2, y2, 1, nullptr, nullptr, Jac0<T>(),
+                                              Nod0<T>());
 }
 
 // Products with the auxiliary operators (N, P, P^T, Gx^T): 24 entries or fewer
@@ -1896,16 +1977,6 @@ __global__ void __launch_bounds__(256) k_aux_fin(int k, MatV<T> M, const T *__re
   row.store(ep, i, k, j0, c1, c2, acc);
 }
 
-// Optional epilogue of k_spmv2_sell over level-0 edge rows: u = damp y / d_l1,
-// the edge smoother's first sweep from zero, formed from y while it is in
-// registers instead of by a separate pass over y.
-template <class T>
-struct Jac0 {
-  const T *kd0 = nullptr, *kd1 = nullptr, *kd2 = nullptr, *kl0 = nullptr, *kl1 = nullptr, *kl2 = nullptr;
-  C2<T> *u = nullptr;
-  T damp = (T)1;
-};
-
 // SELL M2(w) = c1 v0 + i c2 v1: y = r - M2 x (mode 0), y -= M2 x (1), y = M2 x (2)
 template <class T, int SPL, int LPR, int ES>
 __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> M, const T *__restrict__ c1v,
@@ -1951,17 +2022,7 @@ __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> 
     else o[q] = {o[q].x - acc[q].x, o[q].y - acc[q].y};
   }
   store_slots<T, KS>(y + i * k + j0, o);
-  if (jz.u) {
-    const T d0 = jz.kd0[i], d1 = jz.kd1[i], d2 = jz.kd2[i], l0 = jz.kl0[i], l1 = jz.kl1[i], l2 = jz.kl2[i];
-    C2<T> uo[KS];
-#pragma unroll
-    for (int q = 0; q < KS; ++q) {
-      const C2<T> dq = l1diag<T>({d0 + c1[q] * d1, c2[q] * d2}, l0 + fabs(c1[q]) * l1 + c2[q] * l2);
-      const C2<T> z = cdiv(o[q], dq);
-      uo[q] = {jz.damp * z.x, jz.damp * z.y};
-    }
-    store_slots<T, KS>(jz.u + i * k + j0, uo);
-  }
+  if (jz.u) jac0_store<T, KS>(jz, i, k, j0, c1, c2, o);
 }
 
 // k_spmv2_sell (one entry group, no long rows) on an operator of
@@ -2320,6 +2381,23 @@ Lanes lanes_shape(int64_t nr, int k) {
   return L;
 }
 
+// go(slots per lane, lanes per row) as compile-time constants
+template <class T, class F>
+void lanes_go(const Lanes &ln, F &&go) {
+  auto lanes = [&](auto sp_) {
+    if (ln.lpr == 16) go(sp_, std::integral_constant<int, 16>());
+    else if (ln.lpr == 8) go(sp_, std::integral_constant<int, 8>());
+    else if (ln.lpr == 4) go(sp_, std::integral_constant<int, 4>());
+    else if (ln.lpr == 2) go(sp_, std::integral_constant<int, 2>());
+    else go(sp_, std::integral_constant<int, 1>());
+  };
+  if constexpr (sizeof(T) == 4) {
+    if (ln.sp == 4) { lanes(std::integral_constant<int, 4>()); return; }
+    if (ln.sp == 2) { lanes(std::integral_constant<int, 2>()); return; }
+  }
+  lanes(std::integral_constant<int, 1>());
+}
+
 #define GP_LANES_DISPATCH(KERNEL, ...)                                                                   \
   do {                                                                                                   \
     const Lanes ln_ = lanes_shape<T>(nr, k);                                                             \
@@ -2388,6 +2466,21 @@ int entry_split(const SellV<T> &M, const Lanes &L) {
     }                                                                                                    \
   } while (0)
 
+#define GP_LANES_EP_DISPATCH(KERNEL, EP_, MAT, ...)                                                        \
+  do {                                                                                                   \
+    const Lanes ln_ = lanes_shape<T>(nr, k);                                                             \
+    const int es_ = entry_split<T>(MAT, ln_);                                                            \
+    if (es_ > 1) {                                                                                       \
+      const dim3 g_((unsigned)((nr * es_ + 255) / 256), ln_.grid.y);  /* sp = lpr = 1 */                 \
+      if (es_ == 16) KERNEL<T, 1, 1, 16, EP_><<<g_, 256, 0, s>>>(__VA_ARGS__);                           \
+      else KERNEL<T, 1, 1, 4, EP_><<<g_, 256, 0, s>>>(__VA_ARGS__);                                      \
+    } else {                                                                                             \
+      lanes_go<T>(ln_, [&](auto sp_, auto lp_) {                                                         \
+        KERNEL<T, decltype(sp_)::value, decltype(lp_)::value, 1, EP_><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__); \
+      });                                                                                                \
+    }                                                                                                    \
+  } while (0)
+
 template <class T>
 void edge_sell(int64_t nr, int64_t smin, int k, const SellV<T> &K, const SellV<T> &B, const MatV<T> &Kc, const MatV<T> &Bc,
                const T *c1, const T *c2, const T *kd0, const T *kd1, const T *kd2, const T *kl0, const T *kl1,
@@ -2450,15 +2543,35 @@ void node_sell(int64_t nr, int64_t smin, int k, const SellV<T> &N, const MatV<T>
   GP_LANES_ES_DISPATCH(k_node_sell, N, nr, k, N, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp);
 }
 
-template <class T>
+template <class T, int EP = SPMV_PLAIN>
 void spmv_real_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const MatV<T> &Mc, const C2<T> *x, C2<T> *y, int accumulate,
-                    hipStream_t s) {
+                    hipStream_t s, const T *c1 = nullptr, const T *c2 = nullptr, const Jac0<T> &jz = Jac0<T>(),
+                    const Nod0<T> &nz = Nod0<T>()) {
   if (nr == 0) return;
   if (nr < smin) {
     k_spmv_real<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, x, y, accumulate, nullptr);
     return;
   }
-  GP_LANES_ES_DISPATCH(k_spmv_real_sell, M, nr, k, M, x, y, accumulate);
+  GP_LANES_EP_DISPATCH(k_spmv_real_sell, EP, M, nr, k, M, x, y, accumulate, c1, c2, jz, nz);
+}
+
+// y += M x and y2 += M2 x2 in one launch where both take one entry group per row
+template <class T>
+void prolong_sell(int64_t nr, int64_t nr2, int64_t smin, int k, const SellV<T> &M, const MatV<T> &Mc, const C2<T> *x, C2<T> *y,
+                  const SellV<T> &M2, const MatV<T> &M2c, const C2<T> *x2, C2<T> *y2, hipStream_t s) {
+  const Lanes ln = lanes_shape<T>(nr, k), l2 = lanes_shape<T>(nr2, k);
+  if (nr == 0 || nr2 == 0 || nr < smin || nr2 < smin || entry_split<T>(M, ln) != 1 || entry_split<T>(M2, ln) != 1) {
+    spmv_real_sell<T>(nr, smin, k, M, Mc, x, y, 1, s);
+    spmv_real_sell<T>(nr2, smin, k, M2, M2c, x2, y2, 1, s);
+    return;
+  }
+  const dim3 grid(ln.grid.x + l2.grid.x, ln.grid.y);
+  const unsigned nb = ln.grid.x;
+  auto go = [&](auto sp_, auto lp_) {
+    k_prolong_sell<T, decltype(sp_)::value, decltype(lp_)::value>
+        <<<grid, 256, 0, s>>>(nb, nr, nr2, k, M, M2, x, y, x2, y2);
+  };
+  lanes_go<T>(ln, go);
 }
 
 // Returns whether the optional epilogue jz ran (sliced-ELL path only).
@@ -2530,18 +2643,7 @@ void aux_prod(int64_t nr, const VWork<T> &w, const SellV<T> &S, const MatV<T> &M
     k_aux<T, SP, LP, MODE><<<grid, 256, 0, s>>>(nr, k, nbw, S, M, w.c1, w.c2, x, ep, w.lpart);
     if (nfin) k_aux_fin<T, SP, LP, MODE><<<dim3(nfin, grid.y), 256, 0, s>>>(k, M, w.c1, w.c2, x, ep, w.lpart);
   };
-  auto lanes = [&](auto sp_) {
-    if (ln.lpr == 16) go(sp_, std::integral_constant<int, 16>());
-    else if (ln.lpr == 8) go(sp_, std::integral_constant<int, 8>());
-    else if (ln.lpr == 4) go(sp_, std::integral_constant<int, 4>());
-    else if (ln.lpr == 2) go(sp_, std::integral_constant<int, 2>());
-    else go(sp_, std::integral_constant<int, 1>());
-  };
-  if constexpr (sizeof(T) == 4) {
-    if (ln.sp == 4) { lanes(std::integral_constant<int, 4>()); return; }
-    if (ln.sp == 2) { lanes(std::integral_constant<int, 2>()); return; }
-  }
-  lanes(std::integral_constant<int, 1>());
+  lanes_go<T>(ln, go);
 }
 
 }  // namespace
@@ -2561,6 +2663,16 @@ int march_lds_setup() {
   return v;
 }
 
+
+// First edge sweep of level l, into the buffer that vcycle_level starts from
+template <class T>
+static Jac0<T> jac0_of(const MgLevel &L, const VWork<T> &w, int l, int nu_pre, int nu_post) {
+  Jac0<T> jz;
+  jz.kd0 = arr<T>(L.kd[0], L.kdf[0]); jz.kd1 = arr<T>(L.kd[1], L.kdf[1]); jz.kd2 = arr<T>(L.kd[2], L.kdf[2]);
+  jz.kl0 = arr<T>(L.kl[0], L.klf[0]); jz.kl1 = arr<T>(L.kl[1], L.klf[1]); jz.kl2 = arr<T>(L.kl[2], L.klf[2]);
+  jz.u = (((nu_pre - 1) + nu_post) & 1) ? w.tmp[l] : w.u[l];
+  return jz;
+}
 
 template <class T>
 static gp_status vcycle_level(const Hierarchy &H, VWork<T> &w, hipStream_t s, int l, int nu_pre, int nu_post) {
@@ -2621,13 +2733,30 @@ static gp_status vcycle_level(const Hierarchy &H, VWork<T> &w, hipStream_t s, in
     edge_sell<T>(ne, w.sell_min_rows, k, KS, BS, K, B, w.c1, w.c2, kd0, kd1, kd2, kl0, kl1, kl2, rr, uu, pp, oo, mode,
                  use_phi, dmp, st);
   };
+  // rn = G^T res and the nodal smoother's first sweep from zero, d = rn / d_n, in
+  // one launch; where that sweep is the only one, sum += d with it (returned)
+  // and rn stays in registers
+  auto nodal_first = [&](C2<T> *d, C2<T> *sum, int nu) {
+    if (nn == 0) return true;
+    if (nn < w.sell_min_rows) {
+      spmv_real_sell<T>(nn, w.sell_min_rows, k, GTS, GT, res, rn, 0, s);
+      node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, nullptr, d, damp, s);
+      return false;
+    }
+    Nod0<T> nz;
+    nz.nd0 = nd0; nz.nd1 = nd1; nz.nl0 = nl0; nz.nl1 = nl1;
+    nz.d = d; nz.damp = damp;
+    nz.sum = nu == 1 ? sum : nullptr;
+    spmv_real_sell<T, SPMV_NOD0>(nn, w.sell_min_rows, k, GTS, GT, res, nu == 1 ? nullptr : rn, 0, s, w.c1, w.c2, Jac0<T>(), nz);
+    return nz.sum != nullptr;
+  };
   // u and tmp trade places after every Jacobi sweep but the first; start from
   // the buffer that makes the last sweep write the level's own u (no copy)
   if (((nu_pre - 1) + nu_post) & 1) std::swap(u, tmp);
   if ((nu_pre - 1) & 1) std::swap(phi, d2);
-  // pre-smoothing on the edges (phi = 0); at level 0 the first sweep may have
-  // come out of the pass that formed r (precond, Jac0)
-  if (l == 0 && w.u0_ready) {
+  // pre-smoothing on the edges (phi = 0); the first sweep may have come out of
+  // the pass that formed r (Jac0)
+  if (w.u0_ready) {
     w.u0_ready = false;
   } else {
     tb0();
@@ -2644,8 +2773,7 @@ static gp_status vcycle_level(const Hierarchy &H, VWork<T> &w, hipStream_t s, in
   tb0();
   edge(r, u, nullptr, res, EdgeMode::RES, 0, damp, s);
   te0(EdgeMode::RES, 0);
-  spmv_real_sell<T>(nn, w.sell_min_rows, k, GTS, GT, res, rn, 0, s);
-  node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, nullptr, phi, damp, s);
+  nodal_first(phi, nullptr, nu_pre);
   for (int it = 1; it < nu_pre; ++it) {
     node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, phi, d2, damp, s);
     std::swap(phi, d2);
@@ -2657,22 +2785,27 @@ static gp_status vcycle_level(const Hierarchy &H, VWork<T> &w, hipStream_t s, in
   edge(res, u, phi, tmp, EdgeMode::RES | EdgeMode::NOK, 1, damp, s);
   te0(EdgeMode::RES | EdgeMode::NOK, 1);
   const int64_t nec = H.L[l + 1].ne, nnc = H.L[l + 1].nn;
-  spmv_real_sell<T>(nec, w.sell_min_rows, k, PTS, PT, tmp, w.r[l + 1], 0, s);
+  if (l + 2 < (int)H.L.size() && nec >= w.sell_min_rows) {  // with the next level's first sweep
+    const MgLevel &C = H.L[l + 1];
+    spmv_real_sell<T, SPMV_JAC0>(nec, w.sell_min_rows, k, PTS, PT, tmp, w.r[l + 1], 0, s, w.c1, w.c2,
+                                 jac0_of<T>(C, w, l + 1, nu_pre, nu_post));
+    w.u0_ready = nec > 0;
+  } else {
+    spmv_real_sell<T>(nec, w.sell_min_rows, k, PTS, PT, tmp, w.r[l + 1], 0, s);
+  }
   GP_TRY(vcycle_level<T>(H, w, s, l + 1, nu_pre, nu_post));
-  spmv_real_sell<T>(ne, w.sell_min_rows, k, PS, P, w.u[l + 1], u, 1, s);
-  spmv_real_sell<T>(nn, w.sell_min_rows, k, PnS, Pn, w.phi[l + 1], phi, 1, s);
+  prolong_sell<T>(ne, nn, w.sell_min_rows, k, PS, P, w.u[l + 1], u, PnS, Pn, w.phi[l + 1], phi, s);
   (void)nnc;
   // post-smoothing: nodal, then edges
   tb0();
   edge(r, u, phi, res, EdgeMode::RES, 1, damp, s);
   te0(EdgeMode::RES, 1);
-  spmv_real_sell<T>(nn, w.sell_min_rows, k, GTS, GT, res, rn, 0, s);
-  node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, nullptr, d1, damp, s);
+  const bool added = nodal_first(d1, phi, nu_post);
   for (int it = 1; it < nu_post; ++it) {
     node_sell<T>(nn, w.sell_min_rows, k, NS, N, w.c1, w.c2, nd0, nd1, nl0, nl1, rn, d1, d2, damp, s);
     std::swap(d1, d2);
   }
-  k_add<T><<<gn, 256, 0, s>>>(nn * k, phi, d1);
+  if (!added) k_add<T><<<gn, 256, 0, s>>>(nn * k, phi, d1);
   for (int it = 0; it < nu_post; ++it) {
     // the first sweep starts from res = r - K u - B phi_old for this u: only
     // B d1 (the nodal correction just added to phi) is subtracted
@@ -2781,11 +2914,7 @@ gp_status precond(const Hierarchy &H, VWork<T> &w, hipStream_t s, int nu_pre, in
   // the edge V-cycle's first level-0 sweep (u = r / d_l1 from zero) comes out
   // of the same pass, into the buffer that sweep would write
   Jac0<T> jz;
-  if (H.L.size() > 1) {
-    jz.kd0 = arr<T>(L0.kd[0], L0.kdf[0]); jz.kd1 = arr<T>(L0.kd[1], L0.kdf[1]); jz.kd2 = arr<T>(L0.kd[2], L0.kdf[2]);
-    jz.kl0 = arr<T>(L0.kl[0], L0.klf[0]); jz.kl1 = arr<T>(L0.kl[1], L0.klf[1]); jz.kl2 = arr<T>(L0.kl[2], L0.klf[2]);
-    jz.u = (((nu_pre - 1) + nu_post) & 1) ? w.tmp[0] : w.u[0];
-  }
+  if (H.L.size() > 1) jz = jac0_of<T>(L0, w, 0, nu_pre, nu_post);
   w.u0_ready = spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, nullptr, w.a, w.r[0], 1, s, jz);
   // edge V-cycle on the remaining residual
   GP_TRY(vcycle<T>(H, w, s, nu_pre, nu_post));

@@ -58,6 +58,29 @@ def test_aux_products_match_csr_kernels(prec, slots):
     lay.close()
 
 
+@pytest.mark.parametrize("prec", [capi.GP_PREC_FP64, capi.GP_PREC_MIXED])
+@pytest.mark.parametrize("sweeps", [1, 2])
+@pytest.mark.parametrize("slots", [1, 2, 3, 6, 12, 32, 64])
+def test_fused_transfers_match_csr_kernels(slots, sweeps, prec):
+    """Restrictions with the next level's first sweep, G^T products with the nodal
+    one (which keeps its right-hand side only for a second sweep) and both
+    prolongations in a launch, at every slots-per-lane and lanes-per-row shape,
+    against the separate (row, slot) CSR kernels: the same Z to 100 times the
+    residual."""
+    m = M.Mesh(M.manhattan_spec((24, 20, 10), n_ports=3, nfreq=3, f_range=(2e8, 4e9), seed=11))
+    lay = Layout(m)
+    fs = np.geomspace(2e8, 4e9, -(-slots // 3))
+    kw = dict(ports=list(range(min(slots, 3))), precision=prec, rtol=1e-10, batch=slots, max_iters=400,
+              smooth_edge=sweeps)
+    Za, sa, _ = lay.solve(fs, **kw)
+    Zb, sb, _ = lay.solve(fs, sell_min_rows=1 << 40, **kw)
+    print(f"[kernels] fused transfers, {slots} slots, {sweeps} sweeps, precision {prec}: iterations {max(sa['iters'])} / "
+          f"{max(sb['iters'])}, dZ {np.abs(Za - Zb).max() / np.abs(Zb).max():.2e}", flush=True)
+    assert sa["status"] == sb["status"] == capi.GP_OK
+    assert np.abs(Za - Zb).max() <= 1e-8 * np.abs(Zb).max()
+    lay.close()
+
+
 def _dense_coo(A):
     r, c = np.nonzero(np.ones_like(A))
     return r.astype(np.int64), c.astype(np.int64), A.ravel()
