@@ -163,7 +163,7 @@ __global__ void k_outer(OuterOp op, int k, const double *__restrict__ omega, con
   out[i * k + j] = {(TO)acc.x, (TO)acc.y};
 }
 
-template <class TZ, int KS, int NB>
+template <class TZ, int KS, int NB, bool NT = false>
 __device__ __forceinline__ void outer_batch(const SellV<double> &SS, int64_t b0, int t0, int lane,
                                             const C2<TZ> *__restrict__ u, int k, int j0, Z2 (&acc)[KS]) {
   int32_t c[NB];
@@ -171,9 +171,10 @@ __device__ __forceinline__ void outer_batch(const SellV<double> &SS, int64_t b0,
 #pragma unroll
   for (int h = 0; h < NB; ++h) {
     const int64_t e = b0 + (int64_t)(t0 + h) * 64 + lane;
-    // plain loads, as in the preconditioner's walks (sell_batch)
-    c[h] = SS.ci[e];
-    m[h] = SS.v[0][e];
+    // plain loads, as in the preconditioner's walks (sell_batch); NT where one
+    // column streams past and nothing is read twice (k_amul_sell)
+    c[h] = NT ? __builtin_nontemporal_load(SS.ci + e) : SS.ci[e];
+    m[h] = NT ? __builtin_nontemporal_load(SS.v[0] + e) : SS.v[0][e];
   }
   C2<TZ> x[NB][KS];
 #pragma unroll
@@ -321,6 +322,9 @@ __global__ void __launch_bounds__(256) k_amul_sell(SellV<double> SS, int64_t n, 
                                                    const double *__restrict__ sdiag, const int16_t *__restrict__ mcode,
                                                    const double *__restrict__ tab_eps, const double *__restrict__ tab_sig,
                                                    const Z2 *__restrict__ x, Z2 *__restrict__ y) {
+  // one column of 200x200x24: 104 us with non-temporal loads, 114 with plain
+  // ones; 16 columns 865 and 846
+  constexpr bool NT = SPL * LPR == 1;
   const int64_t t_ = xcd_block_id() * blockDim.x + threadIdx.x;
   const int64_t pos = t_ / LPR;
   if (pos >= n) return;
@@ -335,9 +339,9 @@ __global__ void __launch_bounds__(256) k_amul_sell(SellV<double> SS, int64_t n, 
   const int wd = SS.w[sl];
   int t0 = 0;
   if constexpr (SPL == 1)
-    for (; t0 + 8 <= wd; t0 += 8) outer_batch<double, SPL, 8>(SS, b0, t0, lane, x, k, j0, acc);
-  for (; t0 + 4 <= wd; t0 += 4) outer_batch<double, SPL, 4>(SS, b0, t0, lane, x, k, j0, acc);
-  for (; t0 < wd; ++t0) outer_batch<double, SPL, 1>(SS, b0, t0, lane, x, k, j0, acc);
+    for (; t0 + 8 <= wd; t0 += 8) outer_batch<double, SPL, 8, NT>(SS, b0, t0, lane, x, k, j0, acc);
+  for (; t0 + 4 <= wd; t0 += 4) outer_batch<double, SPL, 4, NT>(SS, b0, t0, lane, x, k, j0, acc);
+  for (; t0 < wd; ++t0) outer_batch<double, SPL, 1, NT>(SS, b0, t0, lane, x, k, j0, acc);
   const int mc = mcode[i];  // layer * 2 + (conductor edge)
   const double er = tab_eps[mc >> 1], sg = (mc & 1) ? tab_sig[mc >> 1] : 0.;
   const double sii = sdiag[i];
