@@ -504,7 +504,9 @@ typedef struct gp_v0_stats {
  * receives sys->x as print_z_V0 leaves it (nfreq*np*np complex, see
  * gp_z_v0_sweep).  rtol is the real solves' relative residual; 0 selects the
  * reference's 1e-4.  Builds the V0 basis if the layout has none; the V0
- * operators and the Ad / Ac hierarchies stay with the layout for later calls. */
+ * operators, the Ad / Ac hierarchies and the vectors of up to eight ports
+ * solved side by side (fewer where device memory is short) stay with the layout
+ * for later calls. */
 gp_status gp_solve_v0(gp_layout *lay, double rtol, double *Z0, double *X, gp_v0_stats *stats);
 
 /* The smoother (gp_real_smoother) of the V0 path's Ad and Ac multigrid, the
