@@ -59,6 +59,16 @@ __device__ __forceinline__ void gj_argmax(double &v, int &r, double *sv, int *si
     if (sv[w] > v || (sv[w] == v && si[w] < r)) { v = sv[w]; r = si[w]; }
 }
 
+// Whether matrix b was found singular, the same answer for the whole workgroup.
+// Workgroups of one launch reach that verdict at different times, so one thread
+// reads the flag: were each wavefront to read it, some would leave and the rest
+// pick a pivot from LDS slots that nobody wrote.
+__device__ __forceinline__ bool gj_gone(const int *bad, int b, int *flag) {
+  if (threadIdx.x == 0) *flag = __hip_atomic_load(bad + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  return *flag != 0;
+}
+
 constexpr int kGJPanel = 8;   // most elimination steps per launch
 constexpr int kGJTile = 8;    // columns per workgroup
 
@@ -72,10 +82,10 @@ constexpr int kGJTile = 8;    // columns per workgroup
 // real AMG at 128x128x16, 1.7 ms now (59 launches).
 template <class Z, int M>
 __global__ void __launch_bounds__(256) k_gj_panel(int n, int c0, const Z *__restrict__ src_, Z *__restrict__ dst_,
-                                                  int32_t *__restrict__ rc_, int *__restrict__ bad) {
+                                                  int32_t *__restrict__ rc_, int *bad) {
   extern __shared__ double2 gj_lds[];
   __shared__ double sv[4];
-  __shared__ int si[4];
+  __shared__ int si[4], gone;
   __shared__ int prow[M];
   __shared__ Z piv[M];
   __shared__ Z X[M][kGJTile];
@@ -83,7 +93,7 @@ __global__ void __launch_bounds__(256) k_gj_panel(int n, int c0, const Z *__rest
   Z *P = reinterpret_cast<Z *>(gj_lds);                             // column q at q n: a wavefront's rows in a line
   unsigned char *used = reinterpret_cast<unsigned char *>(P + (int64_t)n * M);  // n
   const int b = blockIdx.y, tid = threadIdx.x;
-  if (bad[b]) return;
+  if (gj_gone(bad, b, &gone)) return;
   const Z *src = src_ + (int64_t)b * n * n;
   Z *dst = dst_ + (int64_t)b * n * n;
   int32_t *rc = rc_ + (int64_t)b * n;
@@ -162,11 +172,11 @@ __global__ void __launch_bounds__(256) k_gj_panel(int n, int c0, const Z *__rest
 template <class Z>
 __global__ void __launch_bounds__(256) k_gj_step(int n, int c, const Z *__restrict__ src_, Z *__restrict__ dst_,
                                                  int32_t *__restrict__ rc_, int32_t *__restrict__ used_,
-                                                 int *__restrict__ bad) {
+                                                 int *bad) {
   __shared__ double sv[4];
-  __shared__ int si[4];
+  __shared__ int si[4], gone;
   const int b = blockIdx.y, tid = threadIdx.x;
-  if (bad[b]) return;
+  if (gj_gone(bad, b, &gone)) return;
   const Z *src = src_ + (int64_t)b * n * n;
   Z *dst = dst_ + (int64_t)b * n * n;
   // used[r]: one more than the step that took row r (0: none yet); this step's

@@ -128,6 +128,39 @@ def test_dense_inverse_of_stalled_coarsening(n):
     assert np.linalg.norm(x - ref) <= 1e-12 * np.linalg.norm(ref)
 
 
+def _solve_singular(row, col, val, n):
+    from gds2para_amd.layout import solve_real
+    with pytest.raises(capi.GpError, match="singular"):
+        solve_real(row, col, val, n, np.ones(n), rtol=1e-12)
+
+
+@pytest.mark.parametrize("n,col", [(1, 0), (2, 1), (64, 0), (64, 63), (250, 100), (512, 0), (512, 255), (512, 511)])
+def test_dense_inverse_singular(n, col):
+    """A zero column leaves the elimination without a pivot in that column's
+    step, in the first launch or a later one: the call reports the singular
+    matrix, and the next one is solved."""
+    from gds2para_amd.layout import solve_real
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n)) + 2.0 * n * np.eye(n)
+    good = A.copy()
+    A[:, col] = 0.0
+    print(f"[kernels] singular matrix n={n}, column {col}", flush=True)
+    _solve_singular(*_dense_coo(A), n)
+    x, it, rr = solve_real(*_dense_coo(good), n, good @ np.ones(n), rtol=1e-12)
+    assert it <= 2 and np.abs(x - 1.0).max() <= 1e-10
+
+
+@pytest.mark.parametrize("n", [1000, 1900, 3800])
+def test_dense_inverse_singular_of_stalled_coarsening(n):
+    """The same with narrower panels and a launch per step (pairs across the
+    matrix, see above, one of them without its coupling)."""
+    i = np.arange(n, dtype=np.int64)
+    v = np.random.default_rng(n).uniform(0.5, 2.0, n)
+    v[n // 3] = 0.0
+    print(f"[kernels] singular matrix of {n} unknowns", flush=True)
+    _solve_singular(i, n - 1 - i, v, n)
+
+
 @pytest.mark.parametrize("runs", [(1, 47, 48, 49), (1023, 1024, 1025, 5), (2047, 2049, 3500, 2)])
 def test_duplicate_sums(runs):
     """Triplets of equal (row, column) are summed by one thread up to 48 of
