@@ -749,6 +749,7 @@ gp_status coarse_table_write(const Hierarchy &H, CoarseCache &C, hipStream_t s) 
   }
   GP_HIP(hipMemcpyAsync((void *)C.tab, h.data(), sizeof(double *) * h.size(), hipMemcpyHostToDevice, s));
   GP_HIP(hipStreamSynchronize(s));  // h goes out of scope
+  C.stale = false;
   return GP_OK;
 }
 
@@ -851,56 +852,87 @@ gp_status aux_coarse_dense(const Hierarchy &H, double w, std::vector<std::comple
   return GP_OK;
 }
 
+namespace {
+
+// Forms the coarsest-level operators at angular frequency w in b, the layout of
+// an entry's memory: K^-1, N^-1 G^T, B, the auxiliary inverse.
+gp_status coarse_form(const Hierarchy &H, double w, C2<double> *b, hipStream_t s) {
+  const int64_t ne = H.neL, nn = H.nnL, na = H.aux.nL;
+  TmpArena T;
+  struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
+  C2<double> *nbuf = nullptr;
+  GP_TRY(T.alloc(&nbuf, nn * nn));
+  C2<double> *pb = b + ne * ne, *bb = pb + ne * nn, *ab = bb + ne * nn;
+  if (ne) k_form_freq<<<blocks_for(ne * ne), 256, 0, s>>>(ne * ne, w, H.KLd[0], H.KLd[1], H.KLd[2], b);
+  if (nn) {
+    k_form_freq<<<blocks_for(nn * nn), 256, 0, s>>>(nn * nn, w, nullptr, H.NLd[0], H.NLd[1], nbuf);
+    k_form_freq<<<blocks_for(ne * nn), 256, 0, s>>>(ne * nn, w, nullptr, H.BLd[0], H.BLd[1], bb);
+  }
+  GP_TRY(dense_inverse_batched(b, (int)ne, 1, s));
+  GP_TRY(dense_inverse_batched(nbuf, (int)nn, 1, s));
+  if (nn) k_coarse_ng<<<blocks_for(nn * ne), 256, 0, s>>>(nn, ne, nbuf, H.GTLd, pb);
+  GP_HIP(hipStreamSynchronize(s));  // nbuf is freed here
+  if (na && !H.aux.eig) GP_TRY(aux_coarse_inverse(H.aux, w, ab, s));
+  return GP_OK;
+}
+
+// A new entry's slot.  The entry joins the cache only once its matrices are
+// formed: a call that fails leaves nothing that a later one would find.
+gp_status coarse_add(const Hierarchy &H, CoarseCache &C, double w, int32_t *slot, hipStream_t s) {
+  const int64_t eb = std::max<int64_t>(coarse_entry_bytes(H), 16);
+  GP_TRY(coarse_make_room(C, eb, s));
+  void *mem = nullptr;
+  if (hipMalloc(&mem, (size_t)eb) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(GP_ERR_NOMEM, "coarse cache entry allocation failed");
+  }
+  const gp_status st = coarse_form(H, w, (C2<double> *)mem, s);
+  if (st != GP_OK) {
+    (void)hipStreamSynchronize(s);
+    (void)hipFree(mem);
+    return st;
+  }
+  int32_t q = 0;
+  while (q < (int32_t)C.e.size() && C.e[q].mem) ++q;
+  if (q == (int32_t)C.e.size()) C.e.emplace_back();
+  CoarseEntry &x = C.e[q];
+  x.omega = w;
+  x.mem = mem;
+  x.bytes = eb;
+  C.bytes += eb;
+  C.stale = true;
+  *slot = q;
+  return GP_OK;
+}
+
+}  // namespace
+
 gp_status coarse_cache_lookup(const Hierarchy &H, CoarseCache &C, const std::vector<double> &omegas,
                               std::vector<int32_t> *slots, hipStream_t s, int pin) {
   const auto t0 = std::chrono::steady_clock::now();
   ScratchScope scratch(s);
   slots->assign(omegas.size(), -1);
-  const int64_t ne = H.neL, nn = H.nnL, na = H.aux.nL;
-  const int64_t eb = coarse_entry_bytes(H);
-  if (na > 0 && H.aux.nblk == 0) return fail(GP_ERR_STATE, "auxiliary coarsest level without its block structure");
+  if (H.aux.nL > 0 && H.aux.nblk == 0) return fail(GP_ERR_STATE, "auxiliary coarsest level without its block structure");
+  // a call that fails keeps no pins
+  struct Unpin {
+    CoarseCache &c; const std::vector<int32_t> &v; size_t n;
+    ~Unpin() { for (size_t i = 0; i < n; ++i) coarse_cache_unpin(c, v[i]); }
+  } pins{C, *slots, 0};
   bool fresh = false;
   for (size_t i = 0; i < omegas.size(); ++i) {
     int32_t q = -1;
     for (int32_t t = 0; t < (int32_t)C.e.size(); ++t)
       if (C.e[t].mem && C.e[t].omega == omegas[i]) { q = t; break; }
     if (q < 0) {
-      TmpArena T;
-      struct Free { Arena &a; ~Free() { a.free_all(); } } fr{T};
-      C2<double> *nbuf = nullptr;
-      GP_TRY(T.alloc(&nbuf, nn * nn));
-      GP_TRY(coarse_make_room(C, eb, s));
-      for (int32_t t = 0; t < (int32_t)C.e.size(); ++t)
-        if (!C.e[t].mem) { q = t; break; }
-      if (q < 0) { q = (int32_t)C.e.size(); C.e.emplace_back(); }
-      CoarseEntry &x = C.e[q];
-      if (hipMalloc(&x.mem, (size_t)std::max<int64_t>(eb, 16)) != hipSuccess) {
-        (void)hipGetLastError();
-        x = CoarseEntry{};
-        return fail(GP_ERR_NOMEM, "coarse cache entry allocation failed");
-      }
-      x.omega = omegas[i];
-      x.bytes = std::max<int64_t>(eb, 16);
-      C.bytes += x.bytes;
-      C2<double> *kb = (C2<double> *)x.mem, *pb = kb + ne * ne, *bb = pb + ne * nn, *ab = bb + ne * nn;
-      const double w = x.omega;
-      if (ne) k_form_freq<<<blocks_for(ne * ne), 256, 0, s>>>(ne * ne, w, H.KLd[0], H.KLd[1], H.KLd[2], kb);
-      if (nn) {
-        k_form_freq<<<blocks_for(nn * nn), 256, 0, s>>>(nn * nn, w, nullptr, H.NLd[0], H.NLd[1], nbuf);
-        k_form_freq<<<blocks_for(ne * nn), 256, 0, s>>>(ne * nn, w, nullptr, H.BLd[0], H.BLd[1], bb);
-      }
-      GP_TRY(dense_inverse_batched(kb, (int)ne, 1, s));
-      GP_TRY(dense_inverse_batched(nbuf, (int)nn, 1, s));
-      if (nn) k_coarse_ng<<<blocks_for(nn * ne), 256, 0, s>>>(nn, ne, nbuf, H.GTLd, pb);
-      GP_HIP(hipStreamSynchronize(s));  // nbuf is freed here
-      if (na && !H.aux.eig) GP_TRY(aux_coarse_inverse(H.aux, w, ab, s));
+      GP_TRY(coarse_add(H, C, omegas[i], &q, s));
       fresh = true;
     }
     C.e[q].used = ++C.clock;
-    if (pin) ++C.e[q].pins;
     (*slots)[i] = q;
+    if (pin) { ++C.e[q].pins; pins.n = i + 1; }
   }
-  if (fresh || !C.tab) GP_TRY(coarse_table_write(H, C, s));
+  if (C.stale || !C.tab) GP_TRY(coarse_table_write(H, C, s));
+  pins.n = 0;
   if (fresh) C.form_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return GP_OK;
 }
@@ -916,6 +948,7 @@ void coarse_cache_free(CoarseCache &C) {
   C.e.clear();
   C.tab = nullptr;
   C.cap = 0;
+  C.stale = false;
   C.bytes = 0;
 }
 

@@ -220,6 +220,7 @@ struct CoarseCache {
   std::vector<CoarseEntry> e;    // index = slot; mem == nullptr marks a free slot
   const double **tab = nullptr;
   int cap = 0;
+  bool stale = false;            // an entry joined since tab was last written
   int64_t bytes = 0;             // entries plus the pointer table
   uint64_t clock = 0;
   int max_entries = 64;

@@ -89,6 +89,34 @@ def test_coarse_cache_bounded():
         assert _relerr(col, ref) < 1e-6, (k, _relerr(col, ref))
 
 
+@pytest.mark.parametrize("prec", [capi.GP_PREC_FP64, capi.GP_PREC_MIXED])
+def test_failed_coarse_entry_leaves_no_trace(prec):
+    """At 1e-170 Hz w^2 underflows and the coarsest nodal matrix has no pivot:
+    the call reports it each time it is made, also beside a frequency that was
+    formed before the failure, and leaves an entry for that one only.  Solves
+    that follow give the bits of a layout that never saw the failure."""
+    m = M.Mesh(_spec())
+    kw = dict(ports=[0], precision=prec, batch=1)
+    ref = Layout(m)
+    Zr = [ref.solve([f], **kw)[0] for f in (1e9, 2e9)]
+    ref.close()
+    lay = Layout(m)
+    for first in (True, False):  # without a pointer table, and with one
+        print(f"[mem] singular coarse matrix, precision {prec}, first call {first}", flush=True)
+        before = lay.hierarchy_info()["coarse_entries"] if not first else 0
+        for _ in range(2):
+            with pytest.raises(capi.GpError, match="singular"):
+                lay.solve([1e-170], **kw)
+        assert lay.hierarchy_info()["coarse_entries"] == before
+        assert np.array_equal(lay.solve([1e9], **kw)[0], Zr[0])
+    with pytest.raises(capi.GpError, match="singular"):
+        lay.solve([2e9, 1e-170], **kw)
+    assert lay.hierarchy_info()["coarse_entries"] == 2
+    assert np.array_equal(lay.solve([2e9], **kw)[0], Zr[1])
+    assert np.array_equal(lay.solve([1e9], **kw)[0], Zr[0])
+    lay.close()
+
+
 @pytest.mark.parametrize("f", [1e7, 1e9, 5e10])
 def test_aux_coarse_block_inverse(f):
     """The auxiliary coarsest level is inverted block by block (its connected
