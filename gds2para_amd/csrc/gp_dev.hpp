@@ -212,10 +212,14 @@ struct Arena {
   }
 };
 
-// Buffers that live for one function: from the thread's ScratchScope, if one is
-// open, else allocated as they are.
+// Buffers that live for one function, whichever way it is left: from the
+// thread's ScratchScope, if one is open (and then opened before the TmpArena),
+// else allocated as they are.
 struct TmpArena : Arena {
   TmpArena() { tmp_ = true; }
+  ~TmpArena() { free_all(); }
+  TmpArena(const TmpArena &) = delete;
+  TmpArena &operator=(const TmpArena &) = delete;
 };
 
 // Deep host copy of a gp_mesh so the caller's arrays may be released.

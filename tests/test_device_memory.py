@@ -1,0 +1,34 @@
+"""The device memory bookkeeping of the library's host code, on the CPU against
+a stand-in device (arena_main.cpp)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIP = os.environ.get("ROCM_PATH", "/opt/rocm") + "/include"
+
+
+@pytest.fixture(scope="module")
+def arena_main(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if cxx is None or not os.path.exists(os.path.join(HIP, "hip", "hip_runtime.h")):
+        pytest.skip("no g++ or HIP headers")
+    exe = tmp_path_factory.mktemp("arena") / "arena_main"
+    csrc = os.path.join(ROOT, "gds2para_amd", "csrc")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-g", "-w", "-D__HIP_PLATFORM_AMD__", "-I", HIP, "-I", csrc, "-I",
+                    os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "arena_main.cpp"),
+                    os.path.join(csrc, "status.cpp"), "-o", str(exe)], check=True)
+    return exe
+
+
+def _run(exe, scenario):
+    r = subprocess.run([str(exe), scenario], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_failed_setup_frees_its_temporaries(arena_main):
+    """A setup step that leaves early gives back every temporary, the pool's and
+    those allocated by themselves."""
+    _run(arena_main, "failed_setup")
