@@ -128,11 +128,17 @@ gp_status aux_coarse_eigen(Arena &A, AuxAMG &X, hipStream_t s) {
   rocblas_int *info = nullptr;
   GP_TRY(T.alloc(&a, n * n)); GP_TRY(T.alloc(&b, n * n)); GP_TRY(T.alloc(&e, n)); GP_TRY(T.alloc(&info, 1));
   GP_TRY(T.alloc(&lam, n));
-  // symmetric inputs: row- and column-major agree
-  GP_HIP(hipMemcpyAsync(a, X.NLd[1], sizeof(double) * n * n, hipMemcpyDeviceToDevice, s));
-  GP_HIP(hipMemcpyAsync(b, X.NLd[0], sizeof(double) * n * n, hipMemcpyDeviceToDevice, s));
-  const rocblas_status rs = rocsolver_dsygvd(h, rocblas_eform_ax, rocblas_evect_original, rocblas_fill_upper,
-                                             (rocblas_int)n, a, (rocblas_int)n, b, (rocblas_int)n, lam, e, info);
+  rocblas_status rs = rocblas_status_success;
+  for (int attempt = 0; attempt < 2; ++attempt) {
+    // symmetric inputs: row- and column-major agree
+    GP_HIP(hipMemcpyAsync(a, X.NLd[1], sizeof(double) * n * n, hipMemcpyDeviceToDevice, s));
+    GP_HIP(hipMemcpyAsync(b, X.NLd[0], sizeof(double) * n * n, hipMemcpyDeviceToDevice, s));
+    rs = rocsolver_dsygvd(h, rocblas_eform_ax, rocblas_evect_original, rocblas_fill_upper, (rocblas_int)n, a,
+                          (rocblas_int)n, b, (rocblas_int)n, lam, e, info);
+    if (rs != rocblas_status_memory_error) break;
+    (void)hipGetLastError();
+    scratch_trim();  // its workspace is not ours: once more with the pool's idle chunks given back
+  }
   rocblas_int hinfo = -1;
   GP_HIP(hipMemcpyAsync(&hinfo, info, sizeof(rocblas_int), hipMemcpyDeviceToHost, s));
   GP_HIP(hipStreamSynchronize(s));

@@ -45,9 +45,13 @@ inline unsigned blocks_for(int64_t n, int threads = 256) {
 // A freed range is handed out again at once, which is safe because everything
 // inside a scope runs on the scope's one stream; at its end the scope waits for
 // that stream and gives everything back, so nothing outlives the call and no
-// two threads share a pool.
+// two threads share a pool.  Ranges that fit no request stay idle meanwhile: an
+// allocation that fails gives the idle chunks back and tries again
+// (device_malloc), and a caller that goes on to other large buffers inside its
+// scope gives them back first (scratch_trim).
 class ScratchPool {
  public:
+  explicit ScratchPool(hipStream_t s) : s_(s) {}
   void *get(size_t bytes) {
     bytes = (bytes + 511) & ~(size_t)511;
     if (bytes > kDirect) return nullptr;
@@ -93,6 +97,20 @@ class ScratchPool {
     return true;
   }
   bool empty() const { return chunk_.empty(); }
+  // Gives back the chunks that hold no buffer; false if there was none.
+  bool trim() {
+    bool any = false;
+    for (auto c = chunk_.begin(); c != chunk_.end();) {
+      auto f = free_.find(c->first);
+      if (f == free_.end() || f->second != c->second) { ++c; continue; }
+      if (!any) (void)hipStreamSynchronize(s_);
+      any = true;
+      (void)hipFree(c->first);
+      free_.erase(f);
+      c = chunk_.erase(c);
+    }
+    return any;
+  }
   void drop() {
     for (auto &c : chunk_) (void)hipFree(c.first);
     chunk_.clear();
@@ -103,14 +121,30 @@ class ScratchPool {
  private:
   static constexpr size_t kDirect = (size_t)512 << 20;    // larger buffers are allocated by themselves
   static constexpr size_t kChunkMax = (size_t)256 << 20;
+  hipStream_t s_;
   size_t next_ = (size_t)8 << 20;
   std::map<char *, size_t> chunk_, free_, used_;
 };
 
 inline thread_local ScratchPool *t_scratch = nullptr;
 
+// hipMalloc; where it fails, once more after the thread's pool has given back
+// its idle chunks.
+inline hipError_t device_malloc(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  if (t_scratch && t_scratch->trim()) e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
+inline void scratch_trim() {
+  if (t_scratch) (void)t_scratch->trim();
+}
+
 struct ScratchScope {
-  explicit ScratchScope(hipStream_t s) : s_(s), outer_(t_scratch != nullptr) {
+  explicit ScratchScope(hipStream_t s) : s_(s), outer_(t_scratch != nullptr), pool_(s) {
     if (!outer_) t_scratch = &pool_;
   }
   ~ScratchScope() {
@@ -167,11 +201,8 @@ struct Arena {
       }
     }
     if (!q) {
-      const hipError_t e = hipMalloc(&q, b);
-      if (e != hipSuccess) {
-        (void)hipGetLastError();
+      if (device_malloc(&q, b) != hipSuccess)
         return fail(GP_ERR_NOMEM, "hipMalloc of " + std::to_string(b) + " bytes failed");
-      }
     }
     *p = (T *)q;
     bytes += (int64_t)b;

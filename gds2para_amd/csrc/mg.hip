@@ -728,8 +728,7 @@ gp_status coarse_table_write(const Hierarchy &H, CoarseCache &C, hipStream_t s) 
       C.tab = nullptr;
     }
     const double **tab = nullptr;
-    if (hipMalloc((void **)&tab, sizeof(double *) * 4 * (size_t)cap) != hipSuccess) {
-      (void)hipGetLastError();
+    if (device_malloc((void **)&tab, sizeof(double *) * 4 * (size_t)cap) != hipSuccess) {
       C.cap = 0;
       return fail(GP_ERR_NOMEM, "coarse cache table allocation failed");
     }
@@ -882,10 +881,7 @@ gp_status coarse_add(const Hierarchy &H, CoarseCache &C, double w, int32_t *slot
   const int64_t eb = std::max<int64_t>(coarse_entry_bytes(H), 16);
   GP_TRY(coarse_make_room(C, eb, s));
   void *mem = nullptr;
-  if (hipMalloc(&mem, (size_t)eb) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(GP_ERR_NOMEM, "coarse cache entry allocation failed");
-  }
+  if (device_malloc(&mem, (size_t)eb) != hipSuccess) return fail(GP_ERR_NOMEM, "coarse cache entry allocation failed");
   const gp_status st = coarse_form(H, w, (C2<double> *)mem, s);
   if (st != GP_OK) {
     (void)hipStreamSynchronize(s);

@@ -965,6 +965,7 @@ extern "C" gp_status gp_solve_real_ex(const int64_t *row, const int64_t *col, co
   RealAMG *G = nullptr;
   GP_TRY(real_amg_create(n, nnz, dr, dc, dv, smoother, &G, s));
   struct GGuard { RealAMG *g; ~GGuard() { real_amg_destroy(g); } } gg{G};
+  scratch_trim();  // the setup's temporaries, before the 61 Krylov vectors
   int32_t it = 0;
   double rel = 0.;
   gp_status st = real_amg_solve(G, 1, bd, xd, tol, 1000, &it, &rel, s);

@@ -2,6 +2,7 @@
 // ScratchScope) on the CPU: the HIP allocation calls below stand in for a device
 // of a given size.  Addresses are handed out but never touched.  The scenario is
 // the first argument; the exit status is 0 when every check holds.
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -79,11 +80,79 @@ void failed_setup() {
   }
 }
 
+// a long-lived buffer, and one larger than the pool hands out, on a device whose
+// memory the pool's idle chunks hold
+void idle_chunks() {
+  g_size = (size_t)1200 * MB;
+  {
+    ScratchScope scope(nullptr);
+    Arena keep;
+    char *p = nullptr, *q = nullptr;
+    for (int pass = 0; pass < 2; ++pass) {
+      TmpArena tmp;
+      char *t[8] = {};
+      for (char *&x : t) CHECK(tmp.alloc(&x, 100 * MB) == GP_OK);
+    }
+    CHECK(g_held >= (size_t)800 * MB);   // idle, in the pool
+    CHECK(keep.alloc(&p, 900 * MB) == GP_OK && p);
+    TmpArena tmp;
+    CHECK(tmp.alloc(&q, 250 * MB) == GP_OK && q);
+    CHECK(keep.alloc(&p, 900 * MB) == GP_ERR_NOMEM && !p);
+    keep.free_all();
+    CHECK(tmp.alloc(&p, 700 * MB) == GP_OK && p);
+    scratch_trim();                      // keeps the chunk of the buffer in use
+    CHECK(g_held >= (size_t)950 * MB);
+  }
+  CHECK(g_live.empty());
+}
+
+// random buffers of a scope: no two that are in use overlap, everything is given
+// back, with idle chunks given back now and then and on a device too small for
+// every request
+void pool() {
+  std::mt19937_64 rng(1);
+  for (size_t size : {(size_t)1 << 40, (size_t)600 * MB}) {
+    g_size = size;
+    ScratchScope scope(nullptr);
+    TmpArena tmp;
+    std::map<char *, int64_t> used;
+    int refused = 0;
+    for (int step = 0; step < 20000; ++step) {
+      if (rng() % 500 == 0) scratch_trim();
+      if (used.empty() || rng() % 2) {
+        const int64_t n = (int64_t)std::exp2((double)(rng() % 2900) / 100.0);
+        char *p = nullptr;
+        if (tmp.alloc(&p, n) != GP_OK) { ++refused; continue; }
+        auto next = used.lower_bound(p);
+        CHECK(next == used.end() || p + n <= next->first);
+        if (next != used.begin()) { --next; CHECK(next->first + next->second <= p); }
+        auto chunk = g_live.upper_bound(p);
+        CHECK(chunk != g_live.begin());
+        --chunk;
+        CHECK(p + n <= chunk->first + chunk->second);
+        used[p] = n;
+      } else {
+        auto it = used.begin();
+        std::advance(it, (long)(rng() % used.size()));
+        char *p = it->first;
+        tmp.release(p, it->second);
+        used.erase(it);
+      }
+    }
+    CHECK(size > (size_t)1 << 38 ? refused == 0 : refused > 0);
+    tmp.free_all();
+    scratch_trim();
+    CHECK(g_live.empty());
+  }
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "failed_setup")) failed_setup();
+  else if (!std::strcmp(what, "idle_chunks")) idle_chunks();
+  else if (!std::strcmp(what, "pool")) pool();
   else { std::printf("unknown scenario '%s'\n", what); return 2; }
   return 0;
 }

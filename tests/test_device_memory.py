@@ -32,3 +32,15 @@ def test_failed_setup_frees_its_temporaries(arena_main):
     """A setup step that leaves early gives back every temporary, the pool's and
     those allocated by themselves."""
     _run(arena_main, "failed_setup")
+
+
+def test_idle_chunks_are_given_back_when_memory_runs_out(arena_main):
+    """The pool's idle chunks never make an allocation fail that would succeed
+    without them."""
+    _run(arena_main, "idle_chunks")
+
+
+def test_pool_buffers(arena_main):
+    """Buffers of a scope lie apart and inside what the device gave, and all of
+    it is given back."""
+    _run(arena_main, "pool")
