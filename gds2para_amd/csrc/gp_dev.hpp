@@ -163,27 +163,26 @@ struct ScratchScope {
   ScratchPool pool_;
 };
 
-// Device allocation with a byte counter (the layout's footprint: the bytes asked
-// for).  Buffers up to kSmall bytes are cut from slabs that live until free_all:
-// a layout holds hundreds, and each hipMalloc / hipFree costs 40-200 us (38 of
-// 134 ms of a whole 48x48x12 run was hipFree).  Slabs double from 64 KB to
-// 32 MB, so the ends left unused stay below what the arena holds.
+// Device allocation with a byte counter: what the arena holds of the device,
+// slabs whole.  Buffers up to kSmall bytes are cut from slabs that live until
+// free_all: a layout holds hundreds, and each hipMalloc / hipFree costs 40-200 us
+// (38 of 134 ms of a whole 48x48x12 run was hipFree).  Slabs double from 64 KB to
+// 32 MB, so their unused ends come to about as much again as the buffers in them
+// at most; releasing a buffer cut from a slab frees nothing before free_all.
 struct Arena {
   int64_t bytes = 0;
-  std::vector<void *> owned;
   template <class T>
   gp_status alloc(T **p, int64_t n) {
     *p = nullptr;
     if (n <= 0) return GP_OK;
     const size_t b = sizeof(T) * (size_t)n;
     void *q = nullptr;
-    if (tmp_ && t_scratch) q = t_scratch->get(b);
     if (!tmp_ && b <= kSmall) {
       const size_t need = (b + 255) & ~(size_t)255;
       if (need > slab_left_) {
         const size_t size = slab_next_ > need ? slab_next_ : need;
         if (hipMalloc(&q, size) == hipSuccess) {
-          owned.push_back(q);
+          keep(q, size, true);
           slab_ = (char *)q;
           slab_left_ = size;
           if (slab_next_ < ((size_t)32 << 20)) slab_next_ *= 2;
@@ -196,35 +195,31 @@ struct Arena {
         *p = (T *)slab_;
         slab_ += need;
         slab_left_ -= need;
-        bytes += (int64_t)b;
         return GP_OK;
       }
     }
-    if (!q) {
-      if (device_malloc(&q, b) != hipSuccess)
-        return fail(GP_ERR_NOMEM, "hipMalloc of " + std::to_string(b) + " bytes failed");
-    }
+    if (tmp_ && t_scratch) q = t_scratch->get(b);
+    if (!q && device_malloc(&q, b) != hipSuccess)
+      return fail(GP_ERR_NOMEM, "hipMalloc of " + std::to_string(b) + " bytes failed");
+    keep(q, b, false);
     *p = (T *)q;
-    bytes += (int64_t)b;
-    owned.push_back(q);
     return GP_OK;
   }
   template <class T>
-  void release(T *&p, int64_t n) {
+  void release(T *&p, int64_t) {
     if (!p) return;
-    bytes -= (int64_t)(sizeof(T) * (size_t)n);
-    for (auto &q : owned)
-      if (q == (void *)p) {
+    for (Held &h : held_)
+      if (h.p == (void *)p) {
         // the first buffer of a slab shares the slab's address: it stays with the rest of it
-        if (tmp_ || sizeof(T) * (size_t)n > kSmall) { give_back(q); q = nullptr; }
+        if (!h.slab) { give_back(h.p); bytes -= (int64_t)h.size; h = Held(); }
         break;
       }
     p = nullptr;
   }
   void free_all() {
-    for (void *q : owned)
-      if (q) give_back(q);
-    owned.clear();
+    for (Held &h : held_)
+      if (h.p) give_back(h.p);
+    held_.clear();
     bytes = 0;
     slab_ = nullptr;
     slab_left_ = 0;
@@ -236,8 +231,22 @@ struct Arena {
 
  private:
   static constexpr size_t kSmall = (size_t)8 << 20, kSlabFirst = (size_t)64 << 10;
+  struct Held {
+    void *p = nullptr;
+    size_t size = 0;
+    bool slab = false;
+  };
+  std::vector<Held> held_;
   char *slab_ = nullptr;
   size_t slab_left_ = 0, slab_next_ = kSlabFirst;
+  void keep(void *q, size_t size, bool slab) {
+    Held h;
+    h.p = q;
+    h.size = size;
+    h.slab = slab;
+    held_.push_back(h);
+    bytes += (int64_t)size;
+  }
   void give_back(void *q) {
     if (!(tmp_ && t_scratch && t_scratch->put(q))) (void)hipFree(q);
   }

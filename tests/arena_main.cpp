@@ -106,6 +106,38 @@ void idle_chunks() {
   CHECK(g_live.empty());
 }
 
+// the byte counter of an arena is what it holds of the device, through random
+// allocations and releases, on a large device and on one that refuses slabs
+void bytes() {
+  std::mt19937_64 rng(2);
+  for (size_t size : {(size_t)1 << 40, (size_t)40 * MB}) {
+    g_size = size;
+    Arena a;
+    std::vector<std::pair<char *, int64_t>> used;
+    int64_t asked = 0;
+    for (int step = 0; step < 4000; ++step) {
+      if (used.empty() || rng() % 4) {
+        const int64_t n = (int64_t)std::exp2((double)(rng() % 2500) / 100.0);
+        char *p = nullptr;
+        if (a.alloc(&p, n) != GP_OK) continue;
+        used.push_back({p, n});
+        asked += n;
+      } else {
+        const size_t i = rng() % used.size();
+        char *p = used[i].first;
+        a.release(p, used[i].second);
+        CHECK(!p);
+        asked -= used[i].second;
+        used.erase(used.begin() + (long)i);
+      }
+      CHECK(a.bytes == (int64_t)g_held);
+      CHECK(a.bytes >= asked);
+    }
+    a.free_all();
+    CHECK(a.bytes == 0 && g_live.empty());
+  }
+}
+
 // random buffers of a scope: no two that are in use overlap, everything is given
 // back, with idle chunks given back now and then and on a device too small for
 // every request
@@ -153,6 +185,7 @@ int main(int argc, char **argv) {
   if (!std::strcmp(what, "failed_setup")) failed_setup();
   else if (!std::strcmp(what, "idle_chunks")) idle_chunks();
   else if (!std::strcmp(what, "pool")) pool();
+  else if (!std::strcmp(what, "bytes")) bytes();
   else { std::printf("unknown scenario '%s'\n", what); return 2; }
   return 0;
 }

@@ -44,3 +44,10 @@ def test_pool_buffers(arena_main):
     """Buffers of a scope lie apart and inside what the device gave, and all of
     it is given back."""
     _run(arena_main, "pool")
+
+
+def test_arena_counts_what_it_holds(arena_main):
+    """An arena's byte counter (what gp_layout_device_bytes adds up) is the
+    memory it holds of the device, slabs whole and released buffers included
+    while their slab stays."""
+    _run(arena_main, "bytes")
