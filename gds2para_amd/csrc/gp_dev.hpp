@@ -169,8 +169,11 @@ struct ScratchScope {
 // (38 of 134 ms of a whole 48x48x12 run was hipFree).  Slabs double from 64 KB to
 // 32 MB, so their unused ends come to about as much again as the buffers in them
 // at most; releasing a buffer cut from a slab frees nothing before free_all.
+// With count_only set before the first call, nothing is allocated: alloc hands
+// out null pointers and bytes becomes what the same calls would hold.
 struct Arena {
   int64_t bytes = 0;
+  bool count_only = false;
   template <class T>
   gp_status alloc(T **p, int64_t n) {
     *p = nullptr;
@@ -181,7 +184,7 @@ struct Arena {
       const size_t need = (b + 255) & ~(size_t)255;
       if (need > slab_left_) {
         const size_t size = slab_next_ > need ? slab_next_ : need;
-        if (hipMalloc(&q, size) == hipSuccess) {
+        if (count_only || hipMalloc(&q, size) == hipSuccess) {
           keep(q, size, true);
           slab_ = (char *)q;
           slab_left_ = size;
@@ -192,14 +195,15 @@ struct Arena {
         q = nullptr;
       }
       if (need <= slab_left_) {
+        slab_left_ -= need;
+        if (count_only) return GP_OK;
         *p = (T *)slab_;
         slab_ += need;
-        slab_left_ -= need;
         return GP_OK;
       }
     }
     if (tmp_ && t_scratch) q = t_scratch->get(b);
-    if (!q && device_malloc(&q, b) != hipSuccess)
+    if (!q && !count_only && device_malloc(&q, b) != hipSuccess)
       return fail(GP_ERR_NOMEM, "hipMalloc of " + std::to_string(b) + " bytes failed");
     keep(q, b, false);
     *p = (T *)q;
@@ -240,12 +244,13 @@ struct Arena {
   char *slab_ = nullptr;
   size_t slab_left_ = 0, slab_next_ = kSlabFirst;
   void keep(void *q, size_t size, bool slab) {
+    bytes += (int64_t)size;
+    if (count_only) return;
     Held h;
     h.p = q;
     h.size = size;
     h.slab = slab;
     held_.push_back(h);
-    bytes += (int64_t)size;
   }
   void give_back(void *q) {
     if (!(tmp_ && t_scratch && t_scratch->put(q))) (void)hipFree(q);

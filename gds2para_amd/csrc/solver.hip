@@ -804,6 +804,58 @@ uint64_t graph_key(const gp_solve_opts &o, const void *tab, int cap, int lanes) 
   return h;
 }
 
+// Edges of every port's first side together, and the most edges of a port.
+void port_edge_counts(const gp_mesh &mesh, int64_t *first, int64_t *most) {
+  *first = 0;
+  *most = 1;
+  for (int32_t p = 0; p < mesh.num_ports; ++p) {
+    const int32_t s0 = mesh.port_side_ptr[p];
+    *first += mesh.side_edge_ptr[s0 + 1] - mesh.side_edge_ptr[s0];
+    int64_t c = 0;
+    for (int32_t sd = s0; sd < mesh.port_side_ptr[p + 1]; ++sd) c += mesh.side_edge_ptr[sd + 1] - mesh.side_edge_ptr[sd];
+    *most = std::max(*most, c);
+  }
+}
+
+// Every device buffer of a workspace; on arenas that only count, its size.
+template <class T, class TV>
+gp_status slot_alloc(gp_layout *lay, const Hierarchy &H, int k, int m, bool want_x, SlotWork<T, TV> *W) {
+  const int64_t n = lay->n, nn = H.L[0].nn, na = H.aux.naux;
+  int64_t nport = 0;
+  port_edge_counts(lay->hm.view, &nport, &W->max_port_edges);
+  GP_TRY(vwork_create<T>(lay, H, k, &W->vw));
+  Arena &A = W->A;
+  GP_TRY(A.alloc(&W->b, n * k)); GP_TRY(A.alloc(&W->xu, n * k)); GP_TRY(A.alloc(&W->xphi, nn * k));
+  GP_TRY(A.alloc(&W->xa, na * k));
+  GP_TRY(A.alloc(&W->V, (int64_t)(m + 1) * n * k)); GP_TRY(A.alloc(&W->w, n * k));
+  // the Arnoldi vector w = A z is stored in the basis precision (its products
+  // and sums are FP64); w itself holds the FP64 restart residuals
+  if constexpr (std::is_same<TV, double>::value) W->wa = W->w;
+  else GP_TRY(A.alloc(&W->wa, n * k));
+  GP_TRY(A.alloc(&W->Zu, (int64_t)m * n * k)); GP_TRY(A.alloc(&W->Zp, (int64_t)m * nn * k));
+  GP_TRY(A.alloc(&W->Za, (int64_t)m * na * k));
+  GP_TRY(A.alloc(&W->om_d, k)); GP_TRY(A.alloc(&W->sc_d, k)); GP_TRY(A.alloc(&W->mask_d, k));
+  GP_TRY(A.alloc(&W->yd, (int64_t)m * k));
+  GP_TRY(W->dots.init(A, k, m + 1));
+  GP_TRY(A.alloc(&W->prow_d, nport)); GP_TRY(A.alloc(&W->xo, nport * k));
+  if (want_x) GP_TRY(A.alloc(&W->xfull, n * k));
+  // right-hand-side entries of newly placed columns: at most k times the
+  // largest port's edge count, allocated once (a free per refill would
+  // synchronise the device and stall other layouts' streams)
+  GP_TRY(A.alloc(&W->rhs_row, W->max_port_edges * k)); GP_TRY(A.alloc(&W->rhs_col, W->max_port_edges * k));
+  GP_TRY(A.alloc(&W->rhs_val, W->max_port_edges * k));
+  return GP_OK;
+}
+
+// Device bytes of a workspace of k slots and restart length m.
+template <class T, class TV>
+int64_t slot_bytes(gp_layout *lay, const Hierarchy &H, int k, int m, bool want_x) {
+  SlotWork<T, TV> W;
+  W.A.count_only = W.vw.arena.count_only = true;
+  (void)slot_alloc(lay, H, k, m, want_x, &W);
+  return W.A.bytes + W.vw.arena.bytes;
+}
+
 template <class T, class TV>
 gp_status slot_work(SolveCtx &cx, int k, int m, bool want_x, SlotWork<T, TV> **out) {
   Solver *sv = cx.sv;
@@ -814,44 +866,15 @@ gp_status slot_work(SolveCtx &cx, int k, int m, bool want_x, SlotWork<T, TV> **o
   }
   release_workspace(sv);
   gp_layout *lay = cx.lay;
-  const Hierarchy &H = sv->H;
   hipStream_t s = lay->stream;
-  const int64_t n = lay->n, nn = H.L[0].nn, na = H.aux.naux;
-  const gp_mesh &mesh = lay->hm.view;
   auto *W = new SlotWork<T, TV>();
   W->k = k; W->m = m; W->tsz = (int)sizeof(T); W->tvsz = (int)sizeof(TV); W->want_x = want_x;
   auto st = [&]() -> gp_status {
-    GP_TRY(vwork_create<T>(lay, H, k, &W->vw));
-    Arena &A = W->A;
-    GP_TRY(A.alloc(&W->b, n * k)); GP_TRY(A.alloc(&W->xu, n * k)); GP_TRY(A.alloc(&W->xphi, nn * k));
-    GP_TRY(A.alloc(&W->xa, na * k));
-    GP_TRY(A.alloc(&W->V, (int64_t)(m + 1) * n * k)); GP_TRY(A.alloc(&W->w, n * k));
-    // the Arnoldi vector w = A z is stored in the basis precision (its products
-    // and sums are FP64); w itself holds the FP64 restart residuals
-    if constexpr (std::is_same<TV, double>::value) W->wa = W->w;
-    else GP_TRY(A.alloc(&W->wa, n * k));
-    GP_TRY(A.alloc(&W->Zu, (int64_t)m * n * k)); GP_TRY(A.alloc(&W->Zp, (int64_t)m * nn * k));
-    GP_TRY(A.alloc(&W->Za, (int64_t)m * na * k));
-    GP_TRY(A.alloc(&W->om_d, k)); GP_TRY(A.alloc(&W->sc_d, k)); GP_TRY(A.alloc(&W->mask_d, k));
-    GP_TRY(A.alloc(&W->yd, (int64_t)m * k));
-    GP_TRY(W->dots.init(A, k, m + 1));
+    GP_TRY(slot_alloc(lay, sv->H, k, m, want_x, W));
     W->prow = port_rows(lay);
     W->map.resize(lay->g.Ne);
-    gp_edge_map(&mesh, W->map.data(), nullptr);
-    GP_TRY(A.alloc(&W->prow_d, (int64_t)W->prow.size())); GP_TRY(A.alloc(&W->xo, (int64_t)W->prow.size() * k));
+    gp_edge_map(&lay->hm.view, W->map.data(), nullptr);
     GP_HIP(hipMemcpyAsync(W->prow_d, W->prow.data(), sizeof(int64_t) * W->prow.size(), hipMemcpyHostToDevice, s));
-    if (want_x) GP_TRY(A.alloc(&W->xfull, n * k));
-    // right-hand-side entries of newly placed columns: at most k times the
-    // largest port's edge count, allocated once (a free per refill would
-    // synchronise the device and stall other layouts' streams)
-    for (int32_t p = 0; p < mesh.num_ports; ++p) {
-      int64_t c = 0;
-      for (int32_t sd = mesh.port_side_ptr[p]; sd < mesh.port_side_ptr[p + 1]; ++sd)
-        c += mesh.side_edge_ptr[sd + 1] - mesh.side_edge_ptr[sd];
-      W->max_port_edges = std::max(W->max_port_edges, c);
-    }
-    GP_TRY(A.alloc(&W->rhs_row, W->max_port_edges * k)); GP_TRY(A.alloc(&W->rhs_col, W->max_port_edges * k));
-    GP_TRY(A.alloc(&W->rhs_val, W->max_port_edges * k));
     GP_HIP(hipStreamSynchronize(s));
     return GP_OK;
   }();
@@ -1348,17 +1371,12 @@ struct CallbackIO : ColumnIO {
   }
 };
 
-// Device bytes one slot of the batched solve needs (basis, preconditioned
-// basis, iterate, V-cycle vectors), for the choice of the slot count.
-int64_t bytes_per_slot(const Hierarchy &H, int m, bool f32, bool v32) {
-  const int64_t n = H.L[0].ne, nn = H.L[0].nn, na = H.aux.naux;
-  const int64_t tz = f32 ? 8 : 16, tv = v32 ? 8 : 16;
-  int64_t b = (int64_t)(m + 1) * n * tv + (int64_t)m * (n + nn + na) * tz + (n * 3 + nn + na) * 16;
-  if (v32) b += n * tv;  // the Arnoldi vector in the basis precision
-  for (const MgLevel &L : H.L) b += (5 * L.ne + 3 * L.nn) * tz;
-  for (const AuxLevel &L : H.aux.L) b += 3 * L.n * tz;
-  b += (H.neL + H.nnL) * 16;
-  return b + (n + na) * tz;
+// Device bytes of the batched solve's workspace at k slots, for the choice of the
+// slot count: precisions as run_slots picks them.
+int64_t workspace_bytes(gp_layout *lay, int k, int m, bool f32, bool v32, bool want_x) {
+  const Hierarchy &H = lay->solver->H;
+  if (!f32) return slot_bytes<double, double>(lay, H, k, m, want_x);
+  return v32 ? slot_bytes<float, float>(lay, H, k, m, want_x) : slot_bytes<float, double>(lay, H, k, m, want_x);
 }
 
 // Preconditioner and basis precision from the options: FP32 preconditioner
@@ -1415,8 +1433,9 @@ gp_status autotune(gp_layout *lay, const gp_solve_opts &o) {
   };
   size_t fre = 0, tot = 0;
   GP_HIP(hipMemGetInfo(&fre, &tot));
-  const int64_t per = bytes_per_slot(sv->H, m, true, true);
-  auto fits = [&](int k) { return (int64_t)k * per <= ((int64_t)fre + (sv->ws ? sv->ws->bytes : 0)) / 2; };
+  auto fits = [&](int k) {
+    return workspace_bytes(lay, k, m, true, true, false) <= ((int64_t)fre + (sv->ws ? sv->ws->bytes : 0)) / 2;
+  };
   // first launches of every kernel instance load code; keep them out of the timing
   GP_TRY(run(fits(8) ? 8 : 1, 16, nullptr));
   const int ks[3] = {8, 16, 32};
@@ -1641,8 +1660,7 @@ extern "C" gp_status gp_solve_fullwave_ex(gp_layout *lay, const double *freqs, i
     size_t fre = 0, tot = 0;
     if (hipMemGetInfo(&fre, &tot) == hipSuccess) {
       const int64_t avail = (int64_t)fre + (sv->ws ? sv->ws->bytes : 0);
-      const int64_t per = bytes_per_slot(sv->H, m, f32, f32 && o.basis != 1);
-      while (kb > 1 && (int64_t)kb * per > avail / 2) kb /= 2;
+      while (kb > 1 && workspace_bytes(lay, pow2_at_least(kb), m, f32, o.basis != 1, X != nullptr) > avail / 2) kb /= 2;
     }
   }
   const int k = pow2_at_least(kb);
@@ -1672,7 +1690,7 @@ extern "C" gp_status gp_solve_workspace_bytes(gp_layout *lay, int32_t precision,
   const CoarseCache &cc = lay->solver->cc;
   const int64_t coarse = std::min<int64_t>(cc.max_bytes, (int64_t)std::max(cc.max_entries, k) *
                                                          coarse_entry_bytes(lay->solver->H));
-  *bytes = (int64_t)k * bytes_per_slot(lay->solver->H, m, f32, f32) + coarse;
+  *bytes = workspace_bytes(lay, k, m, f32, true, false) + coarse;
   return GP_OK;
 }
 

@@ -138,6 +138,24 @@ void bytes() {
   }
 }
 
+// an arena that only counts comes to the bytes of one that allocates
+void count_only() {
+  std::mt19937_64 rng(3);
+  for (int round = 0; round < 200; ++round) {
+    Arena a, c;
+    c.count_only = true;
+    for (int i = 0; i < 60; ++i) {
+      const int64_t n = rng() % 10 ? (int64_t)std::exp2((double)(rng() % 2500) / 100.0) : 0;
+      char *p = nullptr, *q = (char *)&a;
+      CHECK(a.alloc(&p, n) == GP_OK && c.alloc(&q, n) == GP_OK);
+      CHECK(!q && a.bytes == c.bytes);
+    }
+    a.free_all();
+    c.free_all();
+    CHECK(g_live.empty());
+  }
+}
+
 // random buffers of a scope: no two that are in use overlap, everything is given
 // back, with idle chunks given back now and then and on a device too small for
 // every request
@@ -186,6 +204,7 @@ int main(int argc, char **argv) {
   else if (!std::strcmp(what, "idle_chunks")) idle_chunks();
   else if (!std::strcmp(what, "pool")) pool();
   else if (!std::strcmp(what, "bytes")) bytes();
+  else if (!std::strcmp(what, "count_only")) count_only();
   else { std::printf("unknown scenario '%s'\n", what); return 2; }
   return 0;
 }

@@ -51,3 +51,9 @@ def test_arena_counts_what_it_holds(arena_main):
     memory it holds of the device, slabs whole and released buffers included
     while their slab stays."""
     _run(arena_main, "bytes")
+
+
+def test_counting_arena_matches_an_allocating_one(arena_main):
+    """The sizes of gp_solve_workspace_bytes come from the allocation code run
+    on arenas that only count."""
+    _run(arena_main, "count_only")

@@ -64,6 +64,28 @@ def test_workspace_reused_across_calls():
     lay.close()
 
 
+@pytest.mark.parametrize("prec,slots,restart", [(capi.GP_PREC_MIXED, 1, 16), (capi.GP_PREC_MIXED, 8, 16),
+                                                (capi.GP_PREC_MIXED, 4, 50), (capi.GP_PREC_FP64, 2, 16)])
+def test_workspace_is_what_was_stated(prec, slots, restart):
+    """gp_solve_workspace_bytes is the workspace that a solve then holds plus
+    the coarse cache's bound, so a budget kept with it is not exceeded."""
+    import ctypes as C
+    m = M.Mesh(_spec())
+    lay = Layout(m)
+    lay.prepare(prec)
+    base = lay.device_bytes
+    ws = C.c_int64()
+    capi.check(lay.lib.gp_solve_workspace_bytes(lay.h, prec, slots, restart, C.byref(ws)), "gp_solve_workspace_bytes")
+    print(f"[mem] workspace of {slots} slots, restart {restart}, precision {prec}: {ws.value} B stated", flush=True)
+    lay.solve(m.freqs(), precision=prec, batch=slots, restart=restart)
+    info = lay.hierarchy_info()
+    coarse = min(2 << 30, 64 * info["coarse_entry_bytes"])
+    print(f"[mem]   {info['workspace_bytes']} B held, coarse cache up to {coarse} B", flush=True)
+    assert info["workspace_bytes"] == ws.value - coarse
+    assert lay.device_bytes <= base + ws.value
+    lay.close()
+
+
 def test_coarse_cache_bounded():
     """70 distinct frequencies through a cache that holds 64: the oldest
     unpinned entries are evicted, and every column still matches the same
