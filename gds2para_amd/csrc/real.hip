@@ -899,6 +899,12 @@ int64_t real_amg_column_bytes(const RealAMG *G) {
 int64_t real_amg_work_bytes(const RealAMG *G) { return G->W.A.bytes; }
 int64_t real_amg_bytes(const RealAMG *G) { return G->A.bytes + G->W.A.bytes; }
 
+void real_amg_trim(RealAMG *G) {
+  if (!G) return;
+  G->W.A.free_all();
+  G->W.K = 0;
+}
+
 void real_amg_destroy(RealAMG *G) {
   if (!G) return;
   G->W.A.free_all();

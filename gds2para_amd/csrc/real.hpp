@@ -32,6 +32,8 @@ int64_t real_amg_bytes(const RealAMG *G);
 // device bytes of a solve's vectors per column, and those held now
 int64_t real_amg_column_bytes(const RealAMG *G);
 int64_t real_amg_work_bytes(const RealAMG *G);
+// gives a solve's vectors back (none may be running)
+void real_amg_trim(RealAMG *G);
 void real_amg_destroy(RealAMG *G);
 
 }  // namespace gp

@@ -1567,8 +1567,10 @@ extern "C" gp_status gp_coarse_aux_apply(gp_layout *lay, double freq, int32_t k,
 
 extern "C" gp_status gp_layout_trim(gp_layout *lay) {
   if (!lay) return fail(GP_ERR_ARG, "null layout");
-  if (!lay->solver) return GP_OK;
+  if (!lay->solver && !lay->v0path) return GP_OK;
   GP_HIP(hipStreamSynchronize(lay->stream));
+  trim_v0path(lay->v0path);
+  if (!lay->solver) return GP_OK;
   release_workspace(lay->solver);
   for (const CoarseEntry &x : lay->solver->cc.e)
     if (x.pins) return fail(GP_ERR_STATE, "gp_layout_trim: a solve on this layout is running");

@@ -45,7 +45,11 @@ struct V0Path {
 };
 
 void destroy_v0path(V0Path *p) { delete p; }
-int64_t v0path_bytes(const V0Path *p);
+void trim_v0path(V0Path *p) {
+  if (!p) return;
+  real_amg_trim(p->ad);
+  real_amg_trim(p->ac);
+}
 
 namespace {
 

@@ -173,9 +173,10 @@ void gp_layout_destroy(gp_layout *lay);
  * solve workspace and coarse-level cache). */
 int64_t gp_layout_device_bytes(const gp_layout *lay);
 
-/* Releases the solve workspace and the per-frequency coarse-level cache that
- * solves keep with the layout (the matrices and hierarchy stay).  No
- * counterpart in the reference, which frees its PARDISO factors per call. */
+/* Releases the solve workspace, the per-frequency coarse-level cache and the
+ * column vectors that solves (full-wave and V0) keep with the layout (the
+ * matrices and hierarchies stay).  No counterpart in the reference, which
+ * frees its PARDISO factors per call. */
 gp_status gp_layout_trim(gp_layout *lay);
 
 /* ---- stiffness (generateStiff + mklMatrixMulti_nt) ---------------------- */
@@ -506,7 +507,7 @@ typedef struct gp_v0_stats {
  * reference's 1e-4.  Builds the V0 basis if the layout has none; the V0
  * operators, the Ad / Ac hierarchies and the vectors of up to eight ports
  * solved side by side (fewer where device memory is short) stay with the layout
- * for later calls. */
+ * for later calls; gp_layout_trim releases the vectors. */
 gp_status gp_solve_v0(gp_layout *lay, double rtol, double *Z0, double *X, gp_v0_stats *stats);
 
 /* The smoother (gp_real_smoother) of the V0 path's Ad and Ac multigrid, the

@@ -64,6 +64,26 @@ def test_workspace_reused_across_calls():
     lay.close()
 
 
+def test_trim_releases_v0_vectors():
+    """A V0 solve keeps the Krylov vectors of its ports; trim gives them back,
+    on a layout that never prepared the full-wave solver too, and the next
+    solve returns the same bits."""
+    m = M.Mesh(_spec())
+    lay = Layout(m)
+    print("[mem] V0 solve, trim, V0 solve", flush=True)
+    Z1, X1, st = lay.solve_v0(1e-10)
+    held = lay.device_bytes
+    lay.trim()
+    trimmed = lay.device_bytes
+    print(f"[mem] {held} B with the vectors, {trimmed} B without", flush=True)
+    # the vectors of 61 Krylov steps on Ad's rows, four ports wide
+    assert held - trimmed >= 61 * 4 * 8 * st["ad_rows"]
+    Z2, X2, _ = lay.solve_v0(1e-10)
+    assert lay.device_bytes == held
+    assert np.array_equal(Z1, Z2) and np.array_equal(X1, X2)
+    lay.close()
+
+
 @pytest.mark.parametrize("prec,slots,restart", [(capi.GP_PREC_MIXED, 1, 16), (capi.GP_PREC_MIXED, 8, 16),
                                                 (capi.GP_PREC_MIXED, 4, 50), (capi.GP_PREC_FP64, 2, 16)])
 def test_workspace_is_what_was_stated(prec, slots, restart):
