@@ -286,7 +286,10 @@ struct CsrD {            // FP64 CSR, int64 row pointers, int32 columns
 struct V0Data;           // defined in v0.hip
 struct V0Path;           // defined in v0path.hip
 void destroy_v0path(V0Path *);
-void trim_v0path(V0Path *);            // the column vectors that V0 solves keep
+// the column vectors that V0 solves keep: their bytes; giving them back (false:
+// none were held)
+int64_t v0path_work_bytes(const V0Path *);
+bool trim_v0path(V0Path *);
 int64_t v0path_bytes(const V0Path *);
 struct Solver;           // defined in solver.hip
 void destroy_v0(V0Data *);

@@ -868,9 +868,15 @@ gp_status slot_work(SolveCtx &cx, int k, int m, bool want_x, SlotWork<T, TV> **o
   gp_layout *lay = cx.lay;
   hipStream_t s = lay->stream;
   auto *W = new SlotWork<T, TV>();
-  W->k = k; W->m = m; W->tsz = (int)sizeof(T); W->tvsz = (int)sizeof(TV); W->want_x = want_x;
   auto st = [&]() -> gp_status {
-    GP_TRY(slot_alloc(lay, sv->H, k, m, want_x, W));
+    gp_status a = slot_alloc(lay, sv->H, k, m, want_x, W);
+    if (a == GP_ERR_NOMEM && trim_v0path(lay->v0path)) {
+      delete W;
+      W = new SlotWork<T, TV>();
+      a = slot_alloc(lay, sv->H, k, m, want_x, W);
+    }
+    GP_TRY(a);
+    W->k = k; W->m = m; W->tsz = (int)sizeof(T); W->tvsz = (int)sizeof(TV); W->want_x = want_x;
     W->prow = port_rows(lay);
     W->map.resize(lay->g.Ne);
     gp_edge_map(&lay->hm.view, W->map.data(), nullptr);
@@ -1379,6 +1385,13 @@ int64_t workspace_bytes(gp_layout *lay, int k, int m, bool f32, bool v32, bool w
   return v32 ? slot_bytes<float, float>(lay, H, k, m, want_x) : slot_bytes<float, double>(lay, H, k, m, want_x);
 }
 
+// Memory kept from earlier calls that a new workspace may take: the workspace
+// itself is reused or released, and V0 solves' vectors go where it does not fit
+// beside them.
+int64_t kept_bytes(const gp_layout *lay) {
+  return (lay->solver->ws ? lay->solver->ws->bytes : 0) + v0path_work_bytes(lay->v0path);
+}
+
 // Preconditioner and basis precision from the options: FP32 preconditioner
 // with an FP32 basis unless opts.basis asks for FP64; plain FP64 otherwise.
 gp_status run_slots(SolveCtx &cx, ColumnIO &io, int k, bool f32) {
@@ -1434,7 +1447,7 @@ gp_status autotune(gp_layout *lay, const gp_solve_opts &o) {
   size_t fre = 0, tot = 0;
   GP_HIP(hipMemGetInfo(&fre, &tot));
   auto fits = [&](int k) {
-    return workspace_bytes(lay, k, m, true, true, false) <= ((int64_t)fre + (sv->ws ? sv->ws->bytes : 0)) / 2;
+    return workspace_bytes(lay, k, m, true, true, false) <= ((int64_t)fre + kept_bytes(lay)) / 2;
   };
   // first launches of every kernel instance load code; keep them out of the timing
   GP_TRY(run(fits(8) ? 8 : 1, 16, nullptr));
@@ -1512,6 +1525,11 @@ extern "C" gp_status gp_prepare_solver(gp_layout *lay, int32_t precision) {
   }
   auto *sv = new Solver();
   gp_status st = build_hierarchy(lay, sv->arena, &sv->H, want32, 12);
+  if (st == GP_ERR_NOMEM && trim_v0path(lay->v0path)) {  // without the V0 solves' vectors
+    destroy_solver(sv);
+    sv = new Solver();
+    st = build_hierarchy(lay, sv->arena, &sv->H, want32, 12);
+  }
   if (st != GP_OK) { destroy_solver(sv); return st; }
   sv->f32 = want32;
   lay->solver = sv;
@@ -1569,7 +1587,7 @@ extern "C" gp_status gp_layout_trim(gp_layout *lay) {
   if (!lay) return fail(GP_ERR_ARG, "null layout");
   if (!lay->solver && !lay->v0path) return GP_OK;
   GP_HIP(hipStreamSynchronize(lay->stream));
-  trim_v0path(lay->v0path);
+  (void)trim_v0path(lay->v0path);
   if (!lay->solver) return GP_OK;
   release_workspace(lay->solver);
   for (const CoarseEntry &x : lay->solver->cc.e)
@@ -1657,11 +1675,9 @@ extern "C" gp_status gp_solve_fullwave_ex(gp_layout *lay, const double *freqs, i
   kb = std::min(kb, 64);
   kb = std::min(kb, pow2_at_least(ncol));
   {
-    // a workspace kept from an earlier call is reused or released, so its
-    // bytes count as available
     size_t fre = 0, tot = 0;
     if (hipMemGetInfo(&fre, &tot) == hipSuccess) {
-      const int64_t avail = (int64_t)fre + (sv->ws ? sv->ws->bytes : 0);
+      const int64_t avail = (int64_t)fre + kept_bytes(lay);
       while (kb > 1 && workspace_bytes(lay, pow2_at_least(kb), m, f32, o.basis != 1, X != nullptr) > avail / 2) kb /= 2;
     }
   }

@@ -45,10 +45,16 @@ struct V0Path {
 };
 
 void destroy_v0path(V0Path *p) { delete p; }
-void trim_v0path(V0Path *p) {
-  if (!p) return;
+int64_t v0path_work_bytes(const V0Path *p) {
+  if (!p) return 0;
+  return (p->ad ? real_amg_work_bytes(p->ad) : 0) + (p->ac ? real_amg_work_bytes(p->ac) : 0);
+}
+
+bool trim_v0path(V0Path *p) {
+  if (v0path_work_bytes(p) == 0) return false;
   real_amg_trim(p->ad);
   real_amg_trim(p->ac);
+  return true;
 }
 
 namespace {
@@ -301,7 +307,7 @@ extern "C" gp_status gp_solve_v0(gp_layout *lay, double rtol, double *Z0, double
     GP_HIP(hipMemGetInfo(&fre, &tot));
     const int64_t per = real_amg_column_bytes(P.ad) + (P.ac ? real_amg_column_bytes(P.ac) : 0) +
                         (int64_t)sizeof(double) * (5 * P.ne + 2 * nd + 2 * nc);
-    const int64_t avail = (int64_t)fre + real_amg_work_bytes(P.ad) + (P.ac ? real_amg_work_bytes(P.ac) : 0);
+    const int64_t avail = (int64_t)fre + v0path_work_bytes(&P);
     while (k < kPortCols && k < np && 2 * k * per <= avail / 4) k *= 2;
   }
   PortBufs pb;
