@@ -66,7 +66,8 @@ def test_fused_transfers_match_csr_kernels(slots, sweeps, prec):
     one (which keeps its right-hand side only for a second sweep) and both
     prolongations in a launch, at every slots-per-lane and lanes-per-row shape,
     against the separate (row, slot) CSR kernels: the same Z to 100 times the
-    residual."""
+    residual.  A converged solve hides what the preconditioner does; its kernels
+    themselves are compared in test_one_preconditioner_application."""
     m = M.Mesh(M.manhattan_spec((24, 20, 10), n_ports=3, nfreq=3, f_range=(2e8, 4e9), seed=11))
     lay = Layout(m)
     fs = np.geomspace(2e8, 4e9, -(-slots // 3))
@@ -79,6 +80,38 @@ def test_fused_transfers_match_csr_kernels(slots, sweeps, prec):
     assert sa["status"] == sb["status"] == capi.GP_OK
     assert np.abs(Za - Zb).max() <= 1e-8 * np.abs(Zb).max()
     lay.close()
+
+
+@pytest.mark.parametrize("prec", [capi.GP_PREC_FP64, capi.GP_PREC_MIXED])
+@pytest.mark.parametrize("sweeps", [1, 2])
+@pytest.mark.parametrize("cells,slots", [((24, 20, 10), k) for k in (1, 2, 3, 6, 12, 32, 64)] +
+                         [((48, 48, 12), k) for k in (1, 4, 16)])
+def test_one_preconditioner_application(cells, slots, sweeps, prec):
+    """One FGMRES step from zero returns a multiple of the preconditioner's
+    application to the right-hand side, so its kernels are compared without the
+    solver around them: the fused ones against the separate (row, slot) CSR
+    kernels, at every slots-per-lane and lanes-per-row shape (48x48x12: rows of
+    several chunks in the auxiliary products too).
+
+    In FP64 the two differ by rounding, amplified by at most the 1e9 between
+    the curl-curl and the mass terms: 1e-16 x 1e9 x some tens of products,
+    under 1e-5.  In FP32 both are compared with the FP64 application, and the
+    fused kernels may be off by ten times what the separate ones are (1e-5 at
+    least, some hundred products' rounding).  A sweep left out, a wrong
+    diagonal or a row skipped changes it by percents."""
+    m = M.Mesh(M.manhattan_spec(cells, n_ports=3, nfreq=3, f_range=(2e8, 4e9), seed=11))
+    lay = Layout(m)
+    fs = np.geomspace(2e8, 4e9, -(-slots // 3))
+    kw = dict(ports=list(range(min(slots, 3))), batch=slots, max_iters=1, rtol=1e-10, smooth_edge=sweeps, want_x=True)
+    X = lay.solve(fs, precision=prec, **kw)[2]
+    Xc = lay.solve(fs, precision=prec, sell_min_rows=1 << 40, **kw)[2]
+    X64 = lay.solve(fs, precision=capi.GP_PREC_FP64, sell_min_rows=1 << 40, **kw)[2]
+    lay.close()
+    off = lambda a: (np.linalg.norm(a - X64, axis=1) / np.linalg.norm(X64, axis=1)).max()  # noqa: E731
+    print(f"[kernels] one application, {cells}, {slots} slots, {sweeps} sweeps, precision {prec}: fused off by {off(X):.2e}, "
+          f"separate by {off(Xc):.2e}", flush=True)
+    assert np.all(np.isfinite(X))
+    assert off(X) <= (1e-5 if prec == capi.GP_PREC_FP64 else max(1e-5, 10 * off(Xc)))
 
 
 def _dense_coo(A):
