@@ -1211,11 +1211,10 @@ __device__ __forceinline__ void sell_row(const SellV<T> &M, int64_t b0, int wd, 
 }
 
 // Entry-split walk: the lane group es of ES groups sharing a row takes the
-// entries es, es + ES, es + 2 ES, ... (rows of the coarse auxiliary operators
-// hold 30-250 entries; one group per row walked them serially and left those
-// launches latency-bound).  es_reduce then sums the groups' partial results:
-// the groups of a row sit LPR lanes apart inside an aligned LPR*ES-lane block
-// of the wavefront, so xor shuffles over LPR, 2 LPR, ... stay inside the row.
+// entries es, es + ES, es + 2 ES, ... (see entry_split).  es_reduce then sums
+// the groups' partial results: the groups of a row sit LPR lanes apart inside an
+// aligned LPR*ES-lane block of the wavefront, so xor shuffles over LPR, 2 LPR,
+// ... stay inside the row.
 template <class T, int KS, int NV, int ES, class F>
 __device__ __forceinline__ void sell_row_es(const SellV<T> &M, int64_t b0, int wd, int lane, int es,
                                             const C2<T> *__restrict__ x, int k, int j0, F &&f) {
@@ -1743,16 +1742,14 @@ struct Nod0 {
 // at 200x200x24 333.3 -> 324.9.
 enum SpmvEp { SPMV_PLAIN = 0, SPMV_JAC0 = 1, SPMV_NOD0 = 2 };
 
-template <class T, int SPL, int LPR, int ES, int EP>
+template <class T, int SPL, int LPR, int EP>
 __device__ __forceinline__ void spmv_real_row(int64_t t_, int64_t nr, int k, const SellV<T> &M, const C2<T> *__restrict__ x,
                                               C2<T> *__restrict__ y, int accumulate, const T *__restrict__ c1v,
                                               const T *__restrict__ c2v, const Jac0<T> &jz, const Nod0<T> &nz) {
-  constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each;
-                           // ES such groups split the row's entries
-  const int64_t pos = t_ / (LPR * ES);
+  constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each
+  const int64_t pos = t_ / LPR;
   if (pos >= nr) return;
-  const int sub = (int)(t_ - pos * (LPR * ES)), es = sub / LPR;
-  const int j0 = ((int)blockIdx.y * LPR + (sub - es * LPR)) * SPL;
+  const int j0 = ((int)blockIdx.y * LPR + (int)(t_ - pos * LPR)) * SPL;
   const int64_t i = M.rows ? (int64_t)M.rows[pos] : pos;  // slot position -> row
   C2<T> acc[KS];
 #pragma unroll
@@ -1762,13 +1759,11 @@ __device__ __forceinline__ void spmv_real_row(int64_t t_, int64_t nr, int k, con
     const int lane = (int)(pos & 63);
     const int64_t b0 = M.base[sl];
     const int wd = M.w[sl];
-    sell_row_es<T, KS, 1, ES>(M, b0, wd, lane, es, x, k, j0, [&](T a, T, T, const C2<T>(&xv)[KS]) {
+    sell_row<T, KS, 1>(M, b0, wd, lane, x, k, j0, [&](T a, T, T, const C2<T>(&xv)[KS]) {
 #pragma unroll
       for (int q = 0; q < KS; ++q) { acc[q].x += a * xv[q].x; acc[q].y += a * xv[q].y; }
     });
   }
-  es_reduce<T, KS, LPR, ES>(acc);
-  if (es != 0) return;
   if (EP == SPMV_PLAIN && accumulate) {
     C2<T> o[KS];
     load_slots<T, KS>(y + i * k + j0, o);
@@ -1799,12 +1794,12 @@ __device__ __forceinline__ void spmv_real_row(int64_t t_, int64_t nr, int k, con
   }
 }
 
-template <class T, int SPL, int LPR, int ES, int EP>
+template <class T, int SPL, int LPR, int EP>
 __global__ void __launch_bounds__(256) k_spmv_real_sell(int64_t nr, int k, SellV<T> M, const C2<T> *__restrict__ x,
                                                         C2<T> *__restrict__ y, int accumulate,
                                                         const T *__restrict__ c1v, const T *__restrict__ c2v, Jac0<T> jz,
                                                         Nod0<T> nz) {
-  spmv_real_row<T, SPL, LPR, ES, EP>(xcd_block_id() * blockDim.x + threadIdx.x, nr, k, M, x, y, accumulate, c1v, c2v, jz, nz);
+  spmv_real_row<T, SPL, LPR, EP>(xcd_block_id() * blockDim.x + threadIdx.x, nr, k, M, x, y, accumulate, c1v, c2v, jz, nz);
 }
 
 // y += M x and y2 += M2 x2: workgroups below nb take the first, the others the second
@@ -1814,9 +1809,9 @@ __global__ void __launch_bounds__(256) k_prolong_sell(unsigned nb, int64_t nr, i
                                                       const C2<T> *__restrict__ x2, C2<T> *__restrict__ y2) {
   const int64_t b = xcd_block_id();
   if (b < (int64_t)nb)
-    spmv_real_row<T, SPL, LPR, 1, SPMV_PLAIN>(b * 256 + threadIdx.x, nr, k, M, x, y, 1, nullptr, nullptr, Jac0<T>(), Nod0<T>());
+    spmv_real_row<T, SPL, LPR, SPMV_PLAIN>(b * 256 + threadIdx.x, nr, k, M, x, y, 1, nullptr, nullptr, Jac0<T>(), Nod0<T>());
   else
-    spmv_real_row<T, SPL, LPR, 1, SPMV_PLAIN>((b - nb) * 256 + threadIdx.x, nr2, k, M2, x2, y2, 1, nullptr, nullptr, Jac0<T>(),
+    spmv_real_row<T, SPL, LPR, SPMV_PLAIN>((b - nb) * 256 + threadIdx.x, nr2, k, M2, x2, y2, 1, nullptr, nullptr, Jac0<T>(),
                                               Nod0<T>());
 }
 
@@ -2006,19 +2001,16 @@ __global__ void __launch_bounds__(256) k_aux_fin(int k, MatV<T> M, const T *__re
   row.store(ep, i, k, j0, c1, c2, acc);
 }
 
-// SELL M2(w) = c1 v0 + i c2 v1: y = r - M2 x (mode 0), y -= M2 x (1), y = M2 x (2)
-template <class T, int SPL, int LPR, int ES>
+// SELL y -= M2(w) x, M2 = c1 v0 + i c2 v1
+template <class T, int SPL, int LPR>
 __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> M, const T *__restrict__ c1v,
-                                                    const T *__restrict__ c2v, const C2<T> *__restrict__ r,
-                                                    const C2<T> *__restrict__ x, C2<T> *__restrict__ y, int mode,
-                                                    Jac0<T> jz) {
-  constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each;
-                           // ES such groups split the row's entries
+                                                    const T *__restrict__ c2v, const C2<T> *__restrict__ x,
+                                                    C2<T> *__restrict__ y, Jac0<T> jz) {
+  constexpr int KS = SPL;  // LPR adjacent lanes share a row, SPL slots each
   const int64_t t_ = xcd_block_id() * blockDim.x + threadIdx.x;
-  const int64_t pos = t_ / (LPR * ES);
+  const int64_t pos = t_ / LPR;
   if (pos >= nr) return;
-  const int sub = (int)(t_ - pos * (LPR * ES)), es = sub / LPR;
-  const int j0 = ((int)blockIdx.y * LPR + (sub - es * LPR)) * SPL;
+  const int j0 = ((int)blockIdx.y * LPR + (int)(t_ - pos * LPR)) * SPL;
   const int64_t i = M.rows ? (int64_t)M.rows[pos] : pos;  // slot position -> row
   T c1[KS], c2[KS];
 #pragma unroll
@@ -2031,7 +2023,7 @@ __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> 
     const int lane = (int)(pos & 63);
     const int64_t b0 = M.base[sl];
     const int wd = M.w[sl];
-    sell_row_es<T, KS, 2, ES>(M, b0, wd, lane, es, x, k, j0, [&](T a0, T a1, T, const C2<T>(&xv)[KS]) {
+    sell_row<T, KS, 2>(M, b0, wd, lane, x, k, j0, [&](T a0, T a1, T, const C2<T>(&xv)[KS]) {
 #pragma unroll
       for (int q = 0; q < KS; ++q) {
         const T ar = c1[q] * a0, ai = c2[q] * a1;
@@ -2040,23 +2032,17 @@ __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> 
       }
     });
   }
-  es_reduce<T, KS, LPR, ES>(acc);
-  if (es != 0) return;
   C2<T> o[KS];
-  if (mode == 0) load_slots<T, KS>(r + i * k + j0, o);
-  else if (mode == 1) load_slots<T, KS>(y + i * k + j0, o);
+  load_slots<T, KS>(y + i * k + j0, o);
 #pragma unroll
-  for (int q = 0; q < KS; ++q) {
-    if (mode == 2) o[q] = acc[q];
-    else o[q] = {o[q].x - acc[q].x, o[q].y - acc[q].y};
-  }
+  for (int q = 0; q < KS; ++q) o[q] = {o[q].x - acc[q].x, o[q].y - acc[q].y};
   store_slots<T, KS>(y + i * k + j0, o);
   if (jz.u) jac0_store<T, KS>(jz, i, k, j0, c1, c2, o);
 }
 
-// k_spmv2_sell (one entry group, no long rows) on an operator of
-// kNok2MinRows rows or more (the level-0 Bx product): two rows per lane
-// group, their indices and values, r or y and the epilogue's diagonals
+// k_spmv2_sell on an operator of kNok2MinRows rows or more (the level-0 Bx
+// product): two rows per lane group, their indices and values, y and the
+// epilogue's diagonals
 // loaded before the row gathers, as in k_edge_nok2.  Per row the entries are
 // summed in the same order; the compiler may fuse the complex products'
 // multiply-adds differently from k_spmv2_sell (Z of a 400x400x32 solve moved
@@ -2064,8 +2050,8 @@ __global__ void __launch_bounds__(256) k_spmv2_sell(int64_t nr, int k, SellV<T> 
 template <class T, int SPL, int LPR>
 __global__ void __launch_bounds__(256) k_spmv2_sell2(int64_t nr, int64_t half, int k, SellV<T> M,
                                                      const T *__restrict__ c1v, const T *__restrict__ c2v,
-                                                     const C2<T> *__restrict__ r, const C2<T> *__restrict__ x,
-                                                     C2<T> *__restrict__ y, int mode, Jac0<T> jz) {
+                                                     const C2<T> *__restrict__ x, C2<T> *__restrict__ y,
+                                                     Jac0<T> jz) {
   constexpr int KS = SPL, NR = 2, PF = 4;
   const int64_t t = xcd_block_id() * blockDim.x + threadIdx.x;
   const int64_t q0 = t / LPR;
@@ -2108,8 +2094,7 @@ __global__ void __launch_bounds__(256) k_spmv2_sell2(int64_t nr, int64_t half, i
       }
     }
     if (!ok[n]) continue;
-    if (mode == 0) load_slots<T, KS>(r + i[n] * k + j0, o[n]);
-    else if (mode == 1) load_slots<T, KS>(y + i[n] * k + j0, o[n]);
+    load_slots<T, KS>(y + i[n] * k + j0, o[n]);
     if (jz.u) {
       d[n][0] = jz.kd0[i[n]]; d[n][1] = jz.kd1[i[n]]; d[n][2] = jz.kd2[i[n]];
       d[n][3] = jz.kl0[i[n]]; d[n][4] = jz.kl1[i[n]]; d[n][5] = jz.kl2[i[n]];
@@ -2148,10 +2133,7 @@ __global__ void __launch_bounds__(256) k_spmv2_sell2(int64_t nr, int64_t half, i
     };
     for (int tt = PF; tt < wd[n]; ++tt) sell_batch<T, KS, 2, 1, 1>(M, b0[n], tt, lane[n], x, k, j0, f);
 #pragma unroll
-    for (int q = 0; q < KS; ++q) {
-      if (mode == 2) o[n][q] = acc[n][q];
-      else o[n][q] = {o[n][q].x - acc[n][q].x, o[n][q].y - acc[n][q].y};
-    }
+    for (int q = 0; q < KS; ++q) o[n][q] = {o[n][q].x - acc[n][q].x, o[n][q].y - acc[n][q].y};
     store_slots<T, KS>(y + i[n] * k + j0, o[n]);
     if (jz.u) {
       C2<T> uo[KS];
@@ -2278,11 +2260,10 @@ __global__ void __launch_bounds__(256) k_coarse(int step, int64_t ne, int64_t nn
   }
 }
 
-// y = r - M2(w) x  (mode 0),  y -= M2(w) x  (mode 1),  y = M2(w) x (mode 2); M2 = c1 v0 + i c2 v1
+// y = r - M2(w) x, M2 = c1 v0 + i c2 v1 (r may be y)
 template <class T>
 __global__ void k_spmv2(int64_t nr, int k, MatV<T> M, const T *__restrict__ c1v, const T *__restrict__ c2v,
-                        const C2<T> *__restrict__ r, const C2<T> *__restrict__ x, C2<T> *__restrict__ y, int mode,
-                        const C2<T> *__restrict__ lp) {
+                        const C2<T> *r, const C2<T> *__restrict__ x, C2<T> *y, const C2<T> *__restrict__ lp) {
   int64_t t = xcd_block_id() * blockDim.x + threadIdx.x;
   int64_t i = t / k;
   int j = (int)(t - i * k);
@@ -2299,9 +2280,8 @@ __global__ void k_spmv2(int64_t nr, int k, MatV<T> M, const T *__restrict__ c1v,
     acc.x += a.x * v.x - a.y * v.y;
     acc.y += a.x * v.y + a.y * v.x;
   }
-  if (mode == 0) { C2<T> b = r[i * k + j]; y[i * k + j] = {b.x - acc.x, b.y - acc.y}; }
-  else if (mode == 1) { C2<T> b = y[i * k + j]; y[i * k + j] = {b.x - acc.x, b.y - acc.y}; }
-  else y[i * k + j] = acc;
+  const C2<T> b = r[i * k + j];
+  y[i * k + j] = {b.x - acc.x, b.y - acc.y};
 }
 
 // x = A_f^-1 r at the auxiliary coarsest level, A_f block diagonal
@@ -2427,88 +2407,17 @@ void lanes_go(const Lanes &ln, F &&go) {
   lanes(std::integral_constant<int, 1>());
 }
 
-#define GP_LANES_DISPATCH(KERNEL, ...)                                                                   \
-  do {                                                                                                   \
-    const Lanes ln_ = lanes_shape<T>(nr, k);                                                             \
-    if (ln_.sp == 4) {                                                                            \
-      if (ln_.lpr == 16) KERNEL<T, 4, 16><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                         \
-      else if (ln_.lpr == 8) KERNEL<T, 4, 8><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 4) KERNEL<T, 4, 4><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 2) KERNEL<T, 4, 2><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else KERNEL<T, 4, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                                        \
-    } else if (ln_.sp == 2) {                                                                            \
-      if (ln_.lpr == 16) KERNEL<T, 2, 16><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                         \
-      else if (ln_.lpr == 8) KERNEL<T, 2, 8><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 4) KERNEL<T, 2, 4><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 2) KERNEL<T, 2, 2><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else KERNEL<T, 2, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                                        \
-    } else {                                                                                             \
-      if (ln_.lpr == 16) KERNEL<T, 1, 16><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                         \
-      else if (ln_.lpr == 8) KERNEL<T, 1, 8><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 4) KERNEL<T, 1, 4><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 2) KERNEL<T, 1, 2><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else KERNEL<T, 1, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                                        \
-    }                                                                                                    \
-  } while (0)
-
-// Entry groups per row for the node / real / two-value SELL kernels, from the
-// operator's stored entries per row (slice widths, padding included).  The
-// coarse auxiliary operators hold 30-250 entries per row.  With one slot (the
-// plain FP64 single-column path) a single lane walked such a row serially;
-// 4 or 16 lanes per row took that path from 3.40 to 3.65 solves/s at
-// 200x200x24.  With 16 slots the same levels are bound by the 128 bytes of
-// slot data each entry gathers, not by the walk: 16 groups per row left those
-// launches as slow as before (45 us), so that shape keeps ES = 1.
+// Entry groups per row of the nodal sweep with one slot (the plain FP64
+// single-column path), from the operator's stored entries per row (slice widths,
+// padding included): a single lane walks the 27 entries of a coarse level's row
+// serially.  With more slots a row has more lanes, and the launches are bound by
+// the slot data that each entry gathers, not by the walk.  The other operators
+// here hold at most 18 entries a row (coarse edges restrict 2 x 3 x 3 fine ones).
 template <class T>
 int entry_split(const SellV<T> &M, const Lanes &L) {
   if (!(L.sp == 1 && L.lpr == 1) || M.nr == 0) return 1;
-  const double w = (double)M.nent / (double)M.nr;
-  return w >= 128 ? 16 : w >= 24 ? 4 : 1;
+  return (double)M.nent / (double)M.nr >= 24 ? 4 : 1;
 }
-
-#define GP_LANES_ES_DISPATCH(KERNEL, MAT, ...)                                                           \
-  do {                                                                                                   \
-    const Lanes ln_ = lanes_shape<T>(nr, k);                                                             \
-    const int es_ = entry_split<T>(MAT, ln_);                                                            \
-    if (es_ > 1) {                                                                                       \
-      const dim3 g_((unsigned)((nr * es_ + 255) / 256), ln_.grid.y);  /* sp = lpr = 1 */                 \
-      if (es_ == 16) KERNEL<T, 1, 1, 16><<<g_, 256, 0, s>>>(__VA_ARGS__);                                \
-      else KERNEL<T, 1, 1, 4><<<g_, 256, 0, s>>>(__VA_ARGS__);                                           \
-    } else if (ln_.sp == 4) {                                                                            \
-      if (ln_.lpr == 16) KERNEL<T, 4, 16, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 8) KERNEL<T, 4, 8, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else if (ln_.lpr == 4) KERNEL<T, 4, 4, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else if (ln_.lpr == 2) KERNEL<T, 4, 2, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else KERNEL<T, 4, 1, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                                     \
-    } else if (ln_.sp == 2) {                                                                            \
-      if (ln_.lpr == 16) KERNEL<T, 2, 16, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 8) KERNEL<T, 2, 8, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else if (ln_.lpr == 4) KERNEL<T, 2, 4, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else if (ln_.lpr == 2) KERNEL<T, 2, 2, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else KERNEL<T, 2, 1, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                                     \
-    } else {                                                                                             \
-      if (ln_.lpr == 16) KERNEL<T, 1, 16, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                      \
-      else if (ln_.lpr == 8) KERNEL<T, 1, 8, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else if (ln_.lpr == 4) KERNEL<T, 1, 4, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else if (ln_.lpr == 2) KERNEL<T, 1, 2, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                   \
-      else KERNEL<T, 1, 1, 1><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__);                                     \
-    }                                                                                                    \
-  } while (0)
-
-#define GP_LANES_EP_DISPATCH(KERNEL, EP_, MAT, ...)                                                        \
-  do {                                                                                                   \
-    const Lanes ln_ = lanes_shape<T>(nr, k);                                                             \
-    const int es_ = entry_split<T>(MAT, ln_);                                                            \
-    if (es_ > 1) {                                                                                       \
-      const dim3 g_((unsigned)((nr * es_ + 255) / 256), ln_.grid.y);  /* sp = lpr = 1 */                 \
-      if (es_ == 16) KERNEL<T, 1, 1, 16, EP_><<<g_, 256, 0, s>>>(__VA_ARGS__);                           \
-      else KERNEL<T, 1, 1, 4, EP_><<<g_, 256, 0, s>>>(__VA_ARGS__);                                      \
-    } else {                                                                                             \
-      lanes_go<T>(ln_, [&](auto sp_, auto lp_) {                                                         \
-        KERNEL<T, decltype(sp_)::value, decltype(lp_)::value, 1, EP_><<<ln_.grid, 256, 0, s>>>(__VA_ARGS__); \
-      });                                                                                                \
-    }                                                                                                    \
-  } while (0)
 
 template <class T>
 void edge_sell(int64_t nr, int64_t smin, int k, const SellV<T> &K, const SellV<T> &B, const MatV<T> &Kc, const MatV<T> &Bc,
@@ -2540,7 +2449,11 @@ void edge_sell(int64_t nr, int64_t smin, int k, const SellV<T> &K, const SellV<T
       return;
     }
   }
-  GP_LANES_DISPATCH(k_edge_sell, nr, k, K, B, c1, c2, kd0, kd1, kd2, kl0, kl1, kl2, r, u, phi, out, mode, use_phi, damp);
+  const Lanes ln = lanes_shape<T>(nr, k);
+  lanes_go<T>(ln, [&](auto sp_, auto lp_) {
+    k_edge_sell<T, decltype(sp_)::value, decltype(lp_)::value>
+        <<<ln.grid, 256, 0, s>>>(nr, k, K, B, c1, c2, kd0, kd1, kd2, kl0, kl1, kl2, r, u, phi, out, mode, use_phi, damp);
+  });
 }
 
 template <class T>
@@ -2569,7 +2482,16 @@ void node_sell(int64_t nr, int64_t smin, int k, const SellV<T> &N, const MatV<T>
     k_node<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Nc, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp, nullptr);
     return;
   }
-  GP_LANES_ES_DISPATCH(k_node_sell, N, nr, k, N, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp);
+  const Lanes ln = lanes_shape<T>(nr, k);
+  if (entry_split<T>(N, ln) == 4) {
+    k_node_sell<T, 1, 1, 4><<<dim3((unsigned)((nr * 4 + 255) / 256), ln.grid.y), 256, 0, s>>>(
+        nr, k, N, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp);
+    return;
+  }
+  lanes_go<T>(ln, [&](auto sp_, auto lp_) {
+    k_node_sell<T, decltype(sp_)::value, decltype(lp_)::value, 1>
+        <<<ln.grid, 256, 0, s>>>(nr, k, N, c1, c2, nd0, nd1, nl0, nl1, rn, d, dout, damp);
+  });
 }
 
 template <class T, int EP = SPMV_PLAIN>
@@ -2581,15 +2503,19 @@ void spmv_real_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const Ma
     k_spmv_real<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, x, y, accumulate, nullptr);
     return;
   }
-  GP_LANES_EP_DISPATCH(k_spmv_real_sell, EP, M, nr, k, M, x, y, accumulate, c1, c2, jz, nz);
+  const Lanes ln = lanes_shape<T>(nr, k);
+  lanes_go<T>(ln, [&](auto sp_, auto lp_) {
+    k_spmv_real_sell<T, decltype(sp_)::value, decltype(lp_)::value, EP>
+        <<<ln.grid, 256, 0, s>>>(nr, k, M, x, y, accumulate, c1, c2, jz, nz);
+  });
 }
 
-// y += M x and y2 += M2 x2 in one launch where both take one entry group per row
+// y += M x and y2 += M2 x2 in one launch
 template <class T>
 void prolong_sell(int64_t nr, int64_t nr2, int64_t smin, int k, const SellV<T> &M, const MatV<T> &Mc, const C2<T> *x, C2<T> *y,
                   const SellV<T> &M2, const MatV<T> &M2c, const C2<T> *x2, C2<T> *y2, hipStream_t s) {
   const Lanes ln = lanes_shape<T>(nr, k), l2 = lanes_shape<T>(nr2, k);
-  if (nr == 0 || nr2 == 0 || nr < smin || nr2 < smin || entry_split<T>(M, ln) != 1 || entry_split<T>(M2, ln) != 1) {
+  if (nr == 0 || nr2 == 0 || nr < smin || nr2 < smin) {
     spmv_real_sell<T>(nr, smin, k, M, Mc, x, y, 1, s);
     spmv_real_sell<T>(nr2, smin, k, M2, M2c, x2, y2, 1, s);
     return;
@@ -2603,21 +2529,20 @@ void prolong_sell(int64_t nr, int64_t nr2, int64_t smin, int k, const SellV<T> &
   lanes_go<T>(ln, go);
 }
 
-// Returns whether the optional epilogue jz ran (sliced-ELL path only).
+// y -= M2(w) x.  Returns whether the optional epilogue jz ran (sliced-ELL path only).
 template <class T>
-bool spmv2_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const MatV<T> &Mc, const T *c1, const T *c2, const C2<T> *r,
-                const C2<T> *x, C2<T> *y, int mode, hipStream_t s,
-                const Jac0<T> &jz = Jac0<T>()) {
+bool spmv2_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const MatV<T> &Mc, const T *c1, const T *c2,
+                const C2<T> *x, C2<T> *y, hipStream_t s, const Jac0<T> &jz = Jac0<T>()) {
   if (nr == 0) return false;
   if (nr < smin) {
-    k_spmv2<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, c1, c2, r, x, y, mode, nullptr);
+    k_spmv2<T><<<blocks_for(nr * k), 256, 0, s>>>(nr, k, Mc, c1, c2, y, x, y, nullptr);
     return false;
   }
   if (nr >= kNok2MinRows) {  // large operator: two rows per lane group
     const int64_t half = (nr + 1) / 2;
     const Lanes ln = lanes_shape<T>(half, k);
-    if (ln.sp == 4 && entry_split<T>(M, ln) == 1) {
-#define GP_SPMV2X(L) k_spmv2_sell2<T, 4, L><<<ln.grid, 256, 0, s>>>(nr, half, k, M, c1, c2, r, x, y, mode, jz)
+    if (ln.sp == 4) {
+#define GP_SPMV2X(L) k_spmv2_sell2<T, 4, L><<<ln.grid, 256, 0, s>>>(nr, half, k, M, c1, c2, x, y, jz)
       if (ln.lpr == 16) GP_SPMV2X(16);
       else if (ln.lpr == 8) GP_SPMV2X(8);
       else if (ln.lpr == 4) GP_SPMV2X(4);
@@ -2627,7 +2552,10 @@ bool spmv2_sell(int64_t nr, int64_t smin, int k, const SellV<T> &M, const MatV<T
       return jz.u != nullptr;
     }
   }
-  GP_LANES_ES_DISPATCH(k_spmv2_sell, M, nr, k, M, c1, c2, r, x, y, mode, jz);
+  const Lanes ln = lanes_shape<T>(nr, k);
+  lanes_go<T>(ln, [&](auto sp_, auto lp_) {
+    k_spmv2_sell<T, decltype(sp_)::value, decltype(lp_)::value><<<ln.grid, 256, 0, s>>>(nr, k, M, c1, c2, x, y, jz);
+  });
   return jz.u != nullptr;
 }
 
@@ -2655,7 +2583,7 @@ void aux_prod(int64_t nr, const VWork<T> &w, const SellV<T> &S, const MatV<T> &M
     if (MODE == AX_JAC)
       k_node<T><<<g, 256, 0, s>>>(nr, k, M, w.c1, w.c2, ep.d0, ep.d1, ep.l0, ep.l1, ep.r, x, ep.y, (T)1, w.lp);
     else if (MODE == AX_RES)
-      k_spmv2<T><<<g, 256, 0, s>>>(nr, k, M, w.c1, w.c2, ep.r, x, ep.y, 0, w.lp);
+      k_spmv2<T><<<g, 256, 0, s>>>(nr, k, M, w.c1, w.c2, ep.r, x, ep.y, w.lp);
     else
       k_spmv_real<T><<<g, 256, 0, s>>>(nr, k, M, x, ep.y, ep.accumulate, w.lp);
     if (MODE == AX_REAL && ep.z)
@@ -2944,7 +2872,7 @@ gp_status precond(const Hierarchy &H, VWork<T> &w, hipStream_t s, int nu_pre, in
   // of the same pass, into the buffer that sweep would write
   Jac0<T> jz;
   if (H.L.size() > 1) jz = jac0_of<T>(L0, w, 0, nu_pre, nu_post);
-  w.u0_ready = spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, nullptr, w.a, w.r[0], 1, s, jz);
+  w.u0_ready = spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, w.a, w.r[0], s, jz);
   // edge V-cycle on the remaining residual
   GP_TRY(vcycle<T>(H, w, s, nu_pre, nu_post));
   // The second auxiliary correction (on r0 - K u - B phi - Bx a) makes the
@@ -2964,7 +2892,7 @@ gp_status precond(const Hierarchy &H, VWork<T> &w, hipStream_t s, int nu_pre, in
   if (!marched)
     edge_sell<T>(n, w.sell_min_rows, k, KS, BS, K, B, w.c1, w.c2, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                  w.r0, w.u[0], w.phi[0], w.res[0], EdgeMode::RES, 1, (T)1, s);
-  spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, nullptr, w.a, w.res[0], 1, s);
+  spmv2_sell<T>(n, w.sell_min_rows, k, BxS, Bx, w.c1, w.c2, w.a, w.res[0], s);
   aux_prod<T, AX_REAL>(na, w, GxTS, GxT, w.res[0], aux_first<T>(X, w, 0), s);
   GP_TRY(aux_cycle<T>(H, w, s, 0));
   k_add<T><<<blocks_for(na * k), 256, 0, s>>>(na * k, w.a, w.ax[0]);

@@ -294,7 +294,7 @@ struct VWork {
   C2<T> *lpart = nullptr;                   // per-chunk partial products [nchunk][nv][k]
   int nu_aux = 2;
   bool aux_post = false;  // auxiliary correction after the edge V-cycle too (symmetric)
-  bool u0_ready = false;  // level 0's first edge sweep already written (set by precond)
+  bool u0_ready = false;  // the next level's first edge sweep came with its right-hand side (Jac0)
   int64_t sell_min_rows = 1;  // operators with fewer rows use the (row, slot) CSR kernels
   bool edge_march = false;    // level-0 K u gathers through the LDS plane march (FP32, k % 8 == 0)
   KTimer *kt = nullptr;               // times the level-0 edge smoother launches
