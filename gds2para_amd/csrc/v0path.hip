@@ -62,8 +62,9 @@ namespace {
 // Ports solved side by side: their vectors are interleaved (row i, port column j
 // at i*k + j), so the V0 matrices, the Ad and Ac hierarchies and every launch
 // serve all of them.  One port after the other (the layout before) left the 24
-// solves of 8 ports bound by launches and by the longest rows' latency: 820 ms
-// at 200x200x24 (2,900,000 edges), 56 ms now.
+// solves of 8 ports bound by launches, host synchronisations and the longest
+// rows' latency: 512 to 820 ms at 200x200x24 (2,900,000 edges) on four boxes, 54
+// to 59 ms now.
 constexpr int kPortCols = 8;
 
 // y0d /= (2 pi freqStart freqUnit)
