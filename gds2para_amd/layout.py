@@ -42,7 +42,8 @@ class Layout:
         return int(self.lib.gp_layout_device_bytes(self.h))
 
     def trim(self):
-        """Releases the cached solve workspace and coarse-level cache."""
+        """Releases the cached solve workspace, the coarse-level cache and the V0
+        solves' column vectors."""
         capi.check(self.lib.gp_layout_trim(self.h), "gp_layout_trim")
 
     # generateStiff --------------------------------------------------------

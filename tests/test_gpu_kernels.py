@@ -142,7 +142,7 @@ def test_dense_inverse_small(n):
     assert np.linalg.norm(x - ref) <= 1e-11 * c * np.linalg.norm(ref)
 
 
-@pytest.mark.parametrize("n", [1000, 1900, 3800])
+@pytest.mark.parametrize("n", [1000, 1900, 2500, 3800])
 def test_dense_inverse_of_stalled_coarsening(n):
     """Rows coupled in pairs across the matrix with a zero diagonal: nothing
     aggregates, so the dense inverse takes all n unknowns (narrower panels, and
@@ -183,7 +183,7 @@ def test_dense_inverse_singular(n, col):
     assert it <= 2 and np.abs(x - 1.0).max() <= 1e-10
 
 
-@pytest.mark.parametrize("n", [1000, 1900, 3800])
+@pytest.mark.parametrize("n", [1000, 1900, 2500, 3800])
 def test_dense_inverse_singular_of_stalled_coarsening(n):
     """The same with narrower panels and a launch per step (pairs across the
     matrix, see above, one of them without its coupling)."""
